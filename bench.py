@@ -242,7 +242,7 @@ def calibrate_copy(nbytes):
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "extend_plain_1080p_hbm_traffic.md")
 
 
-KERNEL_SOURCES = ("kernels.hip", "pathmath.hpp", "layout.hpp", "engine.hip")
+KERNEL_SOURCES = ("kernels.hip", "paths.hip", "kernel_util.hpp", "pathmath.hpp", "layout.hpp", "engine.hip")
 
 
 def kernel_sources_sha16():

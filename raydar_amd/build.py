@@ -38,7 +38,7 @@ HIP_FLAGS = [
 CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wextra",
              "-Wno-unknown-pragmas"]
 
-HIP_SOURCES = ["kernels.hip", "engine.hip", "api.hip", "batch.hip"]
+HIP_SOURCES = ["kernels.hip", "paths.hip", "engine.hip", "api.hip", "batch.hip"]
 CXX_SOURCES = ["bvh.cpp", "rscn.cpp", "camera.cpp"]
 
 

@@ -85,6 +85,9 @@ void Engine::release_buffers() {
   if (first_hit_) { (void)hipFree(first_hit_); first_hit_ = nullptr; }
   first_hit_px_ = 0;
   first_hit_frame_ = 0;
+  if (cam_) { (void)hipFree(cam_); cam_ = nullptr; }
+  cam_px_ = 0;
+  cam_frame_ = 0;
   q_alloc = 0;
   l_alloc = 0;
   if (d_tickets) { (void)hipFree(d_tickets); d_tickets = nullptr; }
@@ -112,9 +115,9 @@ uint32_t Engine::queued(const QueueCtl &c, int parity) {
   return n;
 }
 
-bool Engine::ensure_buffers(std::string *err) {
+bool Engine::ensure_buffers(std::string *err, bool queues) {
   if (opt.queue < 1024) opt.queue = 1024;
-  const uint32_t need = segment_slots();
+  const uint32_t need = queues || external_ ? segment_slots() : 0;
   if (external_) {
     // borrowed buffers: they must already fit these options
     if (opt.queue != q_alloc || need > seg_cap || opt.l_capacity > l_alloc) {
@@ -123,7 +126,7 @@ bool Engine::ensure_buffers(std::string *err) {
     }
     return true;
   }
-  if (q_alloc != opt.queue || need > seg_cap) {
+  if (queues && (q_alloc != opt.queue || need > seg_cap)) {
     const uint64_t slots = (uint64_t)kSegments * need;
     for (int p = 0; p < 2; ++p) {
       void *f[] = {q[p].ray, q[p].dir, q[p].word, q[p].att, q[p].light};
@@ -165,7 +168,8 @@ bool Engine::ensure_buffers(std::string *err) {
 uint64_t Engine::device_bytes() const {
   // two queues of 14 words per slot plus the 8-byte hit record
   uint64_t b = (uint64_t)kSegments * seg_cap * (2 * 56 + 8) + l_alloc * sizeof(float4) +
-               (uint64_t)ticket_alloc * (sizeof(DevTicket) + 8) + first_hit_px_ * sizeof(HitWord);
+               (uint64_t)ticket_alloc * (sizeof(DevTicket) + 8) + first_hit_px_ * sizeof(HitWord) +
+               cam_px_ * kCamBytes;
   for (const auto &e : aux_) b += e->device_bytes();
   return b;
 }
@@ -420,12 +424,171 @@ bool Engine::launch_iteration(const IterArgs &a, int parity, std::string *err, u
          timed(1, err, launch_extend, a, parity, bound) && timed(2, err, launch_shade, a, parity, bound);
 }
 
+bool Engine::ensure_aux(int n, std::string *err) {
+  while ((int)aux_.size() < n) {
+    auto e = std::make_unique<Engine>();
+    e->device = device;
+    if (!e->init(err)) return false;
+    aux_.push_back(std::move(e));
+  }
+  return true;
+}
+
+// Automatic: two pipes when the scene is traversed from LDS (extend bound by
+// VALU issue), three otherwise (extend also waits on node fetches, so a third
+// stream hides more of it).
+int Engine::pipes_for(const DevJob &j, const DevTicket &t) const {
+  const uint64_t tree = opt.bvh4 && j.n_nodes4 ? 128ull * j.n_nodes4 : 64ull * j.n_nodes;
+  const bool lds = tree + 32ull * j.n_prims <= opt.lds_bvh;
+  const int want = opt.pipes > 0 ? opt.pipes : (lds ? 2 : 3);
+  const uint64_t per_pipe = std::min<uint64_t>(opt.queue / 2, 1ull << 22);
+  const uint64_t by_size = t.paths / std::max<uint64_t>(1, per_pipe);
+  return std::max(1, (int)std::min<uint64_t>({(uint64_t)want, t.spp, by_size}));
+}
+
+// Every one-scene pass whose tree the kernel can walk (the 4-wide tree, 16-bit
+// stack entries, no deeper than the stack), from the smallest (128x128x8:
+// 0.25 -> 0.17 ms the whole call) to the largest measured (1080p, 64 spp: 20.0
+// -> 12.8 ms).  The wavefront keeps what only it does: several jobs in one
+// work list, binary and deeper trees, the linear scan (a scene without a
+// tree), event counts, and the launch forms asked for by option (one ray per
+// lane, other workgroup sizes, every camera ray traced).
+bool Engine::takes_paths(const std::vector<DevJob> &jobs, const std::vector<DevTicket> &tickets) const {
+  if (!launch_paths || external_ || jobs.size() != 1 || tickets.size() != 1) return false;
+  const DevJob &j = jobs[0];
+  return !opt.vk && !opt.count && opt.hit_reuse && !opt.brute_force && opt.refill > 0 && opt.bvh4 &&
+         opt.block == 256 && j.max_bounces > 0 && j.max_bounces <= 255 && tickets[0].spp < (1u << 24) &&
+         j.n_nodes4 > 0 && j.n_nodes <= kNarrowStackNodes && j.stack4 + 3 <= (uint32_t)kStackDepth;
+}
+
+bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame,
+                       std::string *err) {
+  const uint64_t npix = (uint64_t)j.width * j.height;
+  if (npix > cam_px_) {
+    if (cam_) (void)hipFree(cam_);
+    cam_ = nullptr;
+    cam_px_ = 0;
+    cam_frame_ = 0;
+    if (!check(hipMalloc((void **)&cam_, kCamBytes * npix), "hipMalloc(camera hits)", err)) return false;
+    cam_px_ = npix;
+  }
+  // an earlier pass of the same frame recorded them
+  const bool carried = frame != 0 && frame == cam_frame_;
+  cam_frame_ = 0;
+
+  PathArgs a{};
+  a.job = d_job;
+  a.ctl = ctl;
+  a.cam_ray = reinterpret_cast<float4 *>(cam_);
+  a.cam_hit = reinterpret_cast<uint2 *>(cam_ + sizeof(float4) * npix);
+  a.L = L;
+  a.l_cap = l_alloc;
+  a.l_offset = t.l_offset;
+  a.npix = (uint32_t)npix;
+  a.sample_base = t.sample_base;
+  a.spp = t.spp;
+  a.refill = (uint32_t)opt.refill;
+  a.stack_rows = j.stack4 + 3;
+  a.leaf1 = j.max_leaf == 1 ? 1 : 0;
+  const uint64_t tree = sizeof(DevNode4) * (uint64_t)j.n_nodes4 + sizeof(DevPrim) * (uint64_t)j.n_prims;
+  a.lds_bvh_bytes = tree <= opt.lds_bvh ? (uint32_t)tree : 0u;
+  const uint64_t objects = sizeof(DevObject) * (uint64_t)j.n_prims;
+  a.lds_obj_bytes = objects <= opt.lds_objects ? (uint32_t)objects : 0u;
+
+  // Everything is queued without a wait in between; the caller waits for the
+  // accumulation.  A launch's waves take its work list in chunks through a
+  // device counter, so the pipes' launches share one list.
+  const int np = pipes_used = pipes_for(j, t);
+  if (!ensure_aux(np - 1, err)) return false;
+  if (!check(launch_set_ctl(ctl, 0, 0, stream), "set ctl", err)) return false;
+  struct DrainOnError {
+    Engine *e;
+    bool ok = false;
+    ~DrainOnError() {
+      if (ok) return;
+      (void)hipStreamSynchronize(e->stream);
+      for (auto &x : e->aux_) (void)hipStreamSynchronize(x->stream);
+    }
+  } drain{this};
+  auto launch = [&](bool record) {
+    a.cursor = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(ctl) +
+                                            offsetof(QueueCtl, count)) +
+               (record ? 0 : kSegments * kSegStride);
+    a.spp = record ? 1u : t.spp;
+    a.chunks = (uint32_t)((npix + 63) / 64) * a.spp;
+    const int full = opt.grid > 0 ? opt.grid : num_cus * path_blocks_per_cu(a, record);
+    const int fill = (int)std::min<uint64_t>((uint64_t)full, (a.chunks + 3ull) / 4);
+    const int n = record || opt.kernel_timing ? 1 : std::min(np, fill);
+    a.slices = std::min<uint32_t>(kPathSlices, (uint32_t)(fill / n));
+    a.step_groups = a.slices / a.spp;
+    a.step_samples = a.slices % a.spp;
+    // few requests, and small ones so that the waves end together
+    a.request = std::min<uint32_t>(8, std::max<uint32_t>(1, a.chunks / (64u * (uint32_t)fill)));
+    if (n > 1) {
+      if (!arena_free_ &&
+          !check(hipEventCreateWithFlags(&arena_free_, hipEventDisableTiming), "hipEventCreate", err))
+        return false;
+      if (!check(hipEventRecord(arena_free_, stream), "hipEventRecord", err)) return false;
+    }
+    for (int k = 0; k < n; ++k) {
+      Engine &e = k == 0 ? *this : *aux_[k - 1];
+      if (k > 0 && !check(hipStreamWaitEvent(e.stream, arena_free_, 0), "hipStreamWaitEvent", err))
+        return false;
+      const int grid = (int)((int64_t)fill * (k + 1) / n - (int64_t)fill * k / n);
+      if (!check(launch_paths(a, record, grid, e.stream), "launch paths", err)) return false;
+      ++iterations;
+      if (k == 0) continue;
+      if (!e.arena_free_ &&
+          !check(hipEventCreateWithFlags(&e.arena_free_, hipEventDisableTiming), "hipEventCreate", err))
+        return false;
+      if (!check(hipEventRecord(e.arena_free_, e.stream), "hipEventRecord", err) ||
+          !check(hipStreamWaitEvent(stream, e.arena_free_, 0), "hipStreamWaitEvent", err))
+        return false;
+    }
+    return true;
+  };
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (opt.kernel_timing) {
+    if (!check(hipEventCreate(&e0), "hipEventCreate", err) || !check(hipEventCreate(&e1), "hipEventCreate", err) ||
+        !check(hipEventRecord(e0, stream), "hipEventRecord", err))
+      return false;
+  }
+  if (!carried && !launch(true)) return false;
+  if (!launch(false)) return false;
+  if (opt.kernel_timing) {
+    // both launches count as the closest-hit stage, which they are bound by
+    if (!check(hipEventRecord(e1, stream), "hipEventRecord", err) ||
+        !check(hipEventSynchronize(e1), "hipEventSynchronize", err))
+      return false;
+    float ms = 0.f;
+    (void)hipEventElapsedTime(&ms, e0, e1);
+    kernel_ms[1] += ms;
+    kernel_launches[1] += 1;
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+  }
+#ifdef RDH_CHECKED
+  if (!check(hipMemcpyAsync(ctl_host, ctl, sizeof(QueueCtl), hipMemcpyDeviceToHost, stream),
+             "read violations", err) ||
+      !check(hipStreamSynchronize(stream), "paths", err))
+    return false;
+  if (ctl_host->violation) {
+    *err = "device bounds check failed, mask " + std::to_string(ctl_host->violation) + " (internal error)";
+    return false;
+  }
+#endif
+  drain.ok = true;
+  cam_frame_ = frame;
+  return true;
+}
+
 bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
                          const std::vector<DevJob> &host_jobs, std::string *err) {
   const uint64_t frame = hit_frame;  // set by the caller for this pass only
   hit_frame = 0;
   if (tickets.empty()) return true;
-  if (!ensure_buffers(err)) return false;
+  const bool paths = takes_paths(host_jobs, tickets);
+  if (!ensure_buffers(err, !paths)) return false;
   uint64_t w = 0;
   uint32_t max_bounces = 1;
   std::vector<DevTicket> traced;
@@ -444,27 +607,16 @@ bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
            std::to_string(l_alloc);
     return false;
   }
-  if (!traced.empty()) {
+  if (paths) {
+    if (!run_paths(d_jobs, host_jobs[0], traced[0], frame, err)) return false;
+  } else if (!traced.empty()) {
     // Pipes: a one-job pass is divided by samples (pipe k traces samples
     // [s_k, s_k+1) into their own radiance slots), anything else runs whole.
     // Each pipe must still get 4M paths (or half its queue, if smaller):
     // below that the extra launches cost more than the overlap gains
     // (measured break-even between 4M and 8M paths per pass).
     std::vector<std::vector<DevTicket>> parts;
-    int np = 1;
-    if (traced.size() == 1 && host_jobs.size() == 1) {
-      // automatic: two pipes when the scene is traversed from LDS (extend
-      // bound by VALU issue), three otherwise (extend also waits on node
-      // fetches, so a third stream hides more of it)
-      const DevJob &j = host_jobs[0];
-      const uint64_t tree = opt.bvh4 && j.n_nodes4 ? 128ull * j.n_nodes4 : 64ull * j.n_nodes;
-      const bool lds = tree + 32ull * j.n_prims <= opt.lds_bvh;
-      const int want = opt.pipes > 0 ? opt.pipes : (lds ? 2 : 3);
-      const uint64_t per_pipe = std::min<uint64_t>(q_alloc / 2, 1ull << 22);
-      const uint64_t by_size = traced[0].paths / std::max<uint64_t>(1, per_pipe);
-      np = (int)std::min<uint64_t>({(uint64_t)want, traced[0].spp, by_size});
-      np = std::max(np, 1);
-    }
+    const int np = traced.size() == 1 && host_jobs.size() == 1 ? pipes_for(host_jobs[0], traced[0]) : 1;
     pipes_used = np;
     if (np <= 1) {
       parts.push_back(traced);
@@ -484,12 +636,7 @@ bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
         s0 = s1;
       }
     }
-    while ((int)aux_.size() < np - 1) {
-      auto e = std::make_unique<Engine>();
-      e->device = device;
-      if (!e->init(err)) return false;
-      aux_.push_back(std::move(e));
-    }
+    if (!ensure_aux(np - 1, err)) return false;
     // Pipes 1.. write this engine's radiance arena from their own streams:
     // they start after the work already queued here (the previous pass's
     // accumulation still reads the arena).

@@ -20,6 +20,7 @@
 #include "bvh.hpp"
 #include "kernels.hpp"
 #include "layout.hpp"
+#include "paths.hpp"
 
 namespace rdh {
 
@@ -119,7 +120,9 @@ class Engine {
   // engine frees nothing it borrowed.
   void bind_external(const ExternalBuffers &b, const Engine &owner);
   bool external() const { return external_; }
-  bool ensure_buffers(std::string *err);  // (re)allocates for current options
+  // (Re)allocates for the current options; without `queues` only what a pass
+  // of the path kernel uses (radiance arena, control block).
+  bool ensure_buffers(std::string *err, bool queues = true);
   void release_buffers();
 
   bool upload_scene(const BuiltScene &b, DeviceScene *out, std::string *err);
@@ -190,6 +193,14 @@ class Engine {
                                                              const LaunchShape &, bool,
                                                              hipStream_t),
              const IterArgs &a, int parity, uint32_t bound);
+  // Pipes of a one-job pass (see run_tickets).
+  int pipes_for(const DevJob &j, const DevTicket &t) const;
+  // Whether the path kernel renders this pass, its launch arguments, and the
+  // pass itself (everything but the accumulation, not waited for).
+  bool takes_paths(const std::vector<DevJob> &jobs, const std::vector<DevTicket> &tickets) const;
+  bool run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame,
+                 std::string *err);
+  bool ensure_aux(int n, std::string *err);
   bool external_ = false;  // buffers, stream and control copy are borrowed
   std::vector<hipEvent_t> ev_pool_;
   std::vector<std::unique_ptr<Engine>> aux_;  // pipes 1.. of run_tickets
@@ -199,6 +210,9 @@ class Engine {
   HitWord *first_hit_ = nullptr;              // per-pixel camera-ray hits (IterArgs::first_hit)
   uint64_t first_hit_px_ = 0;                 // pixels first_hit_ holds
   uint64_t first_hit_frame_ = 0;              // hit_frame whose hits first_hit_ holds (0: none)
+  unsigned char *cam_ = nullptr;              // the path kernel's camera-hit table
+  uint64_t cam_px_ = 0;                       // pixels it holds
+  uint64_t cam_frame_ = 0;                    // hit_frame whose hits it holds (0: none)
 };
 
 // Message returned by rd_last_error(NULL) (calls with no renderer handle).

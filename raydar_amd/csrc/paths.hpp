@@ -1,0 +1,49 @@
+// The path kernel (paths.hip): whole camera paths of one scene in one launch.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "layout.hpp"
+
+namespace rdh {
+
+constexpr uint32_t kPathSlices = kSegments;  // slices of a work list at most
+
+struct PathArgs {
+  const DevJob *job;
+  QueueCtl *ctl;                // (bounds-checked builds' violation mask)
+  uint32_t *cursor;             // chunks of each slice handed out, kSegStride words apart;
+                                // zero at launch
+  // Camera-ray hits by rank, the pixels in the order their paths start
+  // (tile_order_pixel): direction and distance; hit id (kNoHit) and pixel.
+  float4 *cam_ray;
+  uint2 *cam_hit;
+  float4 *L;                    // radiance arena
+  unsigned long long l_offset;  // slot of local sample 0, pixel 0
+  uint32_t npix;
+  uint32_t sample_base;         // global index of local sample 0
+  uint32_t spp;                 // samples of the pass, below 2^24
+  uint32_t chunks;              // work list: groups of 64 ranks * spp
+  uint32_t slices;              // slices it is dealt to, at most the launch's workgroups
+  uint32_t request;             // chunks a wave asks for at once
+  uint32_t step_groups;         // slices / spp and slices % spp: from one chunk of a
+  uint32_t step_samples;        // slice to the next
+  uint32_t refill;              // idle lanes at which a wave stops to shade and refill
+  uint32_t lds_bvh_bytes;       // > 0: nodes and primitives copied to LDS
+  uint32_t lds_obj_bytes;       // > 0: objects copied to LDS
+  uint32_t stack_rows;          // traversal stack entries per lane
+  int leaf1;                    // every leaf holds one primitive
+  unsigned long long l_cap;     // radiance arena entries (bounds-checked builds)
+};
+
+// Bytes of the camera-hit table per pixel.
+constexpr uint64_t kCamBytes = sizeof(float4) + sizeof(uint2);
+
+// Workgroups of the kernel that fit on one CU, and its launch.  Weak: a host
+// build without the device kernels has neither, and the engine then runs the
+// wavefront's launchers.
+__attribute__((weak)) int path_blocks_per_cu(const PathArgs &a, bool record);
+__attribute__((weak)) hipError_t launch_paths(const PathArgs &a, bool record, int grid,
+                                              hipStream_t st);
+
+}  // namespace rdh

@@ -12,7 +12,7 @@ use std::env;
 use std::path::{Path, PathBuf};
 use std::process::Command;
 
-const HIP_SOURCES: [&str; 4] = ["kernels.hip", "engine.hip", "api.hip", "batch.hip"];
+const HIP_SOURCES: [&str; 5] = ["kernels.hip", "paths.hip", "engine.hip", "api.hip", "batch.hip"];
 const CXX_SOURCES: [&str; 3] = ["bvh.cpp", "rscn.cpp", "camera.cpp"];
 
 fn run(cmd: &mut Command) {

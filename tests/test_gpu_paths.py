@@ -1,0 +1,50 @@
+"""The path kernel (paths.hip): one scene's whole paths in one launch.
+
+Frames against the oracle bit for bit (every draw is keyed by pixel, sample
+and bounce, so neither the order of the paths nor the lanes that carry them
+may show) where its work list and its turns have edges: images of fewer
+pixels than a group of 64, groups that are not full, sample counts that do
+not divide the slices, one workgroup, turns at 1 to 64 idle lanes, a tree in
+LDS or not, leaves of several primitives, one bounce.
+"""
+import numpy as np
+import pytest
+
+import oracle
+import raydar_amd as ra
+from raydar_amd import scenegen
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("size,spp,bounces,opts", [
+    ((1, 1), 3, 12, dict()), ((1, 1), 200, 4, dict()), ((7, 9), 5, 12, dict()),
+    ((8, 8), 33, 12, dict()), ((65, 1), 32, 12, dict()), ((3, 43), 31, 8, dict()),
+    ((64, 64), 2, 1, dict()), ((200, 130), 1, 12, dict()), ((121, 77), 7, 12, dict(grid=1)),
+    ((121, 77), 6, 12, dict(refill=1)), ((121, 77), 6, 12, dict(refill=15, grid=3)),
+    ((121, 77), 6, 12, dict(refill=16)), ((121, 77), 6, 12, dict(refill=64)),
+    ((121, 77), 6, 12, dict(lds_bvh=0, lds_objects=0)), ((121, 77), 6, 12, dict(leaf=5)),
+    ((121, 77), 6, 255, dict(leaf=8, lds_bvh=0)), ((121, 77), 9, 12, dict(pipes=3, queue=4096))])
+def test_path_kernel_matches_oracle(size, spp, bounces, opts):
+    sc = scenegen.plain_1080p(3, *size)
+    print(f"frame {size} spp={spp} bounces={bounces} opts={opts}", flush=True)
+    with ra.HipRenderer(max_sample_count=spp, max_bounces=bounces, seed=17, **opts) as r:
+        img = r.render_frame(sc)
+        acc = r.accumulator()
+    ref = oracle.render(sc, spp, bounces, 17)
+    np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
+    np.testing.assert_array_equal(img.reshape(-1), oracle.tonemap(ref, spp))
+
+
+def test_path_kernel_and_wavefront_alternate_on_one_renderer():
+    # the camera-hit tables of the two are separate: a pass of either must not
+    # leave the other with the hits of an earlier frame or scene
+    a, b = scenegen.plain_1080p(3, 96, 54), scenegen.clustered(4, 300, 96, 54)
+    with ra.HipRenderer(max_sample_count=4, max_bounces=12, seed=5) as r:
+        for sc in (a, b):
+            r.new_frame(sc)
+            for block in (256, 128, 256, 128):  # the path kernel has one workgroup size
+                r.set_option("block", block)
+                r.render_sample(sc)
+            ref = oracle.render(sc, 4, 12, 5)
+            np.testing.assert_array_equal(r.accumulator().view(np.uint32), ref.view(np.uint32))
