@@ -249,8 +249,9 @@ rd_status refresh_job(rd_renderer *r) {
 // that is the last sample's time, as CpuRenderer reports (cpu.rs:196, 218).
 //
 // Vulkan semantics: a pixel's samples share one PCG stream whose position
-// after a sample depends on that sample's draws, so each pass holds one
-// sample (all pixels), and the next pass continues every pixel's stream.
+// after a sample depends on that sample's draws, so they follow one another:
+// inside a pass of the path kernel, or in passes of one sample (all pixels)
+// of the wavefront.  The next pass continues every pixel's stream.
 rd_status render_samples(rd_renderer *r, uint32_t k) {
   const rdh::EngineOptions &o = r->eng.opt;
   if (o.vk != r->frame_vk)
@@ -270,7 +271,13 @@ rd_status render_samples(rd_renderer *r, uint32_t k) {
   while (done < k) {
     uint64_t fit = r->eng.opt.l_capacity / npix;
     if (fit == 0) return r->fail(RD_ERR_INVALID_ARGUMENT, "image larger than the radiance arena");
-    if (o.vk) fit = 1;
+    if (o.vk) {
+      // the wavefront's passes hold one sample, the path kernel takes a
+      // pixel's samples one after another
+      rdh::DevTicket probe{};
+      probe.spp = 1;
+      fit = r->eng.takes_paths(host_jobs, {probe}) ? (1u << 24) - 1u : 1u;
+    }
     uint32_t spp = (uint32_t)std::min<uint64_t>({(uint64_t)(k - done), fit, 0xffffffffull / npix});
     rdh::DevTicket t{};
     t.job = 0;

@@ -456,7 +456,7 @@ int Engine::pipes_for(const DevJob &j, const DevTicket &t) const {
 bool Engine::takes_paths(const std::vector<DevJob> &jobs, const std::vector<DevTicket> &tickets) const {
   if (!launch_paths || external_ || jobs.size() != 1 || tickets.size() != 1) return false;
   const DevJob &j = jobs[0];
-  return !opt.vk && !opt.count && opt.hit_reuse && !opt.brute_force && opt.refill > 0 && opt.bvh4 &&
+  return !opt.count && opt.hit_reuse && !opt.brute_force && opt.refill > 0 && opt.bvh4 &&
          opt.block == 256 && j.max_bounces > 0 && j.max_bounces <= 255 && tickets[0].spp < (1u << 24) &&
          j.n_nodes4 > 0 && j.n_nodes <= kNarrowStackNodes && j.stack4 + 3 <= (uint32_t)kStackDepth;
 }
@@ -486,7 +486,8 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
   a.l_offset = t.l_offset;
   a.npix = (uint32_t)npix;
   a.sample_base = t.sample_base;
-  a.spp = t.spp;
+  a.samples = t.spp;
+  a.vk = opt.vk;
   a.refill = (uint32_t)opt.refill;
   a.stack_rows = j.stack4 + 3;
   a.leaf1 = j.max_leaf == 1 ? 1 : 0;
@@ -514,7 +515,7 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
     a.cursor = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(ctl) +
                                             offsetof(QueueCtl, count)) +
                (record ? 0 : kSegments * kSegStride);
-    a.spp = record ? 1u : t.spp;
+    a.spp = record || opt.vk ? 1u : t.spp;
     a.chunks = (uint32_t)((npix + 63) / 64) * a.spp;
     const int full = opt.grid > 0 ? opt.grid : num_cus * path_blocks_per_cu(a, record);
     const int fill = (int)std::min<uint64_t>((uint64_t)full, (a.chunks + 3ull) / 4);
@@ -602,7 +603,8 @@ bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
       max_bounces = std::max(max_bounces, j.max_bounces);
     }
   }
-  if (w > l_alloc) {
+  const bool accumulated = paths && opt.vk;  // by the path kernel, without radiance slots
+  if (w > l_alloc && !accumulated) {
     *err = "pass needs " + std::to_string(w) + " radiance slots, arena holds " +
            std::to_string(l_alloc);
     return false;
@@ -833,6 +835,7 @@ bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
       e.iterations = 0;
     }
   }
+  if (accumulated) return true;
   // Accumulate every ticket in order: per pixel, samples in sample order.
   for (const auto &t : tickets) {
     const DevJob &j = host_jobs[t.job];

@@ -143,6 +143,9 @@ class Engine {
   bool run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
                    const std::vector<DevJob> &host_jobs, std::string *err);
 
+  // Whether the path kernel renders this pass.
+  bool takes_paths(const std::vector<DevJob> &jobs, const std::vector<DevTicket> &tickets) const;
+
   bool check(hipError_t e, const char *what, std::string *err);
 
   EngineOptions opt;
@@ -195,9 +198,8 @@ class Engine {
              const IterArgs &a, int parity, uint32_t bound);
   // Pipes of a one-job pass (see run_tickets).
   int pipes_for(const DevJob &j, const DevTicket &t) const;
-  // Whether the path kernel renders this pass, its launch arguments, and the
-  // pass itself (everything but the accumulation, not waited for).
-  bool takes_paths(const std::vector<DevJob> &jobs, const std::vector<DevTicket> &tickets) const;
+  // A pass of the path kernel, not waited for (and, but for Vulkan semantics,
+  // not accumulated).
   bool run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame,
                  std::string *err);
   bool ensure_aux(int n, std::string *err);

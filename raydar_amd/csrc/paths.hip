@@ -35,13 +35,30 @@ namespace {
 #ifndef RDH_PATH_WAVES
 #define RDH_PATH_WAVES 6
 #endif
+constexpr int path_waves(bool record, bool vk) { return vk && !record ? 5 : RDH_PATH_WAVES; }
+
+// The camera rays' common origin.
+template <bool VK>
+__device__ __forceinline__ F3 camera_origin(const DevJob &J) {
+  F3 o = f3(J.position[0], J.position[1], J.position[2]), d;
+  if constexpr (VK) camera_ray_vk(J, 0, 0, &o, &d);
+  return o;
+}
 
 // RECORD: trace every pixel's camera ray and write its hit to the table, in
 // the order the paths are handed out (tile_order_pixel).
 // LDS: the tree and the primitives are copied into LDS by every workgroup.
 // LEAF1: every leaf holds one primitive.
-template <int BLOCK, bool RECORD, bool LDS, bool LEAF1>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RDH_PATH_WAVES, 8)))
+// VK (Vulkan semantics): a pixel's samples share one stream of random numbers,
+// whose place after a sample depends on that sample's draws, so a lane keeps
+// its pixel for all samples of the pass, one after another, with the stream's
+// state in a register, and adds each to the accumulator itself (the order
+// k_accumulate would take).  The camera ray has no draw in it here either.
+// 97 objects, 1280x720, 16 spp: 8.1 -> 3.5 ms, which were 16 passes of one
+// sample with 12 bounces of three launches each; 5 waves per SIMD, as the
+// stream and rank do not fit the registers of 6.
+template <int BLOCK, bool RECORD, bool LDS, bool LEAF1, bool VK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(path_waves(RECORD, VK), 8)))
 void k_paths(PathArgs a) {
   typedef uint16_t StackT;
   extern __shared__ __align__(16) unsigned char dynamic_lds[];
@@ -76,7 +93,8 @@ void k_paths(PathArgs a) {
   // spent 0.3 ms of a 1080p recording asking around.)
   const uint32_t slice = blockIdx.x % a.slices;
   const uint32_t slice_chunks = (a.chunks + a.slices - 1u - slice) / a.slices;
-  const F3 cam_o = f3(J.position[0], J.position[1], J.position[2]);
+  const F3 cam_o = camera_origin<VK>(J);
+  const float cull0 = VK ? cull_limit(kVkTMax, 0u) : INFINITY;  // with no hit yet
   // A lane is walking (active), waits to be shaded (full) or is free.
   bool active = false, full = false;
   // The wave's chunk (group, sample, paths handed out) and the chunks of its
@@ -90,6 +108,7 @@ void k_paths(PathArgs a) {
   F3 o = cam_o, d = cam_o;
   F3 at = f3(1.0f, 1.0f, 1.0f), li = f3(0.0f, 0.0f, 0.0f);
   uint32_t pixel = 0, sb = 0;      // sample in the pass << 8 | bounce (RECORD: the rank)
+  uint32_t vk_rank = 0, vk_state = 0;  // VK: the pixel's rank and random-number state
   float bt = 0.0f, tcull = INFINITY;
   uint32_t bid = kNoHit;
   int32_t node = 0;
@@ -97,7 +116,28 @@ void k_paths(PathArgs a) {
   RayPre r;
   SlabNF nf;
 
+  // The lane's path ends with radiance c.  VK: the pixel's next sample, if the
+  // pass has one, waits at the camera ray's hit.
   auto finish = [&](F3 c) {
+    if constexpr (VK) {
+      float4 *acc = reinterpret_cast<float4 *>(J.acc) + pixel;
+      const float4 v = *acc;
+      *acc = make_float4(v.x + c.x, v.y + c.y, v.z + c.z, v.w + 1.0f);
+      if ((sb >> 8) + 1u < a.samples) {
+        const float4 cr = a.cam_ray[vk_rank];
+        o = cam_o;
+        d = f3(cr.x, cr.y, cr.z);
+        bt = cr.w;
+        bid = a.cam_hit[vk_rank].x;
+        at = f3(1.0f, 1.0f, 1.0f);
+        li = f3(0.0f, 0.0f, 0.0f);
+        sb = ((sb >> 8) + 1u) << 8;
+        full = true;
+      } else {
+        J.vk_rng[pixel] = vk_state;
+      }
+      return;
+    }
     const unsigned long long slot =
         a.l_offset + (unsigned long long)(sb >> 8) * a.npix + pixel;
     a.L[chk(slot, a.l_cap, K_RADIANCE, a.ctl)] = make_float4(c.x, c.y, c.z, 1.0f);
@@ -113,15 +153,16 @@ void k_paths(PathArgs a) {
                            : 4u * (uint32_t)__popcll(waiting) >= 3u * live;
     if (turn || walking == 0) {
       if (!more && live == 0) break;
-      if (RECORD) {
+      if constexpr (RECORD) {
         if (full) {
           a.cam_ray[sb] = make_float4(d.x, d.y, d.z, bid == kNoHit ? 0.0f : bt);
           a.cam_hit[sb] = make_uint2(bid, pixel);
           full = false;
         }
       } else if (full && bid == kNoHit) {
-        finish(add(li, mul(world_sample(J, d), at)));  // cpu.rs:334-337
+        // cpu.rs:334-337 (raytrace.rgen:178)
         full = false;
+        finish(add(li, mul(VK ? world_sample_vk(J, d) : world_sample(J, d), at)));
       }
       // Free lanes take the next paths.  A camera path starts at its pixel's
       // recorded hit, so it is shaded in this turn with the lanes that
@@ -162,9 +203,10 @@ void k_paths(PathArgs a) {
         const uint32_t k = off + lanes_below(need);
         if (!active && !full && k < size) {
           const uint32_t rank = chk(group * 64u + k, a.npix, K_RADIANCE, a.ctl);
-          if (RECORD) {
+          if constexpr (RECORD) {
             pixel = tile_order_pixel(rank, J.width, J.height);
-            camera_ray(J, pixel % J.width, pixel / J.width, &o, &d);
+            if (VK) camera_ray_vk(J, pixel % J.width, pixel / J.width, &o, &d);
+            else camera_ray(J, pixel % J.width, pixel / J.width, &o, &d);
             sb = rank;
             fresh = true;
             full = true;  // (until its walk starts below)
@@ -180,8 +222,26 @@ void k_paths(PathArgs a) {
             // a camera path's attenuation and light (cpu.rs:253-254)
             at = f3(1.0f, 1.0f, 1.0f);
             li = f3(0.0f, 0.0f, 0.0f);
-            if (bid == kNoHit) finish(add(li, mul(world_sample(J, d), at)));
-            else full = true;
+            if constexpr (VK) {
+              vk_rank = rank;
+              vk_state = a.sample_base == 0 ? pixel % J.width + (pixel / J.width) * 1000u : J.vk_rng[pixel];
+            }
+            if (bid != kNoHit) {
+              full = true;
+            } else {
+              const F3 c = add(li, mul(VK ? world_sample_vk(J, d) : world_sample(J, d), at));
+              if constexpr (VK) {
+                // every sample of the pixel is this one and draws nothing
+                float4 *acc = reinterpret_cast<float4 *>(J.acc) + pixel;
+                float4 v = *acc;
+                for (uint32_t k = 0; k < a.samples; ++k)
+                  v = make_float4(v.x + c.x, v.y + c.y, v.z + c.z, v.w + 1.0f);
+                *acc = v;
+                J.vk_rng[pixel] = vk_state;
+              } else {
+                finish(c);
+              }
+            }
           }
         }
         off += (uint32_t)__popcll(need);
@@ -192,9 +252,14 @@ void k_paths(PathArgs a) {
                                                    lds_objects[4 * oid + 2], lds_objects[4 * oid + 3])
                                      : load_object(J.objects, oid);
         const HitRec h = closest_hit(o, d, bt, ob);
-        BounceDraws dr;
-        dr.init(J.seed, pixel, a.sample_base + (sb >> 8), sb & 0xffu);
-        const ScatterOut so = scatter(d, h, ob, dr, at, li);
+        ScatterOut so;
+        if constexpr (VK) {
+          so = scatter_vk(d, h, ob, vk_state, at, li);
+        } else {
+          BounceDraws dr;
+          dr.init(J.seed, pixel, a.sample_base + (sb >> 8), sb & 0xffu);
+          so = scatter(d, h, ob, dr, at, li);
+        }
         li = so.light;
         full = false;
         if ((sb & 0xffu) + 1u < J.max_bounces) {
@@ -222,11 +287,12 @@ void k_paths(PathArgs a) {
             for (uint32_t j = 0; j < J.n_prims; ++j) {
               DevPrim pr;
               load_prim(J.prims, j, &pr);
-              test_prim(r, pr, &bt, &bid);
+              if (VK) test_prim_vk(r, pr, &bt, &bid);
+              else test_prim(r, pr, &bt, &bid);
             }
         }
         nf = slab_nf(slab_ray(r, ray_tolerance(r, J.r0_tol)));
-        tcull = cull_limit(bt, bid);
+        tcull = VK && bid == kNoHit ? cull0 : cull_limit(bt, bid);
       }
       continue;
     }
@@ -323,9 +389,10 @@ void k_paths(PathArgs a) {
           } else {
             load_prim(J.prims, j, &pr);
           }
-          test_prim(r, pr, &bt, &bid);
+          if (VK) test_prim_vk(r, pr, &bt, &bid);
+          else test_prim(r, pr, &bt, &bid);
         }
-        tcull = cull_limit(bt, bid);
+        tcull = VK && bid == kNoHit ? cull0 : cull_limit(bt, bid);
       }
       if (done) {
         active = false;
@@ -337,15 +404,18 @@ void k_paths(PathArgs a) {
 
 constexpr int kPathBlock = 256;
 
-const void *paths_fn(bool record, bool lds, bool leaf1) {
-#define RDH_PATHS(M)                                                                       \
-  return lds ? (leaf1 ? (const void *)k_paths<kPathBlock, M, true, true>                   \
-                      : (const void *)k_paths<kPathBlock, M, true, false>)                 \
-             : (leaf1 ? (const void *)k_paths<kPathBlock, M, false, true>                  \
-                      : (const void *)k_paths<kPathBlock, M, false, false>)
-  if (record) RDH_PATHS(true);
-  RDH_PATHS(false);
-#undef RDH_PATHS
+template <bool RECORD, bool VK>
+const void *paths_fn_of(bool lds, bool leaf1) {
+  return lds ? (leaf1 ? (const void *)k_paths<kPathBlock, RECORD, true, true, VK>
+                      : (const void *)k_paths<kPathBlock, RECORD, true, false, VK>)
+             : (leaf1 ? (const void *)k_paths<kPathBlock, RECORD, false, true, VK>
+                      : (const void *)k_paths<kPathBlock, RECORD, false, false, VK>);
+}
+
+const void *paths_fn(const PathArgs &a, bool record) {
+  const bool lds = a.lds_bvh_bytes > 0, leaf1 = a.leaf1 != 0;
+  if (a.vk) return record ? paths_fn_of<true, true>(lds, leaf1) : paths_fn_of<false, true>(lds, leaf1);
+  return record ? paths_fn_of<true, false>(lds, leaf1) : paths_fn_of<false, false>(lds, leaf1);
 }
 
 uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
@@ -358,7 +428,7 @@ uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
 int path_blocks_per_cu(const PathArgs &a, bool record) {
   int n = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &n, paths_fn(record, a.lds_bvh_bytes > 0, a.leaf1 != 0), kPathBlock,
+          &n, paths_fn(a, record), kPathBlock,
           dynamic_lds_bytes(a, record)) != hipSuccess) {
     (void)hipGetLastError();
     return 1;
@@ -369,7 +439,7 @@ int path_blocks_per_cu(const PathArgs &a, bool record) {
 hipError_t launch_paths(const PathArgs &a, bool record, int grid, hipStream_t st) {
   PathArgs args = a;
   void *kargs[] = {&args};
-  return hipLaunchKernel(paths_fn(record, a.lds_bvh_bytes > 0, a.leaf1 != 0), dim3(grid),
+  return hipLaunchKernel(paths_fn(a, record), dim3(grid),
                          dim3(kPathBlock), kargs, dynamic_lds_bytes(a, record), st);
 }
 

@@ -22,7 +22,8 @@ struct PathArgs {
   unsigned long long l_offset;  // slot of local sample 0, pixel 0
   uint32_t npix;
   uint32_t sample_base;         // global index of local sample 0
-  uint32_t spp;                 // samples of the pass, below 2^24
+  uint32_t spp;                 // samples of a group of ranks in the work list, below 2^24
+  uint32_t samples;             // vk: samples a lane takes of its pixel, below 2^24
   uint32_t chunks;              // work list: groups of 64 ranks * spp
   uint32_t slices;              // slices it is dealt to, at most the launch's workgroups
   uint32_t request;             // chunks a wave asks for at once
@@ -33,6 +34,8 @@ struct PathArgs {
   uint32_t lds_obj_bytes;       // > 0: objects copied to LDS
   uint32_t stack_rows;          // traversal stack entries per lane
   int leaf1;                    // every leaf holds one primitive
+  int vk;                       // Vulkan semantics: the work list holds each group once and
+                                // the launch accumulates (L is not used)
   unsigned long long l_cap;     // radiance arena entries (bounds-checked builds)
 };
 

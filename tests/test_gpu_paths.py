@@ -48,3 +48,20 @@ def test_path_kernel_and_wavefront_alternate_on_one_renderer():
                 r.render_sample(sc)
             ref = oracle.render(sc, 4, 12, 5)
             np.testing.assert_array_equal(r.accumulator().view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("size,spp,bounces,opts", [
+    ((1, 1), 9, 12, dict()), ((7, 9), 5, 12, dict()), ((65, 1), 3, 1, dict()),
+    ((121, 77), 6, 12, dict(grid=1)), ((121, 77), 6, 12, dict(refill=1)),
+    ((121, 77), 6, 12, dict(refill=64, leaf=5)), ((121, 77), 6, 40, dict(lds_bvh=0, lds_objects=0))])
+def test_path_kernel_vulkan_semantics_match_oracle(size, spp, bounces, opts):
+    # a lane takes its pixel's samples one after another on the pixel's one
+    # stream of random numbers
+    sc = scenegen.plain_1080p(3, *size)
+    print(f"vulkan frame {size} spp={spp} bounces={bounces} opts={opts}", flush=True)
+    with ra.HipRenderer(max_sample_count=spp, max_bounces=bounces, semantics=1, **opts) as r:
+        img = r.render_frame(sc)
+        acc = r.accumulator()
+    ref = oracle.vk_render(sc, ra.camera_vulkan_inverse_view(sc.camera), spp, bounces, threads=8)
+    np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
+    np.testing.assert_array_equal(img.reshape(-1), oracle.vk_tonemap(ref, spp))
