@@ -503,6 +503,7 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   const uint64_t o_prims = take(sizeof(rdh::DevPrim) * b.prims.size());
   const uint64_t o_obj = take(sizeof(rdh::DevObject) * b.objects.size());
   const uint64_t o_acc = take(16 * npix), o_img = take(4 * npix);
+  const uint64_t o_rest = off;
   uint64_t o_q[2][5];
   for (int p = 0; p < 2; ++p) {
     o_q[p][0] = take(sizeof(rdh::QRay) * slots);
@@ -512,15 +513,22 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
     o_q[p][4] = take(sizeof(rdh::QLight) * slots);
   }
   const uint64_t o_hit_t = take(4 * slots), o_hit_id = take(4 * slots);
-  const uint64_t o_L = take(0);
+  uint64_t o_L = take(0);
   // the radiance arena takes the rest: at least one sample of every pixel
-  const uint64_t l_slots = off < rdh::kScratchBytes ? (rdh::kScratchBytes - off) / 16 : 0;
+  uint64_t l_slots = off < rdh::kScratchBytes ? (rdh::kScratchBytes - off) / 16 : 0;
   if (l_slots < npix)
     return r->fail(RD_ERR_INVALID_ARGUMENT,
                    "scene needs " + std::to_string(off + 16 * npix) + " bytes of the " +
                        std::to_string(rdh::kScratchBytes) +
                        "-byte static scratch (image, BVH, queues and one sample of radiance slots); "
                        "rd_render_frame has no such limit");
+  // The path kernel needs no queues: its camera-hit table takes their place,
+  // and the radiance arena what the table leaves of it (longer passes), where
+  // that still holds a sample of every pixel (images up to 3.3 M pixels; larger
+  // ones stay with the wavefront).
+  const uint64_t o_cam = (o_rest + 255) & ~255ull;
+  const uint64_t o_cam_end = (o_cam + rdh::kCamBytes * npix + 255) & ~255ull;
+  const bool cam_fits = o_cam_end + 16 * npix <= rdh::kScratchBytes;
 
   rdh::ExternalBuffers eb{};
   for (int p = 0; p < 2; ++p) {
@@ -541,6 +549,10 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   eb.seg_cap = (uint32_t)seg_cap;
   eb.l_slots = l_slots;
   eb.tickets_n = 1;
+  if (cam_fits) {
+    eb.cam = base + o_cam;
+    eb.cam_px = npix;
+  }
   se.bind_external(eb, r->eng);
 
   // new_frame (cpu.rs:135-140): timers, then the snapshot into the scratch
@@ -586,6 +598,16 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   // as many samples as the radiance slots hold, in sample order
   const std::vector<rdh::DevJob> host_jobs{job};
   const uint32_t total = r->cfg.max_sample_count;
+  rdh::DevTicket probe{};
+  probe.spp = 1;
+  if (se.takes_paths(host_jobs, {probe})) {
+    o_L = o_cam_end;
+    l_slots = (rdh::kScratchBytes - o_L) / 16;
+    eb.L = reinterpret_cast<float4 *>(base + o_L);
+    eb.l_slots = l_slots;
+    se.bind_external(eb, r->eng);
+    se.opt.grid = 0;
+  }
   if (ok && total > 0) {
     r->prepare_timer.end_if_not_ended();
     r->render_timer.start_if_not_started();
@@ -597,6 +619,7 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
       t.sample_base = done;
       t.spp = (uint32_t)std::min<uint64_t>(total - done, fit);
       t.paths = (uint32_t)(t.spp * npix);
+      se.hit_frame = 1;  // (the binding holds no earlier frame's hits)
       ok = se.run_tickets(d_job, {t}, host_jobs, &err);
       done += t.spp;
     }

@@ -66,6 +66,9 @@ void Engine::bind_external(const ExternalBuffers &b, const Engine &owner) {
   seg_cap = b.seg_cap;
   l_alloc = b.l_slots;
   ticket_alloc = b.tickets_n;
+  cam_ = b.cam;
+  cam_px_ = b.cam_px;
+  cam_frame_ = 0;
   opt.queue = b.queue;
   opt.l_capacity = b.l_slots;
   opt.pipes = 1;
@@ -117,10 +120,10 @@ uint32_t Engine::queued(const QueueCtl &c, int parity) {
 
 bool Engine::ensure_buffers(std::string *err, bool queues) {
   if (opt.queue < 1024) opt.queue = 1024;
-  const uint32_t need = queues || external_ ? segment_slots() : 0;
+  const uint32_t need = queues ? segment_slots() : 0;
   if (external_) {
     // borrowed buffers: they must already fit these options
-    if (opt.queue != q_alloc || need > seg_cap || opt.l_capacity > l_alloc) {
+    if ((queues && (opt.queue != q_alloc || need > seg_cap)) || opt.l_capacity > l_alloc) {
       *err = "launch shape needs larger borrowed buffers (internal error)";
       return false;
     }
@@ -454,8 +457,9 @@ int Engine::pipes_for(const DevJob &j, const DevTicket &t) const {
 // tree), event counts, and the launch forms asked for by option (one ray per
 // lane, other workgroup sizes, every camera ray traced).
 bool Engine::takes_paths(const std::vector<DevJob> &jobs, const std::vector<DevTicket> &tickets) const {
-  if (!launch_paths || external_ || jobs.size() != 1 || tickets.size() != 1) return false;
+  if (!launch_paths || jobs.size() != 1 || tickets.size() != 1) return false;
   const DevJob &j = jobs[0];
+  if (external_ && cam_px_ < (uint64_t)j.width * j.height) return false;
   return !opt.count && opt.hit_reuse && !opt.brute_force && opt.refill > 0 && opt.bvh4 &&
          opt.block == 256 && j.max_bounces > 0 && j.max_bounces <= 255 && tickets[0].spp < (1u << 24) &&
          j.n_nodes4 > 0 && j.n_nodes <= kNarrowStackNodes && j.stack4 + 3 <= (uint32_t)kStackDepth;

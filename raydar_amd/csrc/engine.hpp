@@ -108,6 +108,8 @@ struct ExternalBuffers {
   uint32_t seg_cap;     // slots per queue segment
   uint64_t l_slots;     // radiance slots
   uint32_t tickets_n;   // ticket table entries
+  unsigned char *cam;   // the path kernel's camera-hit table, or nullptr
+  uint64_t cam_px;      // pixels it holds
 };
 
 class Engine {

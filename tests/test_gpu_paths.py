@@ -7,12 +7,14 @@ pixels than a group of 64, groups that are not full, sample counts that do
 not divide the slices, one workgroup, turns at 1 to 64 idle lanes, a tree in
 LDS or not, leaves of several primitives, one bounce.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle
 import raydar_amd as ra
-from raydar_amd import scenegen
+from raydar_amd import abi, scenegen
 
 pytestmark = pytest.mark.gpu
 
@@ -48,6 +50,23 @@ def test_path_kernel_and_wavefront_alternate_on_one_renderer():
                 r.render_sample(sc)
             ref = oracle.render(sc, 4, 12, 5)
             np.testing.assert_array_equal(r.accumulator().view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("size,spp", [((5, 3), 3), ((640, 360), 37), ((2048, 1620), 2),
+                                      ((2048, 1650), 2)])
+def test_allocation_free_call_matches_render_frame(size, spp):
+    # the camera-hit table takes the queues' place in the static scratch while
+    # it and a sample of every pixel fit there (images up to 3.3 M pixels: the
+    # third size does, the fourth does not), in one pass or several
+    sc = scenegen.plain_1080p(3, *size)
+    out = np.zeros((sc.height, sc.width, 4), np.uint8)
+    f = ra.lib().rd_render_frame_noalloc
+    f.restype, f.argtypes = C.c_int, [C.c_void_p, C.POINTER(abi.RdScene), C.c_void_p, C.c_size_t]
+    with ra.HipRenderer(max_sample_count=spp, max_bounces=12, seed=5) as r:
+        s = sc.as_rd()
+        for _ in range(2):
+            ra.check(f(r._h, C.byref(s), out.ctypes.data_as(C.c_void_p), out.nbytes), r._h)
+        np.testing.assert_array_equal(out, r.render_frame(sc))
 
 
 @pytest.mark.parametrize("size,spp,bounces,opts", [
