@@ -276,7 +276,7 @@ rd_status render_samples(rd_renderer *r, uint32_t k) {
       // pixel's samples one after another
       rdh::DevTicket probe{};
       probe.spp = 1;
-      fit = r->eng.takes_paths(host_jobs, {probe}) ? (1u << 24) - 1u : 1u;
+      fit = r->eng.takes_paths(r->job_h, probe) ? (1u << 24) - 1u : 1u;
     }
     uint32_t spp = (uint32_t)std::min<uint64_t>({(uint64_t)(k - done), fit, 0xffffffffull / npix});
     rdh::DevTicket t{};
@@ -600,7 +600,7 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   const uint32_t total = r->cfg.max_sample_count;
   rdh::DevTicket probe{};
   probe.spp = 1;
-  if (se.takes_paths(host_jobs, {probe})) {
+  if (se.takes_paths(job, probe)) {
     o_L = o_cam_end;
     l_slots = (rdh::kScratchBytes - o_L) / 16;
     eb.L = reinterpret_cast<float4 *>(base + o_L);

@@ -66,6 +66,7 @@ void Engine::bind_external(const ExternalBuffers &b, const Engine &owner) {
   seg_cap = b.seg_cap;
   l_alloc = b.l_slots;
   ticket_alloc = b.tickets_n;
+  path_ctl_ = b.ctl;  // (no wavefront runs between the passes of a call)
   cam_ = b.cam;
   cam_px_ = b.cam_px;
   cam_frame_ = 0;
@@ -89,6 +90,7 @@ void Engine::release_buffers() {
   first_hit_px_ = 0;
   first_hit_frame_ = 0;
   if (cam_) { (void)hipFree(cam_); cam_ = nullptr; }
+  if (path_ctl_) { (void)hipFree(path_ctl_); path_ctl_ = nullptr; }
   cam_px_ = 0;
   cam_frame_ = 0;
   q_alloc = 0;
@@ -456,12 +458,10 @@ int Engine::pipes_for(const DevJob &j, const DevTicket &t) const {
 // work list, binary and deeper trees, the linear scan (a scene without a
 // tree), event counts, and the launch forms asked for by option (one ray per
 // lane, other workgroup sizes, every camera ray traced).
-bool Engine::takes_paths(const std::vector<DevJob> &jobs, const std::vector<DevTicket> &tickets) const {
-  if (!launch_paths || jobs.size() != 1 || tickets.size() != 1) return false;
-  const DevJob &j = jobs[0];
-  if (external_ && cam_px_ < (uint64_t)j.width * j.height) return false;
+bool Engine::takes_paths(const DevJob &j, const DevTicket &t) const {
+  if (!launch_paths || (external_ && cam_px_ < (uint64_t)j.width * j.height)) return false;
   return !opt.count && opt.hit_reuse && !opt.brute_force && opt.refill > 0 && opt.bvh4 &&
-         opt.block == 256 && j.max_bounces > 0 && j.max_bounces <= 255 && tickets[0].spp < (1u << 24) &&
+         opt.block == 256 && j.max_bounces > 0 && j.max_bounces <= 255 && t.spp < (1u << 24) &&
          j.n_nodes4 > 0 && j.n_nodes <= kNarrowStackNodes && j.stack4 + 3 <= (uint32_t)kStackDepth;
 }
 
@@ -476,13 +476,15 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
     if (!check(hipMalloc((void **)&cam_, kCamBytes * npix), "hipMalloc(camera hits)", err)) return false;
     cam_px_ = npix;
   }
+  if (!path_ctl_ && !check(hipMalloc(&path_ctl_, sizeof(QueueCtl)), "hipMalloc(work list)", err))
+    return false;
   // an earlier pass of the same frame recorded them
   const bool carried = frame != 0 && frame == cam_frame_;
   cam_frame_ = 0;
 
   PathArgs a{};
   a.job = d_job;
-  a.ctl = ctl;
+  a.ctl = path_ctl_;
   a.cam_ray = reinterpret_cast<float4 *>(cam_);
   a.cam_hit = reinterpret_cast<uint2 *>(cam_ + sizeof(float4) * npix);
   a.L = L;
@@ -505,7 +507,7 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
   // device counter, so the pipes' launches share one list.
   const int np = pipes_used = pipes_for(j, t);
   if (!ensure_aux(np - 1, err)) return false;
-  if (!check(launch_set_ctl(ctl, 0, 0, stream), "set ctl", err)) return false;
+  if (!check(launch_set_ctl(path_ctl_, 0, 0, stream), "set ctl", err)) return false;
   struct DrainOnError {
     Engine *e;
     bool ok = false;
@@ -516,7 +518,7 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
     }
   } drain{this};
   auto launch = [&](bool record) {
-    a.cursor = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(ctl) +
+    a.cursor = reinterpret_cast<uint32_t *>(reinterpret_cast<unsigned char *>(path_ctl_) +
                                             offsetof(QueueCtl, count)) +
                (record ? 0 : kSegments * kSegStride);
     a.spp = record || opt.vk ? 1u : t.spp;
@@ -573,7 +575,7 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
     (void)hipEventDestroy(e1);
   }
 #ifdef RDH_CHECKED
-  if (!check(hipMemcpyAsync(ctl_host, ctl, sizeof(QueueCtl), hipMemcpyDeviceToHost, stream),
+  if (!check(hipMemcpyAsync(ctl_host, path_ctl_, sizeof(QueueCtl), hipMemcpyDeviceToHost, stream),
              "read violations", err) ||
       !check(hipStreamSynchronize(stream), "paths", err))
     return false;
@@ -592,7 +594,7 @@ bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
   const uint64_t frame = hit_frame;  // set by the caller for this pass only
   hit_frame = 0;
   if (tickets.empty()) return true;
-  const bool paths = takes_paths(host_jobs, tickets);
+  const bool paths = host_jobs.size() == 1 && tickets.size() == 1 && takes_paths(host_jobs[0], tickets[0]);
   if (!ensure_buffers(err, !paths)) return false;
   uint64_t w = 0;
   uint32_t max_bounces = 1;

@@ -146,7 +146,14 @@ class Engine {
                    const std::vector<DevJob> &host_jobs, std::string *err);
 
   // Whether the path kernel renders this pass.
-  bool takes_paths(const std::vector<DevJob> &jobs, const std::vector<DevTicket> &tickets) const;
+  bool takes_paths(const DevJob &j, const DevTicket &t) const;
+  // A pass of the path kernel into the radiance slots t.l_offset.., queued on
+  // this engine's stream and not waited for (nor, but for Vulkan semantics,
+  // accumulated).  Passes with the same nonzero `frame` share the camera-ray
+  // hits the first of them records.
+  bool run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame,
+                 std::string *err);
+  uint64_t cam_bytes() const { return cam_px_ * kCamBytes; }
 
   bool check(hipError_t e, const char *what, std::string *err);
 
@@ -200,10 +207,6 @@ class Engine {
              const IterArgs &a, int parity, uint32_t bound);
   // Pipes of a one-job pass (see run_tickets).
   int pipes_for(const DevJob &j, const DevTicket &t) const;
-  // A pass of the path kernel, not waited for (and, but for Vulkan semantics,
-  // not accumulated).
-  bool run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame,
-                 std::string *err);
   bool ensure_aux(int n, std::string *err);
   bool external_ = false;  // buffers, stream and control copy are borrowed
   std::vector<hipEvent_t> ev_pool_;
@@ -214,6 +217,8 @@ class Engine {
   HitWord *first_hit_ = nullptr;              // per-pixel camera-ray hits (IterArgs::first_hit)
   uint64_t first_hit_px_ = 0;                 // pixels first_hit_ holds
   uint64_t first_hit_frame_ = 0;              // hit_frame whose hits first_hit_ holds (0: none)
+  QueueCtl *path_ctl_ = nullptr;              // the path kernel's work-list counters (`ctl`
+                                              // may hold a wavefront's queues meanwhile)
   unsigned char *cam_ = nullptr;              // the path kernel's camera-hit table
   uint64_t cam_px_ = 0;                       // pixels it holds
   uint64_t cam_frame_ = 0;                    // hit_frame whose hits it holds (0: none)

@@ -52,6 +52,29 @@ def test_path_kernel_and_wavefront_alternate_on_one_renderer():
             np.testing.assert_array_equal(r.accumulator().view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("opts", [dict(pipes=1), dict(pipes=1, ticket_cap=3), dict(pipes=2),
+                                  dict(pipes=1, queue=4096), dict(pipes=1, l_capacity=1 << 16)])
+def test_batch_mixes_path_kernel_and_wavefront_jobs(opts):
+    # one streamer's ticket list holds passes of both: a scene without a tree
+    # is the wavefront's, the others are the path kernel's
+    from raydar_amd.batch import BatchRenderer, Job
+    empty = scenegen.plain_small(0)
+    empty.objects = empty.objects[:0]
+    specs = [(scenegen.clustered(5, 300, 96, 64), 5, 12, 12), (empty, 3, 12, 1),
+             (scenegen.plain_1080p(1, 120, 68), 4, 12, 13), (empty, 2, 4, 2),
+             (scenegen.plain_1080p(1, 7, 5), 9, 3, 14)]
+    jobs = [Job(s, spp, b, seed, pass_samples=2, progress=k % 2 == 0)
+            for k, (s, spp, b, seed) in enumerate(specs)]
+    with BatchRenderer(**opts) as br:
+        for _ in range(2):
+            br.render(jobs)
+            for job, (s, spp, b, seed) in zip(jobs, specs):
+                ref = oracle.render(s, spp, b, seed)
+                np.testing.assert_array_equal(job.acc.view(np.uint32), ref.view(np.uint32))
+                np.testing.assert_array_equal(job.rgba.reshape(-1), oracle.tonemap(ref, spp))
+                job.acc[:] = 0
+
+
 @pytest.mark.parametrize("size,spp", [((5, 3), 3), ((640, 360), 37), ((2048, 1620), 2),
                                       ((2048, 1650), 2)])
 def test_allocation_free_call_matches_render_frame(size, spp):
