@@ -495,7 +495,7 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
   a.samples = t.spp;
   a.vk = opt.vk;
   a.refill = (uint32_t)opt.refill;
-  a.stack_rows = j.stack4 + 3;
+  a.stack_rows = j.stack4 + 4;  // a sentinel below, and three written above the top
   a.leaf1 = j.max_leaf == 1 ? 1 : 0;
   const uint64_t tree = sizeof(DevNode4) * (uint64_t)j.n_nodes4 + sizeof(DevPrim) * (uint64_t)j.n_prims;
   a.lds_bvh_bytes = tree <= opt.lds_bvh ? (uint32_t)tree : 0u;

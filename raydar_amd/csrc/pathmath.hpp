@@ -38,26 +38,75 @@ RD_HD F3 neg(F3 a) { return f3(-a.x, -a.y, -a.z); }
 RD_HD F3 scale(F3 a, float s) { return f3(a.x * s, a.y * s, a.z * s); }
 RD_HD F3 mul(F3 a, F3 b) { return f3(a.x * b.x, a.y * b.y, a.z * b.z); }
 RD_HD float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-RD_HD F3 normalize(F3 v) { return scale(v, 1.0f / sqrtf(dot(v, v))); }
+RD_HD F3 normalize(F3 v);
 // Rust f32::signum: +-1 by the sign bit (so -0.0 -> -1.0), NaN stays NaN.
 RD_HD float signum(float v) { return isnan(v) ? v : copysignf(1.0f, v); }
 RD_HD uint32_t fbits(float v) { return __builtin_bit_cast(uint32_t, v); }
 RD_HD float bitsf(uint32_t v) { return __builtin_bit_cast(float, v); }
-// sqrtf, correctly rounded.  On the GPU, for x >= 2^-96 (no scaling needed),
-// the hardware square root s (within 1 ulp) is corrected by the sign of the
-// exact residuals x - s'*s of its neighbours s' = s -+ 1 ulp (fma is exact
-// enough to decide which of the three is the rounded root); other x take
-// sqrtf.
+// sqrtf, correctly rounded.  On the GPU, for x in [2^-96, 2^100), one fused
+// correction of x * rsq(x) by its residual (Markstein, IBM J. Res. Dev. 34(1),
+// 1990): equal to the IEEE root for all significands of an even and an odd
+// exponent (2^24 values, enumerated on gfx950; a power of four scales both
+// alike), in 5 instructions.  Other x take sqrtf: the fast form first for every
+// lane, then the others again (a branch around each form costs three times
+// the scalar instructions).
+#if defined(__HIPCC__)
+__device__ __forceinline__ float sqrt_rn_normal(float x) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+}
+__device__ __forceinline__ float rcp_rn_normal(float x) {
+  const float y = __builtin_amdgcn_rcpf(x);
+  return fmaf(fmaf(-x, y, 1.0f), y, y);
+}
+// x outside the positive range [2^lo, 2^hi)
+__device__ __forceinline__ bool outside_pow2(float x, int lo, int hi) {
+  const uint32_t b = (uint32_t)(lo + 127) << 23;
+  return fbits(x) - b >= ((uint32_t)(hi + 127) << 23) - b;
+}
+#endif
 RD_HD float sqrt_rn(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (x >= 0x1p-96f) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float sd = bitsf(fbits(s) - 1u), su = bitsf(fbits(s) + 1u);
-    const float r = fmaf(-sd, s, x) <= 0.0f ? sd : s;
-    return fmaf(-su, s, x) > 0.0f ? su : r;
-  }
-#endif
+  float r = sqrt_rn_normal(x);
+  if (outside_pow2(x, -96, 100)) r = sqrtf(x);
+  return r;
+#else
   return sqrtf(x);
+#endif
+}
+// 1 / x, correctly rounded.  On the GPU, for |x| in [2^-60, 2^60), the
+// hardware reciprocal (within 1 ulp) and one Newton step: equal to the IEEE
+// quotient for all 2^23 significands (enumerated on gfx950; a power of two
+// scales both alike), in 3 instructions instead of 10.
+RD_HD float rcp_rn(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  float r = rcp_rn_normal(x);
+  if (outside_pow2(fabsf(x), -60, 60)) r = 1.0f / x;
+  return r;
+#else
+  return 1.0f / x;
+#endif
+}
+RD_HD F3 normalize(F3 v) {
+  const float q = dot(v, v);
+#if defined(__HIP_DEVICE_COMPILE__)
+  float y = rcp_rn_normal(sqrt_rn_normal(q));
+  if (outside_pow2(q, -96, 96)) y = 1.0f / sqrtf(q);
+#else
+  const float y = 1.0f / sqrtf(q);
+#endif
+  return scale(v, y);
+}
+// n / a, correctly rounded, from y = RN(1/a): one fused correction of the
+// product's remainder (Markstein, IBM J. Res. Dev. 34(1), 1990).  For |n| in
+// [2^-60, 2^60] and |a| in [2^-20, 2^20] the remainder does not underflow; the
+// quotients within 20 / a of a rounding midpoint, for all 2^23 divisor
+// significands (5.0e8 of them), were enumerated and all round as IEEE
+// division does.
+RD_HD float div_rn(float n, float a, float y) {
+  const float q = n * y;
+  return fmaf(fmaf(-a, q, n), y, q);
 }
 
 // -------------------------------------------------------------- Philox ----
@@ -65,6 +114,13 @@ RD_HD float sqrt_rn(float x) {
 struct U4 {
   uint32_t v[4];
 };
+RD_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);  // one instruction
+#else
+  return a ^ b ^ c;
+#endif
+}
 RD_HD U4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
                        uint32_t k1) {
 #pragma unroll
@@ -75,8 +131,8 @@ RD_HD U4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint3
     }
     const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
     const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-    const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
-    const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+    const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0);
+    const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
     c1 = (uint32_t)p1;
     c3 = (uint32_t)p0;
     c0 = n0;
@@ -232,15 +288,14 @@ struct SlabRay {
   float ax, ay, az;     // (o + tol) * inv
   float bx, by, bz;     // (o - tol) * inv
 };
-// On the GPU the reciprocal is the hardware's (within 1 ulp instead of half
-// an ulp): the box test is a cull, and the rounding margin every box carries
-// (1e-6 L, the padding note of bvh.cpp) covers the extra 2^-24 relative error
-// of each plane distance; the near/far plane order below holds for any
-// positive scale.
+// On the GPU the reciprocal is rcp_rn's fast form, the rounded one for every
+// |d| in [2^-60, 2^60); outside that it may be off by an ulp, which the
+// rounding margin every box carries (1e-6 L, the padding note of bvh.cpp)
+// covers.
 RD_HD float safe_inv(float d) {
   const float m = fabsf(d) < 1e-30f ? copysignf(1e-30f, d) : d;
 #if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_rcpf(m);
+  return rcp_rn_normal(m);
 #else
   return 1.0f / m;
 #endif
@@ -365,13 +420,13 @@ RD_HD F3 reflect(F3 v, F3 n) { return sub(v, scale(scale(n, dot(v, n)), 2.0f)); 
 RD_HD F3 refract(F3 v, F3 n, float eta) {
   const float cos_t = fminf(dot(v, neg(n)), 1.0f);
   const F3 perp = scale(add(v, scale(n, cos_t)), eta);
-  const float s = sqrtf(fabsf(1.0f - dot(perp, perp)));
+  const float s = sqrt_rn(fabsf(1.0f - dot(perp, perp)));
   return add(perp, scale(n, -s));
 }
 // utils/mod.rs:37-44
 RD_HD bool can_refract(F3 v, F3 n, float eta) {
   const float cos_t = fminf(dot(v, neg(n)), 1.0f);
-  const float sin_t = sqrtf(1.0f - cos_t * cos_t);
+  const float sin_t = sqrt_rn(1.0f - cos_t * cos_t);
   return eta * sin_t <= 1.0f;
 }
 // utils/mod.rs:47-55: normalize(U[-1,1]^3)
@@ -448,7 +503,7 @@ RD_HD ScatterOut scatter(F3 ray_d, const HitRec &h, const DevObject &ob, Draws &
 RD_HD F3 world_sample(const DevJob &j, F3 d) {
   if (j.world_kind == RD_WORLD_SOLID_COLOR) return f3(j.solid[0], j.solid[1], j.solid[2]);
   const F3 up = f3(0.0f, 1.0f, 0.0f);
-  const float cs = dot(d, up) / (sqrtf(dot(d, d)) * sqrtf(dot(up, up)));
+  const float cs = dot(d, up) / (sqrt_rn(dot(d, d)) * sqrtf(dot(up, up)));
   const F3 bottom = f3(j.bottom[0], j.bottom[1], j.bottom[2]);
   const F3 top = f3(j.top[0], j.top[1], j.top[2]);
   return add(bottom, scale(sub(top, bottom), (cs + 1.0f) * 0.5f));

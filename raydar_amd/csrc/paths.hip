@@ -13,15 +13,21 @@
 // draw is keyed by (pixel, sample, bounce), so the image is the same bit for
 // bit.
 //
-// What bounds it: VALU issue (99% busy on 97 objects in LDS), then the node
-// fetches of a tree outside LDS.  Against the wavefront it gains most in
-// shading: a turn shades only lanes that hit something (a wavefront tile is a
-// third misses), and no lane waits for a path's record to come back from HBM.
-// 77% of the lanes work in an average VALU instruction (wavefront: 54% in
-// extend, 58% in shade).  Measured, wavefront -> paths: 97 objects at 1080p,
-// 64 spp 20.0 -> 12.8 ms; 4096 objects 19.9 -> 17.7 ms; a closed room at
-// 960x540, 16 spp 6.1 -> 4.3 ms; 256x256, 16 spp, whole call 0.56 -> 0.31 ms;
-// one sample at 1080p with a new scene 1.28 -> 1.00 ms.
+// What bounds it: the issue of instructions, one of any kind (scalar ones too)
+// per SIMD and about 2.1 cycles; for a tree outside LDS the L1's rate of node
+// fetches as well.  Against the wavefront it gains most in shading: a turn
+// shades only lanes that hit something (a wavefront tile is a third misses),
+// and no lane waits for a path's record to come back from HBM.  A quarter of
+// the instructions (1.41e10 -> 1.07e10 on the first case below, scalar ones
+// 3.8e9 -> 1.9e9) went with: the inner loop of the walk, which looks at one
+// ballot instead of three; visit order from integer min/med/max; a stack whose
+// pops need no look at the depth; one division a sphere, exact short forms of
+// the roots and reciprocals (pathmath.hpp); camera misses recorded as their
+// radiance.  Measured, wavefront -> paths -> with those: 97 objects at 1080p,
+// 64 spp 20.0 -> 12.7 -> 10.8 ms; 4096 objects 22.4 -> 18.5 -> 16.1 ms; a
+// closed room at 960x540, 16 spp 6.1 -> 4.6 -> 3.8 ms; 183 objects at 4K, 8 spp
+// 15.7 -> 10.2 -> 9.6 ms; 256x256, 16 spp, whole call 0.56 -> 0.32 -> 0.29 ms;
+// one sample at 1080p with a new scene 1.28 -> 1.03 -> 0.94 ms.
 #include <algorithm>
 
 #include "kernel_util.hpp"
@@ -31,11 +37,120 @@ namespace rdh {
 
 namespace {
 
-// Waves per SIMD the path kernel is compiled for.
-#ifndef RDH_PATH_WAVES
-#define RDH_PATH_WAVES 6
-#endif
-constexpr int path_waves(bool record, bool vk) { return vk && !record ? 5 : RDH_PATH_WAVES; }
+// Waves per SIMD the path kernel is compiled for: what its registers allow.
+// Six spill 30 registers around the shading (97 objects at 1080p, 64 spp 12.8
+// against 10.8 ms), four are too few (11.6 ms); with Vulkan semantics, whose
+// lanes also hold the stream's state and the rank, four are the faster by 2 %.
+constexpr int path_waves(bool record, bool vk) { return vk && !record ? 4 : 5; }
+
+// A pooled walk puts the primitives of the leaves it enters on a per-lane list
+// in LDS and tests one of each lane's once kPoolTests lanes have one, so that a
+// test runs with many lanes instead of the few that entered a leaf in this
+// step.  It pays where a step waits for memory: 4096 objects at 1080p, 64 spp
+// 17.3 -> 16.0 ms, 183 at 4K, 8 spp 9.6 -> 9.4 (8 or 12 lanes alike, 16 16.3 ms,
+// 24 17.6); a tree in LDS loses, as the rays' culling distances shrink later:
+// 97 objects 10.8 -> 11.0 ms.  The list's rows: a step adds up to four and
+// writes one past what it keeps, so it starts with at most four in it.
+constexpr uint32_t kPoolTests = 12, kPoolRows = 8;
+template <int BLOCK>
+__host__ __device__ constexpr uint32_t pool_bytes() {
+  return kPoolRows * BLOCK * (uint32_t)sizeof(uint16_t);
+}
+__host__ __device__ constexpr bool pooled(bool lds, bool leaf1) { return leaf1 && !lds; }
+
+// Visit keys of the walk: see the sort in k_paths.
+constexpr uint32_t kNoKey = 0xffffffffu;
+constexpr uint32_t kNoNode = 0xffffu;  // no 4-wide tree with 16-bit entries has this index
+__device__ __forceinline__ uint32_t umin(uint32_t a, uint32_t b) { return a < b ? a : b; }
+__device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
+__device__ __forceinline__ uint32_t umed3(uint32_t a, uint32_t b, uint32_t c) {
+  return umin(umax(a, b), umax(umin(a, b), c));
+}
+
+// A walk's ray: dot(d, d) in [kMinDot, kMaxDot] besides walkable().
+constexpr float kMinDot = 0x1p-20f, kMaxDot = 0x1p20f;
+
+// hit_sphere (cpu.rs:34-62) for a ray of a walk; NaN or negative: no hit.  The
+// reference returns t1 = (-k - s) / a if that is >= 0, else t2 = (-k + s) / a if
+// that is.  With a in [2^-20, 2^20] the sign of t1 is its numerator's (s is 0
+// or at least 2^-75, so a negative -k - s is at most -2^-99 unless s = 0, and
+// its quotient no underflow; with s = 0 both numerators are the same), so one
+// division does, and that by the ray's ya = RN(1/a) (div_rn).
+__device__ __forceinline__ float sphere_distance(const RayPre &r, float ya, const DevPrim &p) {
+  const float dC = r.dx * p.a[0] + r.dy * p.a[1] + r.dz * p.a[2];
+  const float oC = r.ox * p.a[0] + r.oy * p.a[1] + r.oz * p.a[2];
+  const float k = r.od - dC;
+  const float c = r.oo - 2.0f * oC + p.a[3] - p.b[0];
+  const float disc = k * k - r.a * c;
+  const float s = sqrt_rn_normal(disc);  // NaN for a miss
+  const float n1 = -k - s;
+  const float n = n1 >= 0.0f ? n1 : -k + s;
+  float t = div_rn(n, r.a, ya);
+  // a tiny or overflown discriminant, a tiny numerator: as written (and -0 as
+  // +0, which no comparison and no hit point tells apart)
+  const bool slow = (fbits(disc) < 0x0f800000u) | ((int32_t)fbits(disc) >= 0x71800000) |
+                    (fabsf(n) < 0x1p-60f);
+  if (__ballot(slow) != 0) {
+    if (slow) {
+      const float s0 = sqrtf(disc);
+      const float m1 = -k - s0;
+      t = (m1 >= 0.0f ? m1 : -k + s0) / r.a + 0.0f;
+    }
+  }
+  return t;
+}
+
+// hit_cube (cpu.rs:64-98) for a ray of a walk; NaN: no hit.  The six quotients
+// by div_rn with the ray's i = RN(1/d), where d and the numerators allow.
+template <bool VK>
+__device__ __forceinline__ float cube_from(float q0, float q1, float q2, float q3, float q4, float q5) {
+  const float tmin = fmaxf(fmaxf(fminf(q0, q1), fminf(q2, q3)), fminf(q4, q5));
+  const float tmax = fminf(fminf(fmaxf(q0, q1), fmaxf(q2, q3)), fmaxf(q4, q5));
+  if (VK) return !(tmax >= kVkTMin) || tmin > tmax ? NAN : tmin >= kVkTMin ? tmin : tmax;
+  // tmax < 0 or tmin > tmax: no hit; from inside the exit
+  return fmaxf(tmin, 0.0f) > tmax ? NAN : tmin < 0.0f ? tmax : tmin;
+}
+template <bool VK>
+__device__ __forceinline__ float cube_distance(const RayPre &r, float ix, float iy, float iz,
+                                               const DevPrim &p) {
+  const float n0 = p.a[0] - r.ox, n1 = p.b[0] - r.ox, n2 = p.a[1] - r.oy;
+  const float n3 = p.b[1] - r.oy, n4 = p.a[2] - r.oz, n5 = p.b[2] - r.oz;
+  float t = cube_from<VK>(div_rn(n0, r.dx, ix), div_rn(n1, r.dx, ix), div_rn(n2, r.dy, iy),
+                          div_rn(n3, r.dy, iy), div_rn(n4, r.dz, iz), div_rn(n5, r.dz, iz));
+  const float nl = fminf(fminf(fminf(fabsf(n0), fabsf(n1)), fminf(fabsf(n2), fabsf(n3))),
+                         fminf(fabsf(n4), fabsf(n5)));
+  const float nh = fmaxf(fmaxf(fmaxf(fabsf(n0), fabsf(n1)), fmaxf(fabsf(n2), fabsf(n3))),
+                         fmaxf(fabsf(n4), fabsf(n5)));
+  const float dl = fminf(fminf(fabsf(r.dx), fabsf(r.dy)), fabsf(r.dz));
+  const bool slow = !((nl >= 0x1p-60f) & (nh <= 0x1p60f) & (dl >= 0x1p-20f));
+  if (__ballot(slow) != 0) {
+    if (slow)
+      t = cube_from<VK>(n0 / r.dx, n1 / r.dx, n2 / r.dy, n3 / r.dy, n4 / r.dz, n5 / r.dz) + 0.0f;
+  }
+  return t;
+}
+
+// A walk's best hit: distance bits above the object's index.  No distance is
+// NaN in a walk (a sphere's is >= 0, and some component of d is not zero) or
+// -0, so unsigned order is better_hit's: the smaller distance, then the lower
+// index, with misses (NaN, negative) above the +inf that stands for no hit.
+constexpr uint64_t kNoBest = ((uint64_t)0x7f800000u << 32) | kNoHit;
+
+template <bool VK>
+__device__ __forceinline__ void test_in_walk(const RayPre &r, float ya, float ix, float iy, float iz,
+                                             const DevPrim &p, uint64_t *best) {
+  const uint32_t tag = fbits(p.b[3]);
+  const bool cube = (tag & kTagCube) != 0u;
+  float t = NAN;
+  if (__ballot(!cube) != 0) t = sphere_distance(r, ya, p);
+  if (__ballot(cube) != 0) {
+    const float tc = cube_distance<VK>(r, ix, iy, iz, p);
+    t = cube ? tc : t;
+  }
+  if (VK && !(t >= kVkTMin && t <= kVkTMax)) t = NAN;
+  const uint64_t key = ((uint64_t)fbits(t) << 32) | (tag & ~kTagCube);
+  if (key < *best) *best = key;
+}
 
 // The camera rays' common origin.
 template <bool VK>
@@ -55,12 +170,12 @@ __device__ __forceinline__ F3 camera_origin(const DevJob &J) {
 // state in a register, and adds each to the accumulator itself (the order
 // k_accumulate would take).  The camera ray has no draw in it here either.
 // 97 objects, 1280x720, 16 spp: 8.1 -> 3.5 ms, which were 16 passes of one
-// sample with 12 bounces of three launches each; 5 waves per SIMD, as the
-// stream and rank do not fit the registers of 6.
+// sample with 12 bounces of three launches each; 2.8 ms with the shorter walk.
 template <int BLOCK, bool RECORD, bool LDS, bool LEAF1, bool VK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(path_waves(RECORD, VK), 8)))
 void k_paths(PathArgs a) {
   typedef uint16_t StackT;
+  constexpr bool kPooled = pooled(LDS, LEAF1);
   extern __shared__ __align__(16) unsigned char dynamic_lds[];
   // Job fields are scalar loads.  What a walk needs stays in registers; the
   // shading's fields are read again in every turn: held across the walk, they
@@ -72,15 +187,32 @@ void k_paths(PathArgs a) {
   const uint32_t n_nodes4 = load_constant(&a.job->n_nodes4), n_prims = load_constant(&a.job->n_prims);
   (void)n_nodes4;
   const uint32_t stack_bytes = (a.stack_rows * BLOCK * (uint32_t)sizeof(StackT) + 15u) & ~15u;
-  StackT *stk = reinterpret_cast<StackT *>(dynamic_lds) + threadIdx.x;
-  VecF4 *lds_nodes = reinterpret_cast<VecF4 *>(dynamic_lds + stack_bytes);
+  // The lane's stack column: rows of kRow bytes, the last holding kNoNode for
+  // good, so that a pop needs no look at the depth.
+  constexpr uint32_t kRow = BLOCK * (uint32_t)sizeof(StackT);
+  const uint32_t stack_first = (a.stack_rows - 2u) * kRow + threadIdx.x * (uint32_t)sizeof(StackT);
+  auto stack_at = [&](uint32_t off) -> StackT & { return *reinterpret_cast<StackT *>(dynamic_lds + off); };
+  stack_at(stack_first + kRow) = (StackT)kNoNode;
+  // a pooled walk's primitives entered but not yet tested: kPoolRows rows
+  const uint32_t pool_first = stack_bytes + threadIdx.x * (uint32_t)sizeof(StackT);
+  VecF4 *lds_nodes = reinterpret_cast<VecF4 *>(dynamic_lds + stack_bytes + (kPooled ? pool_bytes<BLOCK>() : 0u));
   const uint32_t node_vecs = LDS ? 8 * n_nodes4 : 0u, prim_vecs = LDS ? 2 * n_prims : 0u;
   VecF4 *lds_prims = lds_nodes + node_vecs;
   VecF4 *lds_objects = lds_prims + prim_vecs;
   const bool lds_obj = !RECORD && a.lds_obj_bytes != 0;
   if (LDS) {
     GlobalF4 *gn = (GlobalF4 *)nodes4, *gp = (GlobalF4 *)prims;
-    for (uint32_t i = threadIdx.x; i < node_vecs; i += BLOCK) lds_nodes[i] = gn[i];
+    for (uint32_t i = threadIdx.x; i < node_vecs; i += BLOCK) {
+      VecF4 v = gn[i];
+      if (LEAF1 && (i & 7u) == 6u) {
+        // the children's codes: a one-primitive leaf's becomes its primitive's index
+        VecI4 c = __builtin_bit_cast(VecI4, v);
+        for (int k = 0; k < 4; ++k)
+          if (is_leaf(c[k])) c[k] = (int32_t)(0x80000000u | leaf_first(c[k]));
+        v = __builtin_bit_cast(VecF4, c);
+      }
+      lds_nodes[i] = v;
+    }
     for (uint32_t i = threadIdx.x; i < prim_vecs; i += BLOCK) lds_prims[i] = gp[i];
   }
   if (lds_obj) {
@@ -101,8 +233,10 @@ void k_paths(PathArgs a) {
   const uint32_t slice = blockIdx.x % a.slices;
   const uint32_t slice_chunks = (a.chunks + a.slices - 1u - slice) / a.slices;
   const float cull0 = VK ? cull_limit(kVkTMax, 0u) : INFINITY;  // with no hit yet
-  // A lane is walking (active), waits to be shaded (full) or is free.
-  bool active = false, full = false;
+  // A lane is free (!has), or its path walks (nodes to visit: node != kNoNode;
+  // with a pool, primitives to test: pool != pool_first), or waits to be shaded.
+  bool has = false;
+  uint32_t pool = pool_first;  // byte offset of the pool's next free entry
   // The wave's chunk (group, sample, paths handed out) and the chunks of its
   // last request still to come: wave-uniform.
   uint32_t group = 0, sample = 0, off = 64, left = 0;
@@ -115,12 +249,13 @@ void k_paths(PathArgs a) {
   F3 at = f3(1.0f, 1.0f, 1.0f), li = f3(0.0f, 0.0f, 0.0f);
   uint32_t pixel = 0, sb = 0;      // sample in the pass << 8 | bounce (RECORD: the rank)
   uint32_t vk_rank = 0, vk_state = 0;  // VK: the pixel's rank and random-number state
-  float bt = 0.0f, tcull = INFINITY;
-  uint32_t bid = kNoHit;
-  int32_t node = 0;
-  int sp = 0;
+  uint64_t best = kNoBest;         // the walk's or the waiting path's hit
+  float tcull = INFINITY;
+  uint32_t node = kNoNode;
+  uint32_t sp = 0;          // byte offset two rows past the next stack entry to write
   RayPre r;
   SlabNF nf;
+  float ya = 0.0f;  // RN(1 / dot(d, d))
 
   // The lane's path ends with radiance c.  VK: the pixel's next sample, if the
   // pass has one, waits at the camera ray's hit.
@@ -133,132 +268,151 @@ void k_paths(PathArgs a) {
         const float4 cr = a.cam_ray[vk_rank];
         o = camera_origin<VK>(J);
         d = f3(cr.x, cr.y, cr.z);
-        bt = cr.w;
-        bid = a.cam_hit[vk_rank].x;
+        best = ((uint64_t)fbits(cr.w) << 32) | a.cam_hit[vk_rank].x;
         at = f3(1.0f, 1.0f, 1.0f);
         li = f3(0.0f, 0.0f, 0.0f);
         sb = ((sb >> 8) + 1u) << 8;
-        full = true;
       } else {
         J.vk_rng[pixel] = vk_state;
+        has = false;
       }
-      return;
+    } else {
+      const unsigned long long slot =
+          a.l_offset + (unsigned long long)(sb >> 8) * a.npix + pixel;
+      a.L[chk(slot, a.l_cap, K_RADIANCE, a.ctl)] = make_float4(c.x, c.y, c.z, 1.0f);
+      has = false;
     }
-    const unsigned long long slot =
-        a.l_offset + (unsigned long long)(sb >> 8) * a.npix + pixel;
-    a.L[chk(slot, a.l_cap, K_RADIANCE, a.ctl)] = make_float4(c.x, c.y, c.z, 1.0f);
   };
+  auto walking = [&]() { return kPooled ? node != kNoNode || pool != pool_first : node != kNoNode; };
+  auto hit_id = [&]() { return (uint32_t)best; };
+  auto hit_t = [&]() { return bitsf((uint32_t)(best >> 32)); };
+  // the walk's culling distance (VK: hits beyond t_max do not count)
+  auto cull = [&]() {
+    const float c = hit_t() * 1.0001f + 1e-30f;
+    return VK ? fminf(c, cull0) : c;
+  };
+  auto test = [&](uint32_t j) {
+#ifdef RDH_CHECKED
+    j = chk(j, n_prims, K_PRIM, a.ctl);
+#endif
+    DevPrim pr;
+    if (LDS) {
+      const VecF4 pa = lds_prims[2 * j], pb = lds_prims[2 * j + 1];
+      pr.a[0] = pa.x; pr.a[1] = pa.y; pr.a[2] = pa.z; pr.a[3] = pa.w;
+      pr.b[0] = pb.x; pr.b[1] = pb.y; pr.b[2] = pb.z; pr.b[3] = pb.w;
+    } else {
+      load_prim(prims, j, &pr);
+    }
+    test_in_walk<VK>(r, ya, nf.ix, nf.iy, nf.iz, pr, &best);
+  };
+  // the primitive of a one-primitive leaf (in LDS the code is the index)
+  auto leaf_prim = [&](int32_t code) { return (uint16_t)(LDS && LEAF1 ? code : code >> 4); };
 
   for (;;) {
-    const uint64_t walking = __ballot(active), waiting = __ballot(full);
-    // With work left every lane that is not walking can be put to use; once
-    // the list is empty a lane is only worth shading when it waits, and the
-    // wave shades when three quarters of its live lanes do.
-    const uint32_t live = (uint32_t)__popcll(walking | waiting);
-    const bool turn = more ? 64u - (uint32_t)__popcll(walking) >= a.refill
-                           : 4u * (uint32_t)__popcll(waiting) >= 3u * live;
-    if (turn || walking == 0) {
-      if (!more && live == 0) break;
-      const DevJob J = load_constant(a.job);
-      if constexpr (RECORD) {
-        if (full) {
-          a.cam_ray[sb] = make_float4(d.x, d.y, d.z, bid == kNoHit ? 0.0f : bt);
-          a.cam_hit[sb] = make_uint2(bid, pixel);
-          full = false;
-        }
-      } else if (full && bid == kNoHit) {
-        // cpu.rs:334-337 (raytrace.rgen:178)
-        full = false;
-        finish(J, add(li, mul(VK ? world_sample_vk(J, d) : world_sample(J, d), at)));
+    // ---- a turn: shade the lanes whose walk has ended, refill the free ones
+    const DevJob J = load_constant(a.job);
+    bool full = has && !walking(), fresh = false;
+    if constexpr (RECORD) {
+      if (full) {
+        const bool hit = hit_id() != kNoHit;
+        // a pixel whose camera ray leaves the scene: its samples' radiance
+        const F3 c = add(f3(0.0f, 0.0f, 0.0f), mul(VK ? world_sample_vk(J, d) : world_sample(J, d),
+                                                   f3(1.0f, 1.0f, 1.0f)));
+        a.cam_ray[sb] = hit ? make_float4(d.x, d.y, d.z, hit_t()) : make_float4(c.x, c.y, c.z, 0.0f);
+        a.cam_hit[sb] = make_uint2(hit_id(), pixel);
+        has = full = false;
       }
-      // Free lanes take the next paths.  A camera path starts at its pixel's
-      // recorded hit, so it is shaded in this turn with the lanes that
-      // finished a walk; one that left the scene ends at once, and its lane
-      // asks again.
-      bool fresh = false;
-      while (more) {
-        const uint64_t need = __ballot(!active && !full);
-        if ((uint32_t)__popcll(need) < few) break;
-        const uint32_t in_group = a.npix - group * 64u;
-        const uint32_t size = in_group < 64u ? in_group : 64u;
-        if (off >= size) {
-          // the next chunk of the request, or a new request
-          off = 0;
-          if (left > 0) {
-            --left;
-            group += a.step_groups;
-            sample += a.step_samples;
-            if (sample >= a.spp) {
-              sample -= a.spp;
-              ++group;
-            }
-          } else {
-            uint32_t w = 0;
-            if (lane == 0) w = atomicAdd(&a.cursor[slice * kSegStride], a.request);
-            w = __builtin_amdgcn_readfirstlane(w);
-            if (w >= slice_chunks) {
-              more = false;
-              break;
-            }
-            left = (slice_chunks - w < a.request ? slice_chunks - w : a.request) - 1u;
-            const uint32_t chunk = w * a.slices + slice;
-            group = __builtin_amdgcn_readfirstlane(chunk / a.spp);
-            sample = chunk - group * a.spp;
+    } else {
+      if (full && hit_id() == kNoHit) {
+        // cpu.rs:334-337 (raytrace.rgen:178)
+        finish(J, add(li, mul(VK ? world_sample_vk(J, d) : world_sample(J, d), at)));
+        full = has;
+      }
+    }
+    // Free lanes take the next paths.  A camera path starts at its pixel's
+    // recorded hit, so it is shaded in this turn with the lanes that finished
+    // a walk; one that left the scene ends at once, and its lane asks again.
+    while (more) {
+      const uint64_t need = __ballot(!has);
+      if ((uint32_t)__popcll(need) < few) break;
+      const uint32_t in_group = a.npix - group * 64u;
+      const uint32_t size = in_group < 64u ? in_group : 64u;
+      if (off >= size) {
+        // the next chunk of the request, or a new request
+        off = 0;
+        if (left > 0) {
+          --left;
+          group += a.step_groups;
+          sample += a.step_samples;
+          if (sample >= a.spp) {
+            sample -= a.spp;
+            ++group;
           }
-          continue;
+        } else {
+          uint32_t w = 0;
+          if (lane == 0) w = atomicAdd(&a.cursor[slice * kSegStride], a.request);
+          w = __builtin_amdgcn_readfirstlane(w);
+          if (w >= slice_chunks) {
+            more = false;
+            break;
+          }
+          left = (slice_chunks - w < a.request ? slice_chunks - w : a.request) - 1u;
+          const uint32_t chunk = w * a.slices + slice;
+          group = __builtin_amdgcn_readfirstlane(chunk / a.spp);
+          sample = chunk - group * a.spp;
         }
-        const uint32_t k = off + lanes_below(need);
-        if (!active && !full && k < size) {
-          const uint32_t rank = chk(group * 64u + k, a.npix, K_RADIANCE, a.ctl);
-          if constexpr (RECORD) {
-            pixel = tile_order_pixel(rank, J.width, J.height);
-            if (VK) camera_ray_vk(J, pixel % J.width, pixel / J.width, &o, &d);
-            else camera_ray(J, pixel % J.width, pixel / J.width, &o, &d);
-            sb = rank;
-            fresh = true;
-            full = true;  // (until its walk starts below)
-          } else {
-            const float4 cr = a.cam_ray[rank];
-            const uint2 ch = a.cam_hit[rank];
+        continue;
+      }
+      const uint32_t k = off + lanes_below(need);
+      if (!has && k < size) {
+        const uint32_t rank = chk(group * 64u + k, a.npix, K_RADIANCE, a.ctl);
+        has = true;
+        if constexpr (RECORD) {
+          pixel = tile_order_pixel(rank, J.width, J.height);
+          if constexpr (VK) camera_ray_vk(J, pixel % J.width, pixel / J.width, &o, &d);
+          else camera_ray(J, pixel % J.width, pixel / J.width, &o, &d);
+          sb = rank;
+          fresh = true;
+        } else {
+          const float4 cr = a.cam_ray[rank];
+          const uint2 ch = a.cam_hit[rank];
+          pixel = ch.y;
+          sb = sample << 8;
+          if constexpr (VK) {
+            vk_rank = rank;
+            vk_state = a.sample_base == 0 ? pixel % J.width + (pixel / J.width) * 1000u : J.vk_rng[pixel];
+          }
+          if (ch.x != kNoHit) {
             o = camera_origin<VK>(J);
             d = f3(cr.x, cr.y, cr.z);
-            bt = cr.w;
-            bid = ch.x;
-            pixel = ch.y;
-            sb = sample << 8;
+            best = ((uint64_t)fbits(cr.w) << 32) | ch.x;
             // a camera path's attenuation and light (cpu.rs:253-254)
             at = f3(1.0f, 1.0f, 1.0f);
             li = f3(0.0f, 0.0f, 0.0f);
-            if constexpr (VK) {
-              vk_rank = rank;
-              vk_state = a.sample_base == 0 ? pixel % J.width + (pixel / J.width) * 1000u : J.vk_rng[pixel];
-            }
-            if (bid != kNoHit) {
-              full = true;
-            } else {
-              const F3 c = add(li, mul(VK ? world_sample_vk(J, d) : world_sample(J, d), at));
-              if constexpr (VK) {
-                // every sample of the pixel is this one and draws nothing
-                float4 *acc = reinterpret_cast<float4 *>(J.acc) + pixel;
-                float4 v = *acc;
-                for (uint32_t k = 0; k < a.samples; ++k)
-                  v = make_float4(v.x + c.x, v.y + c.y, v.z + c.z, v.w + 1.0f);
-                *acc = v;
-                J.vk_rng[pixel] = vk_state;
-              } else {
-                finish(J, c);
-              }
-            }
+            full = true;
+          } else if constexpr (VK) {
+            // every sample of the pixel is this one and draws nothing
+            float4 *acc = reinterpret_cast<float4 *>(J.acc) + pixel;
+            float4 v = *acc;
+            for (uint32_t i = 0; i < a.samples; ++i)
+              v = make_float4(v.x + cr.x, v.y + cr.y, v.z + cr.z, v.w + 1.0f);
+            *acc = v;
+            J.vk_rng[pixel] = vk_state;
+            has = false;
+          } else {
+            finish(J, f3(cr.x, cr.y, cr.z));
           }
         }
-        off += (uint32_t)__popcll(need);
       }
-      if (!RECORD && full) {
-        const uint32_t oid = chk(bid, J.n_prims, K_OBJECT, a.ctl);
+      off += (uint32_t)__popcll(need);
+    }
+    if constexpr (!RECORD) {
+      if (full) {
+        const uint32_t oid = chk(hit_id(), J.n_prims, K_OBJECT, a.ctl);
         const DevObject ob = lds_obj ? object_from(lds_objects[4 * oid], lds_objects[4 * oid + 1],
                                                    lds_objects[4 * oid + 2], lds_objects[4 * oid + 3])
                                      : load_object(J.objects, oid);
-        const HitRec h = closest_hit(o, d, bt, ob);
+        const HitRec h = closest_hit(o, d, hit_t(), ob);
         ScatterOut so;
         if constexpr (VK) {
           so = scatter_vk(d, h, ob, vk_state, at, li);
@@ -268,7 +422,6 @@ void k_paths(PathArgs a) {
           so = scatter(d, h, ob, dr, at, li);
         }
         li = so.light;
-        full = false;
         if ((sb & 0xffu) + 1u < J.max_bounces) {
           ++sb;
           o = so.o;
@@ -279,131 +432,152 @@ void k_paths(PathArgs a) {
           finish(J, li);  // bounce budget spent: no sky term (cpu.rs:256)
         }
       }
-      // The walk's per-ray values, for the fresh rays and again (the same
-      // values) for the lanes in mid-walk, which did not keep them.
-      if (fresh || active) {
-        r = ray_pre(o, d);
-        if (fresh) {
-          bt = 0.0f;
-          bid = kNoHit;
+    }
+    // The walk's per-ray values, for the fresh rays and again (the same
+    // values) for the lanes in mid-walk, which did not keep them.
+    if (fresh || walking()) {
+      r = ray_pre(o, d);
+      if (fresh) {
+        best = kNoBest;
+        sp = stack_first - 2u * kRow;
+        if (walkable(r) && r.a >= kMinDot && r.a <= kMaxDot) {
           node = 0;
-          sp = 0;
-          active = walkable(r);
-          full = !active;
-          if (full)  // the linear scan, exact for every ray (cpu.rs:345-349)
-            for (uint32_t j = 0; j < J.n_prims; ++j) {
-              DevPrim pr;
-              load_prim(J.prims, j, &pr);
-              if (VK) test_prim_vk(r, pr, &bt, &bid);
-              else test_prim(r, pr, &bt, &bid);
-            }
+        } else {
+          // the linear scan, exact for every ray (cpu.rs:345-349); the lane
+          // is shaded in the next turn
+          float bt = 0.0f;
+          uint32_t bid = kNoHit;
+          for (uint32_t j = 0; j < J.n_prims; ++j) {
+            DevPrim pr;
+            load_prim(J.prims, j, &pr);
+            if constexpr (VK) test_prim_vk(r, pr, &bt, &bid);
+            else test_prim(r, pr, &bt, &bid);
+          }
+          best = ((uint64_t)fbits(bt) << 32) | bid;
         }
-        nf = slab_nf(slab_ray(r, ray_tolerance(r, J.r0_tol)));
-        tcull = VK && bid == kNoHit ? cull0 : cull_limit(bt, bid);
       }
+      ya = rcp_rn_normal(r.a);
+      nf = slab_nf(slab_ray(r, ray_tolerance(r, J.r0_tol)));
+      tcull = cull();
+    }
+    // ---- the walk, until enough lanes are out of it: with work left every
+    // lane that does not walk can be put to use; once the list is empty one
+    // is only worth shading, so the wave waits for three quarters of them
+    const uint32_t walkers = (uint32_t)__popcll(__ballot(walking()));
+    if (walkers == 0) {
+      if (!more && __ballot(has) == 0) break;
       continue;
     }
-    if (active) {
-#ifdef RDH_CHECKED
-      node = (int32_t)chk((uint32_t)node, n_nodes4, K_NODE, a.ctl);
-#endif
-      // each axis's near and far planes of the four children, picked by the
-      // ray's direction signs (slab_hit_nf)
-      VecF4 xn, xf, yn, yf, zn, zf;
-      VecI4 ch;
-      if (LDS) {
-        const unsigned char *np = reinterpret_cast<const unsigned char *>(lds_nodes + 8 * node);
-        xn = *(const VecF4 *)(np + nf.ox); xf = *(const VecF4 *)((np - nf.ox) + 16);
-        yn = *(const VecF4 *)(np + nf.oy); yf = *(const VecF4 *)((np - nf.oy) + 80);
-        zn = *(const VecF4 *)(np + nf.oz); zf = *(const VecF4 *)((np - nf.oz) + 144);
-        ch = *(const VecI4 *)(np + 96);
-      } else {
-        // 32-bit offsets from the tree's base keep the address arithmetic
-        // out of 64-bit registers
-        const __attribute__((address_space(1))) unsigned char *gb =
-            (const __attribute__((address_space(1))) unsigned char *)nodes4;
-        const uint32_t nb = (uint32_t)node * (uint32_t)sizeof(DevNode4);
-        xn = *(GlobalF4 *)(gb + (nb + nf.ox)); xf = *(GlobalF4 *)(gb + ((nb - nf.ox) + 16u));
-        yn = *(GlobalF4 *)(gb + (nb + nf.oy)); yf = *(GlobalF4 *)(gb + ((nb - nf.oy) + 80u));
-        zn = *(GlobalF4 *)(gb + (nb + nf.oz)); zf = *(GlobalF4 *)(gb + ((nb - nf.oz) + 144u));
-        ch = *(GlobalI4 *)(gb + (nb + 96u));
-      }
-      float t0, t1, t2, t3;
-      const bool h0 = slab_hit_nf(nf, xn.x, xf.x, yn.x, yf.x, zn.x, zf.x, tcull, &t0);
-      const bool h1 = slab_hit_nf(nf, xn.y, xf.y, yn.y, yf.y, zn.y, zf.y, tcull, &t1);
-      const bool h2 = slab_hit_nf(nf, xn.z, xf.z, yn.z, yf.z, zn.z, zf.z, tcull, &t2);
-      const bool h3 = slab_hit_nf(nf, xn.w, xf.w, yn.w, yf.w, zn.w, zf.w, tcull, &t3);
-      const bool l0 = h0 && is_leaf(ch.x), l1 = h1 && is_leaf(ch.y);
-      const bool l2 = h2 && is_leaf(ch.z), l3 = h3 && is_leaf(ch.w);
-      // trip t tests f_k + t for the k-th hit leaf (one primitive each with
-      // LEAF1: trip t is that leaf's first primitive)
-      const uint32_t n0 = l0 ? (LEAF1 ? 1u : leaf_count(ch.x)) : 0u;
-      const uint32_t p1 = n0 + (l1 ? (LEAF1 ? 1u : leaf_count(ch.y)) : 0u);
-      const uint32_t p2 = p1 + (l2 ? (LEAF1 ? 1u : leaf_count(ch.z)) : 0u);
-      const uint32_t n_leaf = p2 + (l3 ? (LEAF1 ? 1u : leaf_count(ch.w)) : 0u);
-      const uint32_t f0 = leaf_first(ch.x), f1 = leaf_first(ch.y) - (LEAF1 ? 0u : n0);
-      const uint32_t f2 = leaf_first(ch.z) - (LEAF1 ? 0u : p1);
-      const uint32_t f3 = leaf_first(ch.w) - (LEAF1 ? 0u : p2);
-      // The next node and the stack are settled before the primitive tests
-      // (they depend only on this node's boxes), so the children's keys and
-      // ids are dead while the primitives are tested.
-      const bool i0 = h0 && !l0, i1 = h1 && !l1, i2 = h2 && !l2, i3 = h3 && !l3;
-      const int cnt = (int)i0 + (int)i1 + (int)i2 + (int)i3;
-      int32_t c0;
-      if (__ballot(cnt > 1) == 0) {
-        // no lane entered two inner children: nothing to order or push
-        c0 = i0 ? ch.x : i1 ? ch.y : i2 ? ch.z : ch.w;
-      } else {
-        float k0 = i0 ? t0 : INFINITY, k1 = i1 ? t1 : INFINITY;
-        float k2 = i2 ? t2 : INFINITY, k3 = i3 ? t3 : INFINITY;
-        int32_t c1 = ch.y, c2 = ch.z, c3 = ch.w;
-        c0 = ch.x;
-        order_pair(k0, c0, k1, c1);
-        order_pair(k2, c2, k3, c3);
-        order_pair(k0, c0, k2, c2);
-        order_pair(k1, c1, k3, c3);
-        order_pair(k1, c1, k2, c2);
-#ifdef RDH_CHECKED
-        sp = (int)chk((uint32_t)sp + 2u, a.stack_rows, K_STACK, a.ctl) - 2;
-        if (sp < 0) sp = 0;
-#endif
-        stk[sp * BLOCK] = (StackT)(cnt == 4 ? c3 : cnt == 3 ? c2 : c1);
-        stk[(sp + 1) * BLOCK] = (StackT)(cnt == 4 ? c2 : c1);
-        stk[(sp + 2) * BLOCK] = (StackT)c1;
-      }
-      const int top = sp > 0 ? sp - 1 : 0;
-      const int32_t popped = (int32_t)stk[top * BLOCK];
-      const bool done = cnt == 0 && sp == 0;
-      if (cnt > 0) {
-        node = c0;
-        sp += cnt - 1;
-      } else if (sp > 0) {
-        node = popped;
-        sp = top;
-      }
-      if (n_leaf) {
-        for (uint32_t t = 0; t < n_leaf; ++t) {
-          DevPrim pr;
-          uint32_t j = LEAF1 ? (t < n0 ? f0 : t < p1 ? f1 : t < p2 ? f2 : f3)
-                             : (t < n0 ? f0 + t : t < p1 ? f1 + t : t < p2 ? f2 + t : f3 + t);
-#ifdef RDH_CHECKED
-          j = chk(j, n_prims, K_PRIM, a.ctl);
-#endif
-          if (LDS) {
-            const VecF4 pa = lds_prims[2 * j], pb = lds_prims[2 * j + 1];
-            pr.a[0] = pa.x; pr.a[1] = pa.y; pr.a[2] = pa.z; pr.a[3] = pa.w;
-            pr.b[0] = pb.x; pr.b[1] = pb.y; pr.b[2] = pb.z; pr.b[3] = pb.w;
-          } else {
-            load_prim(prims, j, &pr);
+    const uint32_t keep = more ? 64u - a.refill : walkers / 4u;
+    for (;;) {
+      const uint64_t at_nodes = __ballot(node != kNoNode);
+      if constexpr (kPooled) {
+        // Test one primitive a lane once many lanes have one, or a pool could
+        // overflow in the next step, or nothing else is left to do.
+        const uint64_t pending = __ballot(pool != pool_first);
+        if ((uint32_t)__popcll(pending) >= kPoolTests || at_nodes == 0 ||
+            __ballot(pool > pool_first + 4u * kRow) != 0) {
+          if (pending == 0) break;
+          if (pool != pool_first) {
+            pool -= kRow;
+            test(stack_at(pool));
+            tcull = cull();
           }
-          if (VK) test_prim_vk(r, pr, &bt, &bid);
-          else test_prim(r, pr, &bt, &bid);
+          continue;
         }
-        tcull = VK && bid == kNoHit ? cull0 : cull_limit(bt, bid);
+        if ((uint32_t)__popcll(at_nodes | pending) <= keep) break;
+      } else {
+        if ((uint32_t)__popcll(at_nodes) <= keep) break;
       }
-      if (done) {
-        active = false;
-        full = true;
+      if (node != kNoNode) {
+#ifdef RDH_CHECKED
+        node = chk(node, n_nodes4, K_NODE, a.ctl);
+#endif
+        // each axis's near and far planes of the four children, picked by the
+        // ray's direction signs (slab_hit_nf)
+        VecF4 xn, xf, yn, yf, zn, zf;
+        VecI4 ch;
+        if (LDS) {
+          const unsigned char *np = reinterpret_cast<const unsigned char *>(lds_nodes + 8 * node);
+          xn = *(const VecF4 *)(np + nf.ox); xf = *(const VecF4 *)((np - nf.ox) + 16);
+          yn = *(const VecF4 *)(np + nf.oy); yf = *(const VecF4 *)((np - nf.oy) + 80);
+          zn = *(const VecF4 *)(np + nf.oz); zf = *(const VecF4 *)((np - nf.oz) + 144);
+          ch = *(const VecI4 *)(np + 96);
+        } else {
+          // 32-bit offsets from the tree's base keep the address arithmetic
+          // out of 64-bit registers
+          const __attribute__((address_space(1))) unsigned char *gb =
+              (const __attribute__((address_space(1))) unsigned char *)nodes4;
+          const uint32_t nb = node * (uint32_t)sizeof(DevNode4);
+          xn = *(GlobalF4 *)(gb + (nb + nf.ox)); xf = *(GlobalF4 *)(gb + ((nb - nf.ox) + 16u));
+          yn = *(GlobalF4 *)(gb + (nb + nf.oy)); yf = *(GlobalF4 *)(gb + ((nb - nf.oy) + 80u));
+          zn = *(GlobalF4 *)(gb + (nb + nf.oz)); zf = *(GlobalF4 *)(gb + ((nb - nf.oz) + 144u));
+          ch = *(GlobalI4 *)(gb + (nb + 96u));
+        }
+        float t0, t1, t2, t3;
+        const bool h0 = slab_hit_nf(nf, xn.x, xf.x, yn.x, yf.x, zn.x, zf.x, tcull, &t0);
+        const bool h1 = slab_hit_nf(nf, xn.y, xf.y, yn.y, yf.y, zn.y, zf.y, tcull, &t1);
+        const bool h2 = slab_hit_nf(nf, xn.z, xf.z, yn.z, yf.z, zn.z, zf.z, tcull, &t2);
+        const bool h3 = slab_hit_nf(nf, xn.w, xf.w, yn.w, yf.w, zn.w, zf.w, tcull, &t3);
+        // The entered inner children, nearest first.  A key is the entry
+        // distance's upper 16 bits (it only orders the visits) above the
+        // child's index; a leaf's code leaves the sign bit set, as kNoKey has
+        // it, so those keys sort behind.  Seven integer min/med/max steps
+        // order distance and child together (the float form took a compare
+        // and four selects for each of five exchanges).
+        const uint32_t e0 = h0 ? (fbits(t0) & 0x7fff0000u) | (uint32_t)ch.x : kNoKey;
+        const uint32_t e1 = h1 ? (fbits(t1) & 0x7fff0000u) | (uint32_t)ch.y : kNoKey;
+        const uint32_t e2 = h2 ? (fbits(t2) & 0x7fff0000u) | (uint32_t)ch.z : kNoKey;
+        const uint32_t e3 = h3 ? (fbits(t3) & 0x7fff0000u) | (uint32_t)ch.w : kNoKey;
+        if constexpr (kPooled) {
+          // the entered leaves' primitives go above the lane's others; a key
+          // plus one has the sign bit set for a leaf's alone
+          stack_at(pool) = leaf_prim(ch.x);
+          pool += ((e0 + 1u) >> 31) * kRow;
+          stack_at(pool) = leaf_prim(ch.y);
+          pool += ((e1 + 1u) >> 31) * kRow;
+          stack_at(pool) = leaf_prim(ch.z);
+          pool += ((e2 + 1u) >> 31) * kRow;
+          stack_at(pool) = leaf_prim(ch.w);
+          pool += ((e3 + 1u) >> 31) * kRow;
+        }
+        const uint32_t lo = umin(umin(e0, e1), e2), mid = umed3(e0, e1, e2), hi = umax(umax(e0, e1), e2);
+        const uint32_t r0 = umin(lo, e3), r1 = umed3(lo, mid, e3);
+        const uint32_t r2 = umed3(mid, hi, e3), r3 = umax(hi, e3);
+        // The stack grows downwards.  The farther ones go on it, farthest
+        // first; an entry that is none (sign bit set) is written too and the
+        // next one put over it.  The nearest is next, or the top of the stack
+        // (kNoNode above the first).
+#ifdef RDH_CHECKED
+        if (chk(sp, stack_bytes - 2u * kRow, K_STACK, a.ctl) == 0u) sp = stack_first - 2u * kRow;
+#endif
+        stack_at(sp + 2u * kRow) = (StackT)r3;
+        sp += (r3 >> 31) * kRow;
+        stack_at(sp + kRow) = (StackT)r2;
+        sp += (r2 >> 31) * kRow;
+        stack_at(sp) = (StackT)r1;
+        sp += (r1 >> 31) * kRow;
+        const uint32_t popped = stack_at(sp);
+        node = (int32_t)r0 < 0 ? popped : r0 & 0xffffu;
+        sp += (r0 >> 31) * kRow - 3u * kRow;
+        if constexpr (!kPooled) {
+          // trip t tests f_k + t for the k-th hit leaf
+          const uint32_t n0 = h0 && is_leaf(ch.x) ? (LEAF1 ? 1u : leaf_count(ch.x)) : 0u;
+          const uint32_t p1 = n0 + (h1 && is_leaf(ch.y) ? (LEAF1 ? 1u : leaf_count(ch.y)) : 0u);
+          const uint32_t p2 = p1 + (h2 && is_leaf(ch.z) ? (LEAF1 ? 1u : leaf_count(ch.z)) : 0u);
+          const uint32_t n_leaf = p2 + (h3 && is_leaf(ch.w) ? (LEAF1 ? 1u : leaf_count(ch.w)) : 0u);
+          if constexpr (LEAF1) {
+            const uint32_t f0 = leaf_prim(ch.x), f1 = leaf_prim(ch.y);
+            const uint32_t f2 = leaf_prim(ch.z), f3 = leaf_prim(ch.w);
+            for (uint32_t t = 0; t < n_leaf; ++t) test(t < n0 ? f0 : t < p1 ? f1 : t < p2 ? f2 : f3);
+          } else {
+            const uint32_t f0 = leaf_first(ch.x), f1 = leaf_first(ch.y) - n0;
+            const uint32_t f2 = leaf_first(ch.z) - p1, f3 = leaf_first(ch.w) - p2;
+            for (uint32_t t = 0; t < n_leaf; ++t)
+              test((t < n0 ? f0 : t < p1 ? f1 : t < p2 ? f2 : f3) + t);
+          }
+          if (n_leaf) tcull = cull();
+        }
       }
     }
   }
@@ -426,8 +600,9 @@ const void *paths_fn(const PathArgs &a, bool record) {
 }
 
 uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
-  return ((a.stack_rows * kPathBlock * 2u + 15u) & ~15u) + a.lds_bvh_bytes +
-         (record ? 0u : a.lds_obj_bytes);
+  return ((a.stack_rows * kPathBlock * 2u + 15u) & ~15u) +
+         (pooled(a.lds_bvh_bytes > 0, a.leaf1 != 0) ? pool_bytes<kPathBlock>() : 0u) +
+         a.lds_bvh_bytes + (record ? 0u : a.lds_obj_bytes);
 }
 
 }  // namespace

@@ -14,7 +14,7 @@ import pytest
 
 import oracle
 import raydar_amd as ra
-from raydar_amd import abi, scenegen
+from raydar_amd import abi, scene, scenegen
 
 pytestmark = pytest.mark.gpu
 
@@ -36,6 +36,43 @@ def test_path_kernel_matches_oracle(size, spp, bounces, opts):
     ref = oracle.render(sc, spp, bounces, 17)
     np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
     np.testing.assert_array_equal(img.reshape(-1), oracle.tonemap(ref, spp))
+
+
+def _arithmetic_scene(view, scale):
+    # spheres and cubes on and around the camera's axis, with faces in the
+    # planes of the camera's position and shared by neighbours
+    sc = scenegen.plain_1080p(3, 61, 41)
+    sc.objects = np.concatenate([sc.objects, np.array([
+        scene.make_object(k, c, size, roughness=0.3, metallic=m)
+        for k, c, size, m in [(abi.RD_CUBE, (0, 0.5, 3), 1, 0.0), (abi.RD_CUBE, (1, 0.5, 3), 1, 1.0),
+                              (abi.RD_CUBE, (-1, 1.5, 3), 1, 0.0), (abi.RD_SPHERE, (0, 1, 6), 1, 1.0),
+                              (abi.RD_SPHERE, (0, 1, 1), 2.0 ** -13, 0.0)]], abi.OBJECT_DTYPE)])
+    for f in ("center", "size"):
+        sc.objects[f] *= np.float32(scale)
+    kw = dict(fov_deg=60) if view == "axis" else dict(ortho_size=6 * scale)
+    sc.camera = scene.make_camera((0, scale, -8 * scale), (0, scale, 0), (0, 1, 0), 61, 41,
+                                  near=0.1 * scale, far=100 * scale, **kw)
+    return sc
+
+
+@pytest.mark.parametrize("lds_bvh", [0, 1 << 16])
+@pytest.mark.parametrize("scale", [2.0 ** -40, 2.0 ** -12, 1.0, 2.0 ** 9, 2.0 ** 30])
+@pytest.mark.parametrize("view", ["axis", "parallel"])
+def test_walk_arithmetic_at_its_limits(view, scale, lds_bvh):
+    # the walk's divisions and roots are exact forms for a range of their
+    # arguments and the plain ones outside: zero direction components and
+    # numerators, tiny and huge discriminants, rays that no walk takes; trees
+    # in memory have the pool of primitives
+    sc = _arithmetic_scene(view, scale)
+    print(f"arithmetic {view} scale={scale} lds={lds_bvh}", flush=True)
+    for semantics in (0, 1):
+        with ra.HipRenderer(max_sample_count=3, max_bounces=12, seed=9, semantics=semantics,
+                            lds_bvh=lds_bvh) as r:
+            r.render_frame(sc)
+            acc = r.accumulator()
+        ref = (oracle.render(sc, 3, 12, 9) if semantics == 0 else
+               oracle.vk_render(sc, ra.camera_vulkan_inverse_view(sc.camera), 3, 12, threads=8))
+        np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
 
 
 def test_path_kernel_and_wavefront_alternate_on_one_renderer():
