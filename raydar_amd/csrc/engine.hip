@@ -441,10 +441,10 @@ bool Engine::ensure_aux(int n, std::string *err) {
 
 // Automatic: two pipes when the scene is traversed from LDS (extend bound by
 // VALU issue), three otherwise (extend also waits on node fetches, so a third
-// stream hides more of it).
-int Engine::pipes_for(const DevJob &j, const DevTicket &t) const {
-  const uint64_t tree = opt.bvh4 && j.n_nodes4 ? 128ull * j.n_nodes4 : 64ull * j.n_nodes;
-  const bool lds = tree + 32ull * j.n_prims <= opt.lds_bvh;
+// stream hides more of it).  The path kernel's pipes share one work list; it
+// is indifferent to them but for three with LDS (183 objects at 4K, 8 spp: 1
+// 8.1 ms, 2 7.9, 3 8.5).
+int Engine::pipes_for(const DevTicket &t, bool lds) const {
   const int want = opt.pipes > 0 ? opt.pipes : (lds ? 2 : 3);
   const uint64_t per_pipe = std::min<uint64_t>(opt.queue / 2, 1ull << 22);
   const uint64_t by_size = t.paths / std::max<uint64_t>(1, per_pipe);
@@ -495,17 +495,13 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
   a.samples = t.spp;
   a.vk = opt.vk;
   a.refill = (uint32_t)opt.refill;
-  a.stack_rows = j.stack4 + 4;  // a sentinel below, and three written above the top
-  a.leaf1 = j.max_leaf == 1 ? 1 : 0;
-  const uint64_t tree = sizeof(DevNode4) * (uint64_t)j.n_nodes4 + sizeof(DevPrim) * (uint64_t)j.n_prims;
-  a.lds_bvh_bytes = tree <= opt.lds_bvh ? (uint32_t)tree : 0u;
-  const uint64_t objects = sizeof(DevObject) * (uint64_t)j.n_prims;
-  a.lds_obj_bytes = objects <= opt.lds_objects ? (uint32_t)objects : 0u;
+  // (the tree bound's default and more: whatever fits)
+  plan_paths(&a, j, opt.lds_bvh >= EngineOptions().lds_bvh ? UINT64_MAX : opt.lds_bvh, opt.lds_objects);
 
   // Everything is queued without a wait in between; the caller waits for the
   // accumulation.  A launch's waves take its work list in chunks through a
   // device counter, so the pipes' launches share one list.
-  const int np = pipes_used = pipes_for(j, t);
+  const int np = pipes_used = pipes_for(t, a.lds_bvh_bytes > 0);
   if (!ensure_aux(np - 1, err)) return false;
   if (!check(launch_set_ctl(path_ctl_, 0, 0, stream), "set ctl", err)) return false;
   struct DrainOnError {
@@ -524,7 +520,7 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
     a.spp = record || opt.vk ? 1u : t.spp;
     a.chunks = (uint32_t)((npix + 63) / 64) * a.spp;
     const int full = opt.grid > 0 ? opt.grid : num_cus * path_blocks_per_cu(a, record);
-    const int fill = (int)std::min<uint64_t>((uint64_t)full, (a.chunks + 3ull) / 4);
+    const int fill = (int)std::min<uint64_t>((uint64_t)full, (a.chunks + kPathBlock / 64 - 1ull) / (kPathBlock / 64));
     const int n = record || opt.kernel_timing ? 1 : std::min(np, fill);
     a.slices = std::min<uint32_t>(kPathSlices, (uint32_t)(fill / n));
     a.step_groups = a.slices / a.spp;
@@ -541,7 +537,11 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
       Engine &e = k == 0 ? *this : *aux_[k - 1];
       if (k > 0 && !check(hipStreamWaitEvent(e.stream, arena_free_, 0), "hipStreamWaitEvent", err))
         return false;
-      const int grid = (int)((int64_t)fill * (k + 1) / n - (int64_t)fill * k / n);
+      // whole rounds of the slices (and of the XCDs) for each launch if there
+      // are enough: three uneven launches took 6.35 ms for 5.90 ms of work
+      const int64_t unit = fill >= 8 * n * (int)a.slices ? a.slices : 1;
+      a.first_block = (uint32_t)(fill / unit * k / n * unit);
+      const int grid = (int)((k + 1 < n ? fill / unit * (k + 1) / n * unit : fill) - a.first_block);
       if (!check(launch_paths(a, record, grid, e.stream), "launch paths", err)) return false;
       ++iterations;
       if (k == 0) continue;
@@ -624,7 +624,12 @@ bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
     // below that the extra launches cost more than the overlap gains
     // (measured break-even between 4M and 8M paths per pass).
     std::vector<std::vector<DevTicket>> parts;
-    const int np = traced.size() == 1 && host_jobs.size() == 1 ? pipes_for(host_jobs[0], traced[0]) : 1;
+    int np = 1;
+    if (traced.size() == 1 && host_jobs.size() == 1) {
+      const DevJob &j = host_jobs[0];
+      const uint64_t tree = opt.bvh4 && j.n_nodes4 ? 128ull * j.n_nodes4 : 64ull * j.n_nodes;
+      np = pipes_for(traced[0], tree + 32ull * j.n_prims <= opt.lds_bvh);
+    }
     pipes_used = np;
     if (np <= 1) {
       parts.push_back(traced);

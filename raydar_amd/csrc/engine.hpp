@@ -206,7 +206,7 @@ class Engine {
                                                              hipStream_t),
              const IterArgs &a, int parity, uint32_t bound);
   // Pipes of a one-job pass (see run_tickets).
-  int pipes_for(const DevJob &j, const DevTicket &t) const;
+  int pipes_for(const DevTicket &t, bool lds) const;
   bool ensure_aux(int n, std::string *err);
   bool external_ = false;  // buffers, stream and control copy are borrowed
   std::vector<hipEvent_t> ev_pool_;

@@ -230,7 +230,7 @@ void k_paths(PathArgs a) {
   // and a dealt slice is a fair sample of the image, so the slices end
   // together.  (Waves that went on to other slices when theirs was used up
   // spent 0.3 ms of a 1080p recording asking around.)
-  const uint32_t slice = blockIdx.x % a.slices;
+  const uint32_t slice = (blockIdx.x + a.first_block) % a.slices;
   const uint32_t slice_chunks = (a.chunks + a.slices - 1u - slice) / a.slices;
   const float cull0 = VK ? cull_limit(kVkTMax, 0u) : INFINITY;  // with no hit yet
   // A lane is free (!has), or its path walks (nodes to visit: node != kNoNode;
@@ -583,8 +583,6 @@ void k_paths(PathArgs a) {
   }
 }
 
-constexpr int kPathBlock = 256;
-
 template <bool RECORD, bool VK>
 const void *paths_fn_of(bool lds, bool leaf1) {
   return lds ? (leaf1 ? (const void *)k_paths<kPathBlock, RECORD, true, true, VK>
@@ -607,11 +605,29 @@ uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
 
 }  // namespace
 
+// A tree is copied into LDS by every workgroup as long as that costs none of
+// the workgroups the registers allow on a CU (five, with Vulkan semantics
+// four); the objects too if they fit beside it.  183 objects (17 KB) at 4K, 8
+// spp: 9.2 ms from memory, 8.0 from LDS.  Larger workgroups that share a copy
+// were slower than the walk in memory: 640 threads 300 objects 1.33 -> 1.45 ms,
+// 500 objects 1.46 -> 1.69 (1280x720, 16 spp, whole call).
+void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh, uint64_t lds_objects) {
+  a->stack_rows = j.stack4 + 4;  // a sentinel below, and three written above the top
+  a->leaf1 = j.max_leaf == 1 ? 1 : 0;
+  const uint64_t blocks = 4 * path_waves(false, a->vk) / (kPathBlock / 64);
+  const uint64_t room = 160 * 1024 / blocks - 1024, stack = 2ull * a->stack_rows * kPathBlock + 16;
+  const uint64_t tree = sizeof(DevNode4) * (uint64_t)j.n_nodes4 + sizeof(DevPrim) * (uint64_t)j.n_prims;
+  const uint64_t objects = sizeof(DevObject) * (uint64_t)j.n_prims;
+  const bool lds = tree <= lds_bvh && stack + tree <= room;
+  a->lds_bvh_bytes = lds ? (uint32_t)tree : 0u;
+  const uint64_t used = stack + (lds ? tree : pool_bytes<kPathBlock>());
+  a->lds_obj_bytes = objects <= lds_objects && used + objects <= room ? (uint32_t)objects : 0u;
+}
+
 int path_blocks_per_cu(const PathArgs &a, bool record) {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &n, paths_fn(a, record), kPathBlock,
-          dynamic_lds_bytes(a, record)) != hipSuccess) {
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, paths_fn(a, record), kPathBlock,
+                                                   dynamic_lds_bytes(a, record)) != hipSuccess) {
     (void)hipGetLastError();
     return 1;
   }
@@ -621,8 +637,8 @@ int path_blocks_per_cu(const PathArgs &a, bool record) {
 hipError_t launch_paths(const PathArgs &a, bool record, int grid, hipStream_t st) {
   PathArgs args = a;
   void *kargs[] = {&args};
-  return hipLaunchKernel(paths_fn(a, record), dim3(grid),
-                         dim3(kPathBlock), kargs, dynamic_lds_bytes(a, record), st);
+  return hipLaunchKernel(paths_fn(a, record), dim3(grid), dim3(kPathBlock), kargs,
+                         dynamic_lds_bytes(a, record), st);
 }
 
 }  // namespace rdh

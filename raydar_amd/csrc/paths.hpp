@@ -7,6 +7,7 @@
 
 namespace rdh {
 
+constexpr int kPathBlock = 256;                // threads of a workgroup
 constexpr uint32_t kPathSlices = kSegments;  // slices of a work list at most
 
 struct PathArgs {
@@ -26,6 +27,7 @@ struct PathArgs {
   uint32_t samples;             // vk: samples a lane takes of its pixel, below 2^24
   uint32_t chunks;              // work list: groups of 64 ranks * spp
   uint32_t slices;              // slices it is dealt to, at most the launch's workgroups
+  uint32_t first_block;         // the launch's first workgroup among all that share the list
   uint32_t request;             // chunks a wave asks for at once
   uint32_t step_groups;         // slices / spp and slices % spp: from one chunk of a
   uint32_t step_samples;        // slice to the next
@@ -42,9 +44,14 @@ struct PathArgs {
 // Bytes of the camera-hit table per pixel.
 constexpr uint64_t kCamBytes = sizeof(float4) + sizeof(uint2);
 
-// Workgroups of the kernel that fit on one CU, and its launch.  Weak: a host
-// build without the device kernels has neither, and the engine then runs the
-// wavefront's launchers.
+// Weak: a host build without the device kernels has none of these, and the
+// engine then runs the wavefront's launchers.
+//
+// Fill in what depends on the scene: the stack and what a workgroup copies into
+// LDS (at most lds_bvh bytes of tree and lds_objects bytes of objects).
+__attribute__((weak)) void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh,
+                                      uint64_t lds_objects);
+// Workgroups of the kernel that fit on one CU, and its launch.
 __attribute__((weak)) int path_blocks_per_cu(const PathArgs &a, bool record);
 __attribute__((weak)) hipError_t launch_paths(const PathArgs &a, bool record, int grid,
                                               hipStream_t st);

@@ -38,6 +38,22 @@ def test_path_kernel_matches_oracle(size, spp, bounces, opts):
     np.testing.assert_array_equal(img.reshape(-1), oracle.tonemap(ref, spp))
 
 
+@pytest.mark.parametrize("semantics", [0, 1])
+@pytest.mark.parametrize("objects,opts", [
+    (130, dict()), (185, dict()), (240, dict()), (320, dict()), (420, dict()),
+    (185, dict(lds_bvh=14335)), (185, dict(lds_bvh=14336, lds_objects=0)),
+    (60, dict(lds_bvh=14335, pipes=3, queue=4096))])
+def test_trees_around_what_fits_in_lds(objects, opts, semantics):
+    # tree and objects in LDS, the tree alone, neither, by size and by option
+    sc = scenegen.clustered(6, objects, 90, 61)
+    with ra.HipRenderer(max_sample_count=3, max_bounces=12, seed=3, semantics=semantics, **opts) as r:
+        r.render_frame(sc)
+        acc = r.accumulator()
+    ref = (oracle.render(sc, 3, 12, 3) if semantics == 0 else
+           oracle.vk_render(sc, ra.camera_vulkan_inverse_view(sc.camera), 3, 12, threads=8))
+    np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
+
+
 def _arithmetic_scene(view, scale):
     # spheres and cubes on and around the camera's axis, with faces in the
     # planes of the camera's position and shared by neighbours
