@@ -125,11 +125,7 @@ struct rd_renderer {
   rdh::Engine noalloc_eng;  // rd_render_frame_noalloc: borrows the static scratch
   rdh::DeviceScene scene;
   rdh::DevJob job_h{};
-  rdh::DevJob *job_d = nullptr;
-  // pinned copy the job record is uploaded from (a pageable source costs a
-  // staging copy on every upload); uploads only when the record changed
-  rdh::DevJob *job_pin = nullptr;
-  bool job_uploaded = false;
+  hipEvent_t rendered = nullptr;  // end of the last render_samples' passes
   float *acc = nullptr;
   uchar4 *rgba_d = nullptr;
   uint32_t *vk_rng = nullptr;  // Vulkan semantics: per-pixel PCG state
@@ -184,7 +180,8 @@ rd_status snapshot(rd_renderer *r, const rd_scene *s, bool zero_acc) {
   rdh::BuiltScene built;
   if (!rdh::build_scene(*s, r->eng.opt.leaf, &built, &err)) return r->fail(RD_ERR_INVALID_ARGUMENT, err);
   if (!rdh::check_bvh(built, &err)) return r->fail(RD_ERR_INVALID_ARGUMENT, "BVH build: " + err);
-  if (!r->eng.upload_scene(built, &r->scene, &err)) return device_fail(r, err);
+  r->has_frame = false;  // until the new one is whole
+  if (!r->eng.alloc_scene(built, &r->scene, &err)) return device_fail(r, err);
   const uint32_t W = s->camera.resolution_x, H = s->camera.resolution_y;
   if (W != r->W || H != r->H || !r->acc) {
     r->eng.dfree(r->acc);
@@ -214,15 +211,7 @@ rd_status snapshot(rd_renderer *r, const rd_scene *s, bool zero_acc) {
       return device_fail(r, err);
     r->job_h.vk_rng = r->vk_rng;
   }
-  if (!r->job_d && !r->eng.check(hipMalloc(&r->job_d, sizeof(rdh::DevJob)), "hipMalloc(job)", &err))
-    return device_fail(r, err);
-  *r->job_pin = r->job_h;  // no upload from it is in flight: every call ends synchronised
-  r->job_uploaded = true;
-  if (!r->eng.check(hipMemcpyAsync(r->job_d, r->job_pin, sizeof(rdh::DevJob),
-                                   hipMemcpyHostToDevice, r->eng.stream),
-                    "upload job", &err) ||
-      !r->eng.check(hipStreamSynchronize(r->eng.stream), "upload job", &err))
-    return device_fail(r, err);
+  if (!r->eng.copy_scene(built, r->scene, &r->job_h, &err)) return device_fail(r, err);
   r->has_frame = true;
   return RD_OK;
 }
@@ -230,20 +219,15 @@ rd_status snapshot(rd_renderer *r, const rd_scene *s, bool zero_acc) {
 // Job fields that can change between passes without a new snapshot.
 rd_status refresh_job(rd_renderer *r) {
   std::string err;
-  if (r->job_uploaded && r->job_h.max_bounces == r->cfg.max_bounces && r->job_h.seed == r->seed)
+  if (r->job_h.max_bounces == r->cfg.max_bounces && r->job_h.seed == r->seed)
     return RD_OK;
   r->job_h.max_bounces = r->cfg.max_bounces;
   r->job_h.seed = r->seed;
-  *r->job_pin = r->job_h;
-  r->job_uploaded = true;
-  if (!r->eng.check(hipMemcpyAsync(r->job_d, r->job_pin, sizeof(rdh::DevJob),
-                                   hipMemcpyHostToDevice, r->eng.stream),
-                    "upload job", &err))
-    return device_fail(r, err);
+  if (!r->eng.upload(r->scene.job, &r->job_h, sizeof(rdh::DevJob), "upload job", &err)) return device_fail(r, err);
   return RD_OK;
 }
 
-// Renders `k` more samples (cpu.rs:193-219 repeated k times).  The k samples
+// Queues `k` more samples (cpu.rs:193-219 repeated k times).  The k samples
 // run as one pass, so the sample timer reports their average, as the Vulkan
 // renderer does for its all-samples dispatch (vulkan.rs:175-177); with k = 1
 // that is the last sample's time, as CpuRenderer reports (cpu.rs:196, 218).
@@ -285,33 +269,41 @@ rd_status render_samples(rd_renderer *r, uint32_t k) {
     t.spp = spp;
     t.paths = (uint32_t)(spp * npix);
     r->eng.hit_frame = r->frame_serial;
-    if (!r->eng.run_tickets(r->job_d, {t}, host_jobs, &err)) return device_fail(r, err);
+    if (!r->eng.run_tickets(r->scene.job, {t}, host_jobs, &err)) return device_fail(r, err);
     done += spp;
   }
-  if (!r->eng.check(hipStreamSynchronize(r->eng.stream), "render", &err)) return device_fail(r, err);
-  r->sample_count += k;
-  if (r->sample_count == r->cfg.max_sample_count) {
-    r->render_timer.end();
-    r->frame_timer.end();
-  }
-  r->sample_timer.end_multiple(k);
   return RD_OK;
 }
 
-// print_frame_buffer (cpu.rs:221-230) on the device, then copy out.
-rd_status tonemap_out(rd_renderer *r, uint8_t *rgba, size_t cap) {
+// print_frame_buffer (cpu.rs:221-230) on the device, then copy out.  The `k`
+// samples that render_samples just queued are waited for and counted; the
+// tonemap is queued behind them, and the timers end before it.
+rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba) {
   std::string err;
   const uint64_t npix = (uint64_t)r->W * r->H;
   const int grid = (int)std::min<uint64_t>((npix + 255) / 256, 8192);
-  if (!r->eng.check(rdh::launch_tonemap(r->job_d, (uint32_t)npix, (float)r->sample_count,
-                                        r->rgba_d, r->eng.counters, r->eng.opt.count != 0, grid,
-                                        r->eng.stream, r->frame_vk != 0),
-                    "tonemap", &err) ||
-      !r->eng.check(hipMemcpyAsync(rgba, r->rgba_d, 4 * npix, hipMemcpyDeviceToHost, r->eng.stream),
-                    "read image", &err) ||
-      !r->eng.check(hipStreamSynchronize(r->eng.stream), "read image", &err))
+  // An event tells when the passes have ended while the tonemap runs on; for
+  // images below a megabyte it costs more (20 us) than the gap it fills.
+  const bool ahead = k && 4 * npix >= 1u << 20;
+  if (ahead && !r->eng.check(hipEventRecord(r->rendered, r->eng.stream), "hipEventRecord", &err))
     return device_fail(r, err);
-  (void)cap;
+  if (k && !ahead && !r->eng.check(hipStreamSynchronize(r->eng.stream), "render", &err))
+    return device_fail(r, err);
+  const hipError_t e = rdh::launch_tonemap(r->scene.job, (uint32_t)npix, (float)(r->sample_count + k), r->rgba_d,
+                                           r->eng.counters, r->eng.opt.count != 0, grid, r->eng.stream,
+                                           r->frame_vk != 0);
+  if (!r->eng.check(e, "tonemap", &err) ||
+      (ahead && !r->eng.check(hipEventSynchronize(r->rendered), "render", &err)))
+    return device_fail(r, err);
+  if (k) {
+    r->sample_count += k;
+    if (r->sample_count == r->cfg.max_sample_count) {
+      r->render_timer.end();
+      r->frame_timer.end();
+    }
+    r->sample_timer.end_multiple(k);
+  }
+  if (!r->eng.read(rgba, r->rgba_d, 4 * npix, "read image", &err)) return device_fail(r, err);
   return RD_OK;
 }
 
@@ -368,8 +360,8 @@ rd_status rd_create(const rd_config *config, rd_renderer **out) {
   r->eng.cache = &r->cache;
   std::string err;
   if (!r->eng.init(&err) ||
-      !r->eng.check(hipHostMalloc((void **)&r->job_pin, sizeof(rdh::DevJob), hipHostMallocDefault),
-                    "hipHostMalloc(job)", &err) ||
+      !r->eng.check(hipEventCreateWithFlags(&r->rendered, hipEventDisableTiming), "hipEventCreate", &err) ||
+      !r->eng.check(r->eng.transfer().reserve(), "hipHostMalloc(transfers)", &err) ||
       !scratch_setup(r->eng.device, &err)) {
     rdh::set_global_error(err);
     delete r;
@@ -386,8 +378,7 @@ void rd_destroy(rd_renderer *r) {
   r->eng.dfree(r->acc);
   r->eng.dfree(r->rgba_d);
   r->eng.dfree(r->vk_rng);
-  if (r->job_d) (void)hipFree(r->job_d);
-  if (r->job_pin) (void)hipHostFree(r->job_pin);
+  if (r->rendered) (void)hipEventDestroy(r->rendered);
   delete r;
 }
 
@@ -433,7 +424,7 @@ rd_status rd_render_sample(rd_renderer *r, const rd_scene *scene, uint8_t *rgba,
                                  : std::min(r->samples_per_pass, r->cfg.max_sample_count - r->sample_count);
   rd_status st = render_samples(r, k);
   if (st != RD_OK) return st;
-  st = tonemap_out(r, rgba, cap);
+  st = finish_image(r, k, rgba);
   if (st != RD_OK) return st;
   *produced = 1;
   return RD_OK;
@@ -445,11 +436,12 @@ rd_status rd_render_frame(rd_renderer *r, const rd_scene *scene, uint8_t *rgba, 
     return r->fail(RD_ERR_BUFFER_TOO_SMALL, "image buffer smaller than W*H*4 bytes");
   rd_status st = rd_new_frame(r, scene);
   if (st != RD_OK) return st;
-  if (r->sample_count < r->cfg.max_sample_count) {
-    st = render_samples(r, r->cfg.max_sample_count - r->sample_count);
+  const uint32_t k = r->cfg.max_sample_count - std::min(r->sample_count, r->cfg.max_sample_count);
+  if (k) {
+    st = render_samples(r, k);
     if (st != RD_OK) return st;
   }
-  return tonemap_out(r, rgba, cap);
+  return finish_image(r, k, rgba);
 }
 
 rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t *rgba,
@@ -577,22 +569,17 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   rdh::fill_job(*scene, ds, acc, r->cfg.max_bounces, r->seed, &job);
   rdh::DevJob *d_job = reinterpret_cast<rdh::DevJob *>(base + o_job);
   const hipStream_t st = se.stream;
-  struct Up {
-    void *dst;
-    const void *src;
-    uint64_t bytes;
-  } ups[] = {{ds.nodes, b.nodes.data(), sizeof(rdh::DevNode) * b.nodes.size()},
-             {ds.nodes4, b.nodes4.data(), sizeof(rdh::DevNode4) * b.nodes4.size()},
-             {ds.prims, b.prims.data(), sizeof(rdh::DevPrim) * b.prims.size()},
-             {ds.objects, b.objects.data(), sizeof(rdh::DevObject) * b.objects.size()},
-             {d_job, &job, sizeof(job)}};
+  // the scene's arrays are neighbours in the scratch
+  const rdh::HostTransfer::Piece scene_pieces[] = {
+      {b.nodes.data(), 0, sizeof(rdh::DevNode) * b.nodes.size()},
+      {b.nodes4.data(), o_nodes4 - o_nodes, sizeof(rdh::DevNode4) * b.nodes4.size()},
+      {b.prims.data(), o_prims - o_nodes, sizeof(rdh::DevPrim) * b.prims.size()},
+      {b.objects.data(), o_obj - o_nodes, sizeof(rdh::DevObject) * b.objects.size()}};
   // every call starts from its own state: the accumulator is cleared by a
   // kernel and the control block by run_tickets; the rest is written before
   // it is read
-  bool ok = true;
-  for (const Up &u : ups)
-    if (ok && u.bytes)
-      ok = se.check(hipMemcpyAsync(u.dst, u.src, u.bytes, hipMemcpyHostToDevice, st), "upload scene", &err);
+  bool ok = se.check(se.transfer().upload(base + o_nodes, scene_pieces, 4, st), "upload scene", &err) &&
+            se.upload(d_job, &job, sizeof(job), "upload job", &err);
   ok = ok && se.check(rdh::launch_zero_acc(acc, 4 * npix, st), "zero accumulator", &err);
   // render_next_sample timers (cpu.rs:194-196, 212-218) around passes of
   // as many samples as the radiance slots hold, in sample order
@@ -629,7 +616,7 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
        se.check(rdh::launch_tonemap(d_job, (uint32_t)npix, (float)(ok ? total : 0), img, eb.counters,
                                     false, grid, st),
                 "tonemap", &err) &&
-       se.check(hipMemcpyAsync(rgba, img, 4 * npix, hipMemcpyDeviceToHost, st), "read image", &err);
+       se.read(rgba, img, 4 * npix, "read image", &err);
   std::string sync_err;
   const bool synced = se.check(hipStreamSynchronize(st), "render", &sync_err);
   if (ok && !synced) err = sync_err;
@@ -687,10 +674,7 @@ rd_status rd_read_accumulator(rd_renderer *r, float *out, size_t cap) {
   const uint64_t n = 4ull * r->W * r->H;
   if (cap < n) return r->fail(RD_ERR_BUFFER_TOO_SMALL, "accumulator buffer too small");
   std::string err;
-  if (!r->eng.check(hipMemcpyAsync(out, r->acc, 4 * n, hipMemcpyDeviceToHost, r->eng.stream),
-                    "read accumulator", &err) ||
-      !r->eng.check(hipStreamSynchronize(r->eng.stream), "read accumulator", &err))
-    return device_fail(r, err);
+  if (!r->eng.read(out, r->acc, 4 * n, "read accumulator", &err)) return device_fail(r, err);
   return RD_OK;
 }
 

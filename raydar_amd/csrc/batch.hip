@@ -360,17 +360,13 @@ class Streamer {
       if (!eng.check(eng.dmalloc((void **)&j->acc, 24 * npix), "hipMalloc(accumulator)", &err)) return false;
       if (!eng.check(eng.dmalloc((void **)&j->rgba_d, 4 * npix), "hipMalloc(image)", &err)) return false;
       if (!eng.check(launch_zero_acc(j->acc, 6 * npix, eng.stream), "zero accumulator", &err)) return false;
-      // the host mirror entry outlives the asynchronous copy
       DevJob &dj = h_jobs_[j->slot];
       fill_job(j->scene, j->dev, j->acc, j->bounces, j->seed, &dj);
       dj.first_hit = reinterpret_cast<HitWord *>(j->acc + 4 * npix);
       DevTicket probe{};
       probe.spp = j->pass_spp;
       j->path_frame = eng.takes_paths(dj, probe) ? ++path_frames_ : 0;
-      if (!eng.check(hipMemcpyAsync(d_jobs_ + j->slot, &dj, sizeof(DevJob), hipMemcpyHostToDevice,
-                                    eng.stream),
-                     "upload job", &err))
-        return false;
+      if (!eng.upload(d_jobs_ + j->slot, &dj, sizeof(DevJob), "upload job", &err)) return false;
       if (j->built.nodes.size() > kNarrowStackNodes) wide_ = true;  // (never a path-kernel job)
       j->built = BuiltScene();  // host copy no longer needed
       j->state = 1;
@@ -580,6 +576,7 @@ class Streamer {
         ticket_fin_[t] = 1;
     // accumulate finished passes in pass order, per job
     std::vector<SJob *> finished;
+    std::vector<HostTransfer::Read> reads;
     for (SJob *j : resident_) {
       bool progressed = false;
       while (!j->tickets.empty() && ticket_fin_[j->tickets.front()] == 1) {
@@ -606,22 +603,17 @@ class Streamer {
                        "tonemap", &err))
           return false;
         uint8_t *dst = j->passes_done == j->passes_total ? j->out_rgba : j->progress;
-        if (j->passes_done == j->passes_total && j->progress &&
-            !eng.check(hipMemcpyAsync(j->progress, j->rgba_d, 4 * npix, hipMemcpyDeviceToHost, eng.stream),
-                       "read image", &err))
-          return false;
-        if (dst && !eng.check(hipMemcpyAsync(dst, j->rgba_d, 4 * npix, hipMemcpyDeviceToHost, eng.stream),
-                              "read image", &err))
-          return false;
+        if (j->passes_done == j->passes_total && j->progress) reads.push_back({j->progress, j->rgba_d, 4 * npix});
+        if (dst) reads.push_back({dst, j->rgba_d, 4 * npix});
       }
       if (j->passes_done == j->passes_total) {
-        const uint64_t npix = (uint64_t)j->W * j->H;
-        if (j->out_acc && !eng.check(hipMemcpyAsync(j->out_acc, j->acc, 16 * npix, hipMemcpyDeviceToHost, eng.stream),
-                                     "read accumulator", &err))
-          return false;
+        if (j->out_acc) reads.push_back({j->out_acc, j->acc, 16ull * j->W * j->H});
         finished.push_back(j);
       }
     }
+    if (!reads.empty() && !eng.check(eng.transfer().read(reads.data(), (int)reads.size(), eng.stream, eng.device),
+                                     "read results", &err))
+      return false;
     while (ticket_lo_ < n && ticket_fin_[ticket_lo_] == 2) ++ticket_lo_;
     if (!finished.empty()) {
       if (!eng.check(hipStreamSynchronize(eng.stream), "read results", &err)) return false;
@@ -938,8 +930,7 @@ class SoloLane {
     DevJob h{};
     if (ok) {
       fill_job(j.scene, j.dev, j.acc, j.bounces, j.seed, &h);
-      ok = eng.check(hipMemcpyAsync(d_job_, &h, sizeof(DevJob), hipMemcpyHostToDevice, eng.stream),
-                     "upload job", &err_);
+      ok = eng.upload(d_job_, &h, sizeof(DevJob), "upload job", &err_);
     }
     const std::vector<DevJob> host{h};
     ++frame_serial_;  // the job's passes share its camera-ray hits
@@ -958,13 +949,12 @@ class SoloLane {
       const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((npix + 255) / 256, 8192));
       ok = eng.check(launch_tonemap(d_job_, (uint32_t)npix, (float)j.spp, j.rgba_d, eng.counters,
                                     false, grid, eng.stream),
-                     "tonemap", &err_) &&
-           (!j.out_rgba || eng.check(hipMemcpyAsync(j.out_rgba, j.rgba_d, 4 * npix,
-                                                    hipMemcpyDeviceToHost, eng.stream),
-                                     "read image", &err_)) &&
-           (!j.out_acc || eng.check(hipMemcpyAsync(j.out_acc, j.acc, 16 * npix,
-                                                   hipMemcpyDeviceToHost, eng.stream),
-                                    "read accumulator", &err_));
+                     "tonemap", &err_);
+      std::vector<HostTransfer::Read> reads;
+      if (j.out_rgba) reads.push_back({j.out_rgba, j.rgba_d, 4 * npix});
+      if (j.out_acc) reads.push_back({j.out_acc, j.acc, 16 * npix});
+      ok = ok && eng.check(eng.transfer().read(reads.data(), (int)reads.size(), eng.stream, eng.device),
+                           "read results", &err_);
     }
     // nothing may be in flight when the job's buffers are freed
     const bool synced = eng.check(hipStreamSynchronize(eng.stream), "render", ok ? &err_ : &ignored);

@@ -52,6 +52,7 @@ void Engine::bind_external(const ExternalBuffers &b, const Engine &owner) {
   device = owner.device;
   num_cus = owner.num_cus;
   stream = owner.stream;
+  transfer_ = owner.transfer_;
   ctl_host = owner.ctl_host;
   q[0] = b.q[0];
   q[1] = b.q[1];
@@ -282,7 +283,24 @@ void Engine::dfree(void *p) {
   else (void)hipFree(p);
 }
 
-bool Engine::upload_scene(const BuiltScene &b, DeviceScene *out, std::string *err) {
+// The job record, then the scene's arrays, each 256-byte aligned.
+static uint64_t scene_pieces(const BuiltScene &b, const DevJob *job, HostTransfer::Piece p[5]) {
+  uint64_t end = 0;
+  int n = 0;
+  auto place = [&](const void *src, uint64_t bytes) {
+    const uint64_t at = (end + 255) & ~255ull;
+    p[n++] = {src, at, bytes};
+    end = at + bytes;
+  };
+  place(job, sizeof(DevJob));
+  place(b.nodes4.data(), sizeof(DevNode4) * b.nodes4.size());
+  place(b.prims.data(), sizeof(DevPrim) * b.prims.size());
+  place(b.objects.data(), sizeof(DevObject) * b.objects.size());
+  place(b.nodes.data(), sizeof(DevNode) * b.nodes.size());
+  return end;
+}
+
+bool Engine::alloc_scene(const BuiltScene &b, DeviceScene *out, std::string *err) {
   free_scene(out);
   out->n_nodes = (uint32_t)b.nodes.size();
   out->n_nodes4 = (uint32_t)b.nodes4.size();
@@ -291,34 +309,28 @@ bool Engine::upload_scene(const BuiltScene &b, DeviceScene *out, std::string *er
   out->n_prims = (uint32_t)b.prims.size();
   out->r0 = b.r0;
   out->depth = b.depth;
-  const size_t nb = sizeof(DevNode) * b.nodes.size(), pb = sizeof(DevPrim) * b.prims.size(),
-               ob = sizeof(DevObject) * b.objects.size(), n4 = sizeof(DevNode4) * b.nodes4.size();
-  out->bytes = nb + pb + ob + n4;
-  if (nb && !check(dmalloc((void **)&out->nodes, nb), "hipMalloc(bvh)", err)) return false;
-  if (n4 && !check(dmalloc((void **)&out->nodes4, n4), "hipMalloc(bvh4)", err)) return false;
-  if (pb && !check(dmalloc((void **)&out->prims, pb), "hipMalloc(prims)", err)) return false;
-  if (ob && !check(dmalloc((void **)&out->objects, ob), "hipMalloc(objects)", err)) return false;
-  if (nb && !check(hipMemcpyAsync(out->nodes, b.nodes.data(), nb, hipMemcpyHostToDevice, stream),
-                   "upload bvh", err))
-    return false;
-  if (n4 && !check(hipMemcpyAsync(out->nodes4, b.nodes4.data(), n4, hipMemcpyHostToDevice, stream),
-                   "upload bvh4", err))
-    return false;
-  if (pb && !check(hipMemcpyAsync(out->prims, b.prims.data(), pb, hipMemcpyHostToDevice, stream),
-                   "upload prims", err))
-    return false;
-  if (ob && !check(hipMemcpyAsync(out->objects, b.objects.data(), ob, hipMemcpyHostToDevice,
-                                  stream),
-                   "upload objects", err))
-    return false;
-  return check(hipStreamSynchronize(stream), "upload scene", err);
+  HostTransfer::Piece p[5];
+  const uint64_t total = scene_pieces(b, nullptr, p);
+  out->bytes = p[1].bytes + p[2].bytes + p[3].bytes + p[4].bytes;
+  if (!check(dmalloc((void **)&out->base, total), "hipMalloc(scene)", err)) return false;
+  auto at = [&](int k) { return p[k].bytes ? out->base + p[k].offset : nullptr; };
+  out->job = reinterpret_cast<DevJob *>(at(0));
+  out->nodes4 = reinterpret_cast<DevNode4 *>(at(1));
+  out->prims = reinterpret_cast<DevPrim *>(at(2));
+  out->objects = reinterpret_cast<DevObject *>(at(3));
+  out->nodes = reinterpret_cast<DevNode *>(at(4));
+  return true;
+}
+
+bool Engine::copy_scene(const BuiltScene &b, const DeviceScene &s, const DevJob *job, std::string *err) {
+  HostTransfer::Piece p[5];
+  scene_pieces(b, job, p);
+  if (!job) p[0].bytes = 0;
+  return check(transfer_->upload(s.base, p, 5, stream), "upload scene", err);
 }
 
 void Engine::free_scene(DeviceScene *s) {
-  dfree(s->nodes);
-  dfree(s->nodes4);
-  dfree(s->prims);
-  dfree(s->objects);
+  dfree(s->base);
   *s = DeviceScene();
 }
 

@@ -21,11 +21,14 @@
 #include "kernels.hpp"
 #include "layout.hpp"
 #include "paths.hpp"
+#include "transfer.hpp"
 
 namespace rdh {
 
-// Device copy of a BuiltScene.
+// Device copy of a BuiltScene, in one allocation.
 struct DeviceScene {
+  unsigned char *base = nullptr;
+  DevJob *job = nullptr;  // a job record's place beside it
   DevNode *nodes = nullptr;
   DevNode4 *nodes4 = nullptr;
   uint32_t n_nodes4 = 0, stack4 = 0;
@@ -117,8 +120,8 @@ class Engine {
   ~Engine();
   // Selects the device and creates the stream; allocation is lazy.
   bool init(std::string *err);
-  // Borrows every device buffer from `b`, the stream and pinned control-block
-  // copy from `owner` (an initialised engine): no allocation, no pipes.  The
+  // Borrows every device buffer from `b`, the stream, pinned control-block
+  // copy and transfers from `owner` (an initialised engine): no allocation, no pipes.  The
   // engine frees nothing it borrowed.
   void bind_external(const ExternalBuffers &b, const Engine &owner);
   bool external() const { return external_; }
@@ -127,7 +130,13 @@ class Engine {
   bool ensure_buffers(std::string *err, bool queues = true);
   void release_buffers();
 
-  bool upload_scene(const BuiltScene &b, DeviceScene *out, std::string *err);
+  // Allocates a scene's device copy; copies it (in stream order), with a job
+  // record if there is one; both.
+  bool alloc_scene(const BuiltScene &b, DeviceScene *out, std::string *err);
+  bool copy_scene(const BuiltScene &b, const DeviceScene &s, const DevJob *job, std::string *err);
+  bool upload_scene(const BuiltScene &b, DeviceScene *out, std::string *err) {
+    return alloc_scene(b, out, err) && copy_scene(b, *out, nullptr, err);
+  }
   void free_scene(DeviceScene *s);
   // Job buffers: from `cache` when one is set, else hipMalloc / hipFree.
   DeviceCache *cache = nullptr;
@@ -154,6 +163,15 @@ class Engine {
   bool run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame,
                  std::string *err);
   uint64_t cam_bytes() const { return cam_px_ * kCamBytes; }
+
+  // Host copies on `stream` (see HostTransfer).
+  HostTransfer &transfer() { return *transfer_; }
+  bool upload(void *dst, const void *src, uint64_t bytes, const char *what, std::string *err) {
+    return check(transfer_->upload(dst, src, bytes, stream), what, err);
+  }
+  bool read(void *dst, const void *src, uint64_t bytes, const char *what, std::string *err) {
+    return check(transfer_->read(dst, src, bytes, stream, device), what, err);
+  }
 
   bool check(hipError_t e, const char *what, std::string *err);
 
@@ -208,6 +226,8 @@ class Engine {
   // Pipes of a one-job pass (see run_tickets).
   int pipes_for(const DevTicket &t, bool lds) const;
   bool ensure_aux(int n, std::string *err);
+  HostTransfer own_transfer_;
+  HostTransfer *transfer_ = &own_transfer_;
   bool external_ = false;  // buffers, stream and control copy are borrowed
   std::vector<hipEvent_t> ev_pool_;
   std::vector<std::unique_ptr<Engine>> aux_;  // pipes 1.. of run_tickets
