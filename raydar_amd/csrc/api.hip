@@ -519,7 +519,8 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   // that still holds a sample of every pixel (images up to 3.3 M pixels; larger
   // ones stay with the wavefront).
   const uint64_t o_cam = (o_rest + 255) & ~255ull;
-  const uint64_t o_cam_end = (o_cam + rdh::kCamBytes * npix + 255) & ~255ull;
+  const uint64_t o_compact = (o_cam + rdh::kCamBytes * npix + 255) & ~255ull;
+  const uint64_t o_cam_end = (o_compact + sizeof(rdh::DevNode4C) * b.nodes4.size() + 255) & ~255ull;
   const bool cam_fits = o_cam_end + 16 * npix <= rdh::kScratchBytes;
 
   rdh::ExternalBuffers eb{};
@@ -544,6 +545,8 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   if (cam_fits) {
     eb.cam = base + o_cam;
     eb.cam_px = npix;
+    eb.compact = reinterpret_cast<rdh::DevNode4C *>(base + o_compact);
+    eb.compact_nodes = (uint32_t)b.nodes4.size();
   }
   se.bind_external(eb, r->eng);
 

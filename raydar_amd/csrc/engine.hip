@@ -71,6 +71,9 @@ void Engine::bind_external(const ExternalBuffers &b, const Engine &owner) {
   cam_ = b.cam;
   cam_px_ = b.cam_px;
   cam_frame_ = 0;
+  compact_ = b.compact;
+  compact_nodes_ = b.compact_nodes;
+  compact_frame_ = 0;
   opt.queue = b.queue;
   opt.l_capacity = b.l_slots;
   opt.pipes = 1;
@@ -92,6 +95,9 @@ void Engine::release_buffers() {
   first_hit_frame_ = 0;
   if (cam_) { (void)hipFree(cam_); cam_ = nullptr; }
   if (path_ctl_) { (void)hipFree(path_ctl_); path_ctl_ = nullptr; }
+  if (compact_) { (void)hipFree(compact_); compact_ = nullptr; }
+  compact_nodes_ = 0;
+  compact_frame_ = 0;
   cam_px_ = 0;
   cam_frame_ = 0;
   q_alloc = 0;
@@ -175,7 +181,7 @@ uint64_t Engine::device_bytes() const {
   // two queues of 14 words per slot plus the 8-byte hit record
   uint64_t b = (uint64_t)kSegments * seg_cap * (2 * 56 + 8) + l_alloc * sizeof(float4) +
                (uint64_t)ticket_alloc * (sizeof(DevTicket) + 8) + first_hit_px_ * sizeof(HitWord) +
-               cam_px_ * kCamBytes;
+               cam_px_ * kCamBytes + compact_nodes_ * sizeof(DevNode4C);
   for (const auto &e : aux_) b += e->device_bytes();
   return b;
 }
@@ -471,7 +477,8 @@ int Engine::pipes_for(const DevTicket &t, bool lds) const {
 // tree), event counts, and the launch forms asked for by option (one ray per
 // lane, other workgroup sizes, every camera ray traced).
 bool Engine::takes_paths(const DevJob &j, const DevTicket &t) const {
-  if (!launch_paths || (external_ && cam_px_ < (uint64_t)j.width * j.height)) return false;
+  if (!launch_paths || (external_ && (cam_px_ < (uint64_t)j.width * j.height || compact_nodes_ < j.n_nodes4)))
+    return false;
   return !opt.count && opt.hit_reuse && !opt.brute_force && opt.refill > 0 && opt.bvh4 &&
          opt.block == 256 && j.max_bounces > 0 && j.max_bounces <= 255 && t.spp < (1u << 24) &&
          j.n_nodes4 > 0 && j.n_nodes <= kNarrowStackNodes && j.stack4 + 3 <= (uint32_t)kStackDepth;
@@ -509,6 +516,20 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
   a.refill = (uint32_t)opt.refill;
   // (the tree bound's default and more: whatever fits)
   plan_paths(&a, j, opt.lds_bvh >= EngineOptions().lds_bvh ? UINT64_MAX : opt.lds_bvh, opt.lds_objects);
+
+  a.n_nodes4 = j.n_nodes4;
+  if (a.tree == kTreeCompact) {
+    if (j.n_nodes4 > compact_nodes_) {
+      if (compact_) (void)hipFree(compact_);
+      compact_ = nullptr;
+      compact_nodes_ = 0;
+      compact_frame_ = 0;
+      const uint32_t n = std::max(1024u, j.n_nodes4 + j.n_nodes4 / 4);
+      if (!check(hipMalloc((void **)&compact_, sizeof(DevNode4C) * n), "hipMalloc(compact tree)", err)) return false;
+      compact_nodes_ = n;
+    }
+    a.compact = compact_;
+  }
 
   // Everything is queued without a wait in between; the caller waits for the
   // accumulation.  A launch's waves take its work list in chunks through a
@@ -571,6 +592,13 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
     if (!check(hipEventCreate(&e0), "hipEventCreate", err) || !check(hipEventCreate(&e1), "hipEventCreate", err) ||
         !check(hipEventRecord(e0, stream), "hipEventRecord", err))
       return false;
+  }
+  if (a.tree == kTreeCompact) {
+    // (an option may have sent the frame's first passes to the other form)
+    const bool have = frame != 0 && frame == compact_frame_;
+    compact_frame_ = 0;
+    if (!have && !check(launch_compact(a, stream), "compact tree", err)) return false;
+    compact_frame_ = frame;
   }
   if (!carried && !launch(true)) return false;
   if (!launch(false)) return false;

@@ -113,6 +113,8 @@ struct ExternalBuffers {
   uint32_t tickets_n;   // ticket table entries
   unsigned char *cam;   // the path kernel's camera-hit table, or nullptr
   uint64_t cam_px;      // pixels it holds
+  DevNode4C *compact;   // and compact tree
+  uint32_t compact_nodes;
 };
 
 class Engine {
@@ -242,6 +244,9 @@ class Engine {
   unsigned char *cam_ = nullptr;              // the path kernel's camera-hit table
   uint64_t cam_px_ = 0;                       // pixels it holds
   uint64_t cam_frame_ = 0;                    // hit_frame whose hits it holds (0: none)
+  DevNode4C *compact_ = nullptr;              // the path kernel's compact tree
+  uint64_t compact_frame_ = 0;                // hit_frame whose tree it is (0: none)
+  uint32_t compact_nodes_ = 0;                // nodes it has room for
 };
 
 // Message returned by rd_last_error(NULL) (calls with no renderer handle).

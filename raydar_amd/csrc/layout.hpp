@@ -70,6 +70,19 @@ struct alignas(16) DevNode4 {
 };
 static_assert(sizeof(DevNode4) == 128, "DevNode4 must be 128 bytes");
 
+// A DevNode4 whose leaves hold one primitive each, in half the bytes (made from
+// it by k_compact in paths.hip): planes as FP16 offsets, in units of a power of
+// two, from an origin of the node's own, rounded outward.
+struct alignas(16) DevNode4C {
+  // origin x, y, z as the upper halves of FP32 words over the codes of children
+  // 0..2 (a node's or a primitive's index); the unit over child 3's, with its
+  // sign bit and lowest mantissa bits telling which children are leaves:
+  // bit 31 child 3, bits 18..16 children 2..0
+  uint32_t head[4];
+  uint16_t x[8], y[8], z[8];  // the children's low planes, then their high ones
+};
+static_assert(sizeof(DevNode4C) == 64, "DevNode4C must be 64 bytes");
+
 // Primitive tag in DevPrim::b.w: original object id | kind << 31.
 struct alignas(16) DevPrim {
   // sphere: a = (cx, cy, cz, dot(C,C)), b = (r*r, 0, 0, tag)

@@ -56,7 +56,6 @@ template <int BLOCK>
 __host__ __device__ constexpr uint32_t pool_bytes() {
   return kPoolRows * BLOCK * (uint32_t)sizeof(uint16_t);
 }
-__host__ __device__ constexpr bool pooled(bool lds, bool leaf1) { return leaf1 && !lds; }
 
 // Visit keys of the walk: see the sort in k_paths.
 constexpr uint32_t kNoKey = 0xffffffffu;
@@ -65,6 +64,12 @@ __device__ __forceinline__ uint32_t umin(uint32_t a, uint32_t b) { return a < b 
 __device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
 __device__ __forceinline__ uint32_t umed3(uint32_t a, uint32_t b, uint32_t c) {
   return umin(umax(a, b), umax(umin(a, b), c));
+}
+
+// the FP16 numbers of a word (v_fma_mix takes them as they are)
+__device__ __forceinline__ float half_lo(int w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)w); }
+__device__ __forceinline__ float half_hi(int w) {
+  return (float)__builtin_bit_cast(_Float16, (uint16_t)((uint32_t)w >> 16));
 }
 
 // A walk's ray: dot(d, d) in [kMinDot, kMaxDot] besides walkable().
@@ -160,10 +165,76 @@ __device__ __forceinline__ F3 camera_origin(const DevJob &J) {
   return o;
 }
 
+// q in [-2, 2] as FP16, rounded down or up and never subnormal.
+__device__ __forceinline__ uint16_t half_toward(float q, bool up) {
+  if (up) q = -q;  // round down the negative
+  uint16_t b;
+  if (fabsf(q) < 0x1p-14f) {
+    b = q < 0.0f ? 0x8400u : 0u;
+  } else {
+    const _Float16 h = (_Float16)q;
+    b = __builtin_bit_cast(uint16_t, h);
+    if ((float)h > q) b = (uint16_t)(q < 0.0f ? b + 1u : b - 1u);
+  }
+  return up ? (uint16_t)(b ^ 0x8000u) : b;
+}
+
+// DevNode4 -> DevNode4C, a thread per node; a few microseconds once a frame.
+__global__ __launch_bounds__(64) void k_compact(const DevJob *job, DevNode4C *out, uint32_t n) {
+  const uint32_t i = blockIdx.x * 64u + threadIdx.x;
+  if (i >= n) return;
+  const DevNode4 nd = load_constant(&job->nodes4)[i];
+  bool used[4];
+  uint32_t code[4], flags = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int32_t c = nd.child[k];
+    used[k] = !is_leaf(c) || leaf_count(c) > 0;
+    code[k] = is_leaf(c) ? (used[k] ? leaf_first(c) : 0u) : (uint32_t)c;
+    if (is_leaf(c)) flags |= k < 3 ? 0x10000u << k : 0x80000000u;
+  }
+  float origin[3], slack[3], reach = 0.0f;
+  auto place = [&](int x, const float *lo, const float *hi) {
+    float a = INFINITY, b = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (used[k]) {
+        a = fminf(a, lo[k]);
+        b = fmaxf(b, hi[k]);
+      }
+    // any origin will do; this one is near the middle
+    origin[x] = bitsf(fbits(0.5f * a + 0.5f * b) & 0xffff0000u);
+    // for the subtractions below and the walk's inner rounding
+    slack[x] = 0x1p-21f * (fabsf(a) + fabsf(b));
+    reach = fmaxf(reach, fmaxf(fabsf(a - origin[x]), fabsf(b - origin[x])) + slack[x]);
+  };
+  place(0, nd.lo_x, nd.hi_x);
+  place(1, nd.lo_y, nd.hi_y);
+  place(2, nd.lo_z, nd.hi_z);
+  // the power of two at or above it
+  const uint32_t unit = min(max((fbits(reach) + 0x7fffffu) & 0x7f800000u, 27u << 23), 247u << 23);
+  const float per = bitsf((254u << 23) - unit);
+  DevNode4C c;
+  auto planes = [&](int x, const float *lo, const float *hi, uint16_t *p) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      p[k] = used[k] ? half_toward((lo[k] - origin[x] - slack[x]) * per, false) : 0x7c00u;
+      p[4 + k] = used[k] ? half_toward((hi[k] - origin[x] + slack[x]) * per, true) : 0xfc00u;
+    }
+  };
+  planes(0, nd.lo_x, nd.hi_x, c.x);
+  planes(1, nd.lo_y, nd.hi_y, c.y);
+  planes(2, nd.lo_z, nd.hi_z, c.z);
+#pragma unroll
+  for (int x = 0; x < 3; ++x) c.head[x] = fbits(origin[x]) | code[x];
+  c.head[3] = unit | code[3] | flags;
+  out[i] = c;
+}
+
 // RECORD: trace every pixel's camera ray and write its hit to the table, in
 // the order the paths are handed out (tile_order_pixel).
-// LDS: the tree and the primitives are copied into LDS by every workgroup.
-// LEAF1: every leaf holds one primitive.
+// LDS trees and the primitives are copied into LDS by every workgroup; LEAF1:
+// every leaf holds one primitive.
 // VK (Vulkan semantics): a pixel's samples share one stream of random numbers,
 // whose place after a sample depends on that sample's draws, so a lane keeps
 // its pixel for all samples of the pass, one after another, with the stream's
@@ -171,11 +242,13 @@ __device__ __forceinline__ F3 camera_origin(const DevJob &J) {
 // k_accumulate would take).  The camera ray has no draw in it here either.
 // 97 objects, 1280x720, 16 spp: 8.1 -> 3.5 ms, which were 16 passes of one
 // sample with 12 bounces of three launches each; 2.8 ms with the shorter walk.
-template <int BLOCK, bool RECORD, bool LDS, bool LEAF1, bool VK>
+template <int BLOCK, bool RECORD, PathTree TREE, bool VK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(path_waves(RECORD, VK), 8)))
 void k_paths(PathArgs a) {
   typedef uint16_t StackT;
-  constexpr bool kPooled = pooled(LDS, LEAF1);
+  constexpr bool LDS = TREE == kTreeLds || TREE == kTreeLdsLeaf1;
+  constexpr bool LEAF1 = TREE != kTreeMemory && TREE != kTreeLds;
+  constexpr bool kCompact = TREE == kTreeCompact, kPooled = LEAF1 && !LDS;
   extern __shared__ __align__(16) unsigned char dynamic_lds[];
   // Job fields are scalar loads.  What a walk needs stays in registers; the
   // shading's fields are read again in every turn: held across the walk, they
@@ -186,6 +259,7 @@ void k_paths(PathArgs a) {
   const DevPrim *prims = load_constant(&a.job->prims);
   const uint32_t n_nodes4 = load_constant(&a.job->n_nodes4), n_prims = load_constant(&a.job->n_prims);
   (void)n_nodes4;
+  (void)nodes4;
   const uint32_t stack_bytes = (a.stack_rows * BLOCK * (uint32_t)sizeof(StackT) + 15u) & ~15u;
   // The lane's stack column: rows of kRow bytes, the last holding kNoNode for
   // good, so that a pop needs no look at the depth.
@@ -255,6 +329,7 @@ void k_paths(PathArgs a) {
   uint32_t sp = 0;          // byte offset two rows past the next stack entry to write
   RayPre r;
   SlabNF nf;
+  bool neg_x = false, neg_y = false, neg_z = false;  // (a compact tree's)
   float ya = 0.0f;  // RN(1 / dot(d, d))
 
   // The lane's path ends with radiance c.  VK: the pixel's next sample, if the
@@ -305,8 +380,9 @@ void k_paths(PathArgs a) {
     }
     test_in_walk<VK>(r, ya, nf.ix, nf.iy, nf.iz, pr, &best);
   };
-  // the primitive of a one-primitive leaf (in LDS the code is the index)
-  auto leaf_prim = [&](int32_t code) { return (uint16_t)(LDS && LEAF1 ? code : code >> 4); };
+  // the primitive of a one-primitive leaf (in LDS and compact trees the code's
+  // lower half)
+  auto leaf_prim = [&](int32_t code) { return (uint16_t)(LDS || kCompact ? code : code >> 4); };
 
   for (;;) {
     // ---- a turn: shade the lanes whose walk has ended, refill the free ones
@@ -458,6 +534,9 @@ void k_paths(PathArgs a) {
       }
       ya = rcp_rn_normal(r.a);
       nf = slab_nf(slab_ray(r, ray_tolerance(r, J.r0_tol)));
+      neg_x = nf.ix < 0.0f;
+      neg_y = nf.iy < 0.0f;
+      neg_z = nf.iz < 0.0f;
       tcull = cull();
     }
     // ---- the walk, until enough lanes are out of it: with work left every
@@ -493,42 +572,92 @@ void k_paths(PathArgs a) {
 #ifdef RDH_CHECKED
         node = chk(node, n_nodes4, K_NODE, a.ctl);
 #endif
-        // each axis's near and far planes of the four children, picked by the
-        // ray's direction signs (slab_hit_nf)
-        VecF4 xn, xf, yn, yf, zn, zf;
-        VecI4 ch;
-        if (LDS) {
-          const unsigned char *np = reinterpret_cast<const unsigned char *>(lds_nodes + 8 * node);
-          xn = *(const VecF4 *)(np + nf.ox); xf = *(const VecF4 *)((np - nf.ox) + 16);
-          yn = *(const VecF4 *)(np + nf.oy); yf = *(const VecF4 *)((np - nf.oy) + 80);
-          zn = *(const VecF4 *)(np + nf.oz); zf = *(const VecF4 *)((np - nf.oz) + 144);
-          ch = *(const VecI4 *)(np + 96);
-        } else {
-          // 32-bit offsets from the tree's base keep the address arithmetic
-          // out of 64-bit registers
-          const __attribute__((address_space(1))) unsigned char *gb =
-              (const __attribute__((address_space(1))) unsigned char *)nodes4;
-          const uint32_t nb = node * (uint32_t)sizeof(DevNode4);
-          xn = *(GlobalF4 *)(gb + (nb + nf.ox)); xf = *(GlobalF4 *)(gb + ((nb - nf.ox) + 16u));
-          yn = *(GlobalF4 *)(gb + (nb + nf.oy)); yf = *(GlobalF4 *)(gb + ((nb - nf.oy) + 80u));
-          zn = *(GlobalF4 *)(gb + (nb + nf.oz)); zf = *(GlobalF4 *)(gb + ((nb - nf.oz) + 144u));
-          ch = *(GlobalI4 *)(gb + (nb + 96u));
-        }
         float t0, t1, t2, t3;
-        const bool h0 = slab_hit_nf(nf, xn.x, xf.x, yn.x, yf.x, zn.x, zf.x, tcull, &t0);
-        const bool h1 = slab_hit_nf(nf, xn.y, xf.y, yn.y, yf.y, zn.y, zf.y, tcull, &t1);
-        const bool h2 = slab_hit_nf(nf, xn.z, xf.z, yn.z, yf.z, zn.z, zf.z, tcull, &t2);
-        const bool h3 = slab_hit_nf(nf, xn.w, xf.w, yn.w, yf.w, zn.w, zf.w, tcull, &t3);
-        // The entered inner children, nearest first.  A key is the entry
-        // distance's upper 16 bits (it only orders the visits) above the
-        // child's index; a leaf's code leaves the sign bit set, as kNoKey has
-        // it, so those keys sort behind.  Seven integer min/med/max steps
-        // order distance and child together (the float form took a compare
-        // and four selects for each of five exchanges).
-        const uint32_t e0 = h0 ? (fbits(t0) & 0x7fff0000u) | (uint32_t)ch.x : kNoKey;
-        const uint32_t e1 = h1 ? (fbits(t1) & 0x7fff0000u) | (uint32_t)ch.y : kNoKey;
-        const uint32_t e2 = h2 ? (fbits(t2) & 0x7fff0000u) | (uint32_t)ch.z : kNoKey;
-        const uint32_t e3 = h3 ? (fbits(t3) & 0x7fff0000u) | (uint32_t)ch.w : kNoKey;
+        uint32_t e0, e1, e2, e3;
+        VecI4 ch;
+        bool h0 = false, h1 = false, h2 = false, h3 = false;
+        if constexpr (kCompact) {
+          // DevNode4C: a plane's distance is (origin + h * unit) * i - n, as
+          // fma(h, unit * i, fma(origin, i, -n)) with an exact first product
+          // (unit is a power of two); the inner one rounds by 2^-24 of the
+          // origin's distance, which the margin of k_compact covers.  A NaN from
+          // overflow drops its axis from the test.
+          const __attribute__((address_space(1))) unsigned char *gb =
+              (const __attribute__((address_space(1))) unsigned char *)a.compact;
+          const uint32_t nb = node * (uint32_t)sizeof(DevNode4C);
+          const VecI4 hd = *(GlobalI4 *)(gb + nb), wx = *(GlobalI4 *)(gb + (nb + 16u));
+          const VecI4 wy = *(GlobalI4 *)(gb + (nb + 32u)), wz = *(GlobalI4 *)(gb + (nb + 48u));
+          const float unit = bitsf((uint32_t)hd.w & 0x7f800000u);
+          const float cx = bitsf((uint32_t)hd.x & 0xffff0000u), cy = bitsf((uint32_t)hd.y & 0xffff0000u);
+          const float cz = bitsf((uint32_t)hd.z & 0xffff0000u);
+          const float sx = unit * nf.ix, sy = unit * nf.iy, sz = unit * nf.iz;
+          const float bnx = fmaf(cx, nf.ix, -nf.nx), bfx = fmaf(cx, nf.ix, -nf.fx);
+          const float bny = fmaf(cy, nf.iy, -nf.ny), bfy = fmaf(cy, nf.iy, -nf.fy);
+          const float bnz = fmaf(cz, nf.iz, -nf.nz), bfz = fmaf(cz, nf.iz, -nf.fz);
+          const int xna = neg_x ? wx.z : wx.x, xnb = neg_x ? wx.w : wx.y;
+          const int xfa = neg_x ? wx.x : wx.z, xfb = neg_x ? wx.y : wx.w;
+          const int yna = neg_y ? wy.z : wy.x, ynb = neg_y ? wy.w : wy.y;
+          const int yfa = neg_y ? wy.x : wy.z, yfb = neg_y ? wy.y : wy.w;
+          const int zna = neg_z ? wz.z : wz.x, znb = neg_z ? wz.w : wz.y;
+          const int zfa = neg_z ? wz.x : wz.z, zfb = neg_z ? wz.y : wz.w;
+          auto enters = [&](float xn, float xf, float yn, float yf, float zn, float zf, float *t) {
+            const float tn = fmaxf(fmaxf(fmaf(xn, sx, bnx), fmaf(yn, sy, bny)),
+                                   fmaxf(fmaf(zn, sz, bnz), 0.0f));
+            const float tf = fminf(fminf(fmaf(xf, sx, bfx), fmaf(yf, sy, bfy)),
+                                   fminf(fmaf(zf, sz, bfz), tcull));
+            *t = tn;
+            return tn <= tf;
+          };
+          h0 = enters(half_lo(xna), half_lo(xfa), half_lo(yna), half_lo(yfa), half_lo(zna), half_lo(zfa), &t0);
+          h1 = enters(half_hi(xna), half_hi(xfa), half_hi(yna), half_hi(yfa), half_hi(zna), half_hi(zfa), &t1);
+          h2 = enters(half_lo(xnb), half_lo(xfb), half_lo(ynb), half_lo(yfb), half_lo(znb), half_lo(zfb), &t2);
+          h3 = enters(half_hi(xnb), half_hi(xfb), half_hi(ynb), half_hi(yfb), half_hi(znb), half_hi(zfb), &t3);
+          // keys as below, the leaf flag moved to the sign bit
+          auto key = [](float t, int code, uint32_t flag) {
+            return (flag & 0x80000000u) | (((uint32_t)code & 0xffffu) | (fbits(t) & 0x7fff0000u));
+          };
+          const uint32_t fl = (uint32_t)hd.w;
+          e0 = h0 ? key(t0, hd.x, fl << 15) : kNoKey;
+          e1 = h1 ? key(t1, hd.y, fl << 14) : kNoKey;
+          e2 = h2 ? key(t2, hd.z, fl << 13) : kNoKey;
+          e3 = h3 ? key(t3, hd.w, fl) : kNoKey;
+          ch = hd;
+        } else {
+          // each axis's near and far planes of the four children, picked by the
+          // ray's direction signs (slab_hit_nf)
+          VecF4 xn, xf, yn, yf, zn, zf;
+          if (LDS) {
+            const unsigned char *np = reinterpret_cast<const unsigned char *>(lds_nodes + 8 * node);
+            xn = *(const VecF4 *)(np + nf.ox); xf = *(const VecF4 *)((np - nf.ox) + 16);
+            yn = *(const VecF4 *)(np + nf.oy); yf = *(const VecF4 *)((np - nf.oy) + 80);
+            zn = *(const VecF4 *)(np + nf.oz); zf = *(const VecF4 *)((np - nf.oz) + 144);
+            ch = *(const VecI4 *)(np + 96);
+          } else {
+            // 32-bit offsets from the tree's base keep the address arithmetic
+            // out of 64-bit registers
+            const __attribute__((address_space(1))) unsigned char *gb =
+                (const __attribute__((address_space(1))) unsigned char *)nodes4;
+            const uint32_t nb = node * (uint32_t)sizeof(DevNode4);
+            xn = *(GlobalF4 *)(gb + (nb + nf.ox)); xf = *(GlobalF4 *)(gb + ((nb - nf.ox) + 16u));
+            yn = *(GlobalF4 *)(gb + (nb + nf.oy)); yf = *(GlobalF4 *)(gb + ((nb - nf.oy) + 80u));
+            zn = *(GlobalF4 *)(gb + (nb + nf.oz)); zf = *(GlobalF4 *)(gb + ((nb - nf.oz) + 144u));
+            ch = *(GlobalI4 *)(gb + (nb + 96u));
+          }
+          h0 = slab_hit_nf(nf, xn.x, xf.x, yn.x, yf.x, zn.x, zf.x, tcull, &t0);
+          h1 = slab_hit_nf(nf, xn.y, xf.y, yn.y, yf.y, zn.y, zf.y, tcull, &t1);
+          h2 = slab_hit_nf(nf, xn.z, xf.z, yn.z, yf.z, zn.z, zf.z, tcull, &t2);
+          h3 = slab_hit_nf(nf, xn.w, xf.w, yn.w, yf.w, zn.w, zf.w, tcull, &t3);
+          // The entered inner children, nearest first.  A key is the entry
+          // distance's upper 16 bits (it only orders the visits) above the
+          // child's index; a leaf's code leaves the sign bit set, as kNoKey has
+          // it, so those keys sort behind.  Seven integer min/med/max steps
+          // order distance and child together (the float form took a compare
+          // and four selects for each of five exchanges).
+          e0 = h0 ? (fbits(t0) & 0x7fff0000u) | (uint32_t)ch.x : kNoKey;
+          e1 = h1 ? (fbits(t1) & 0x7fff0000u) | (uint32_t)ch.y : kNoKey;
+          e2 = h2 ? (fbits(t2) & 0x7fff0000u) | (uint32_t)ch.z : kNoKey;
+          e3 = h3 ? (fbits(t3) & 0x7fff0000u) | (uint32_t)ch.w : kNoKey;
+        }
         if constexpr (kPooled) {
           // the entered leaves' primitives go above the lane's others; a key
           // plus one has the sign bit set for a leaf's alone
@@ -583,23 +712,34 @@ void k_paths(PathArgs a) {
   }
 }
 
-template <bool RECORD, bool VK>
-const void *paths_fn_of(bool lds, bool leaf1) {
-  return lds ? (leaf1 ? (const void *)k_paths<kPathBlock, RECORD, true, true, VK>
-                      : (const void *)k_paths<kPathBlock, RECORD, true, false, VK>)
-             : (leaf1 ? (const void *)k_paths<kPathBlock, RECORD, false, true, VK>
-                      : (const void *)k_paths<kPathBlock, RECORD, false, false, VK>);
+template <bool VK>
+const void *paths_fn_of(PathTree tree, bool record) {
+  switch (tree) {
+    case kTreeMemory:
+      return record ? (const void *)k_paths<kPathBlock, true, kTreeMemory, VK>
+                    : (const void *)k_paths<kPathBlock, false, kTreeMemory, VK>;
+    case kTreeCompact:  // camera rays share their nodes: recorded from the tree itself
+      if (!record) return (const void *)k_paths<kPathBlock, false, kTreeCompact, VK>;
+      [[fallthrough]];
+    case kTreeLeaf1:
+      return record ? (const void *)k_paths<kPathBlock, true, kTreeLeaf1, VK>
+                    : (const void *)k_paths<kPathBlock, false, kTreeLeaf1, VK>;
+    case kTreeLds:
+      return record ? (const void *)k_paths<kPathBlock, true, kTreeLds, VK>
+                    : (const void *)k_paths<kPathBlock, false, kTreeLds, VK>;
+    default:
+      return record ? (const void *)k_paths<kPathBlock, true, kTreeLdsLeaf1, VK>
+                    : (const void *)k_paths<kPathBlock, false, kTreeLdsLeaf1, VK>;
+  }
 }
 
 const void *paths_fn(const PathArgs &a, bool record) {
-  const bool lds = a.lds_bvh_bytes > 0, leaf1 = a.leaf1 != 0;
-  if (a.vk) return record ? paths_fn_of<true, true>(lds, leaf1) : paths_fn_of<false, true>(lds, leaf1);
-  return record ? paths_fn_of<true, false>(lds, leaf1) : paths_fn_of<false, false>(lds, leaf1);
+  return a.vk ? paths_fn_of<true>(a.tree, record) : paths_fn_of<false>(a.tree, record);
 }
 
 uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
   return ((a.stack_rows * kPathBlock * 2u + 15u) & ~15u) +
-         (pooled(a.lds_bvh_bytes > 0, a.leaf1 != 0) ? pool_bytes<kPathBlock>() : 0u) +
+         (a.tree == kTreeLeaf1 || a.tree == kTreeCompact ? pool_bytes<kPathBlock>() : 0u) +
          a.lds_bvh_bytes + (record ? 0u : a.lds_obj_bytes);
 }
 
@@ -611,14 +751,24 @@ uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
 // spp: 9.2 ms from memory, 8.0 from LDS.  Larger workgroups that share a copy
 // were slower than the walk in memory: 640 threads 300 objects 1.33 -> 1.45 ms,
 // 500 objects 1.46 -> 1.69 (1280x720, 16 spp, whole call).
+//
+// A larger tree of one-primitive leaves is walked as DevNode4C from 1280 nodes
+// (160 KB of DevNode4) on: four 16-byte loads a node instead of seven, which
+// counts once the node fetches miss the L1, but a third more instructions.
+// 1280x720, 32 spp, full -> compact: 1000 objects (458 nodes) 1.87 -> 1.91 ms,
+// 1500 2.23 -> 2.32, 2500 3.13 -> 3.15, 4096 (1777 nodes) 4.52 -> 4.40, 8000
+// 7.19 -> 6.71.
 void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh, uint64_t lds_objects) {
+  constexpr uint32_t kCompactNodes = 1280;
   a->stack_rows = j.stack4 + 4;  // a sentinel below, and three written above the top
-  a->leaf1 = j.max_leaf == 1 ? 1 : 0;
+  const bool leaf1 = j.max_leaf == 1;
   const uint64_t blocks = 4 * path_waves(false, a->vk) / (kPathBlock / 64);
   const uint64_t room = 160 * 1024 / blocks - 1024, stack = 2ull * a->stack_rows * kPathBlock + 16;
   const uint64_t tree = sizeof(DevNode4) * (uint64_t)j.n_nodes4 + sizeof(DevPrim) * (uint64_t)j.n_prims;
   const uint64_t objects = sizeof(DevObject) * (uint64_t)j.n_prims;
   const bool lds = tree <= lds_bvh && stack + tree <= room;
+  a->tree = lds ? (leaf1 ? kTreeLdsLeaf1 : kTreeLds)
+                : !leaf1 ? kTreeMemory : j.n_nodes4 >= kCompactNodes ? kTreeCompact : kTreeLeaf1;
   a->lds_bvh_bytes = lds ? (uint32_t)tree : 0u;
   const uint64_t used = stack + (lds ? tree : pool_bytes<kPathBlock>());
   a->lds_obj_bytes = objects <= lds_objects && used + objects <= room ? (uint32_t)objects : 0u;
@@ -639,6 +789,11 @@ hipError_t launch_paths(const PathArgs &a, bool record, int grid, hipStream_t st
   void *kargs[] = {&args};
   return hipLaunchKernel(paths_fn(a, record), dim3(grid), dim3(kPathBlock), kargs,
                          dynamic_lds_bytes(a, record), st);
+}
+
+hipError_t launch_compact(const PathArgs &a, hipStream_t st) {
+  k_compact<<<(a.n_nodes4 + 63) / 64, 64, 0, st>>>(a.job, a.compact, a.n_nodes4);
+  return hipGetLastError();
 }
 
 }  // namespace rdh

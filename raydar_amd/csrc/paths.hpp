@@ -10,6 +10,10 @@ namespace rdh {
 constexpr int kPathBlock = 256;                // threads of a workgroup
 constexpr uint32_t kPathSlices = kSegments;  // slices of a work list at most
 
+// The tree a launch walks: DevNode4 in memory, the same with leaves of one
+// primitive, DevNode4C (the same leaves), DevNode4 in LDS, with one-primitive leaves.
+enum PathTree : int { kTreeMemory, kTreeLeaf1, kTreeCompact, kTreeLds, kTreeLdsLeaf1 };
+
 struct PathArgs {
   const DevJob *job;
   QueueCtl *ctl;                // (bounds-checked builds' violation mask)
@@ -21,6 +25,8 @@ struct PathArgs {
   uint2 *cam_hit;
   float4 *L;                    // radiance arena
   unsigned long long l_offset;  // slot of local sample 0, pixel 0
+  DevNode4C *compact;           // kTreeCompact's nodes (launch_compact makes them)
+  uint32_t n_nodes4;
   uint32_t npix;
   uint32_t sample_base;         // global index of local sample 0
   uint32_t spp;                 // samples of a group of ranks in the work list, below 2^24
@@ -35,7 +41,7 @@ struct PathArgs {
   uint32_t lds_bvh_bytes;       // > 0: nodes and primitives copied to LDS
   uint32_t lds_obj_bytes;       // > 0: objects copied to LDS
   uint32_t stack_rows;          // traversal stack entries per lane
-  int leaf1;                    // every leaf holds one primitive
+  PathTree tree;
   int vk;                       // Vulkan semantics: the work list holds each group once and
                                 // the launch accumulates (L is not used)
   unsigned long long l_cap;     // radiance arena entries (bounds-checked builds)
@@ -55,5 +61,6 @@ __attribute__((weak)) void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds
 __attribute__((weak)) int path_blocks_per_cu(const PathArgs &a, bool record);
 __attribute__((weak)) hipError_t launch_paths(const PathArgs &a, bool record, int grid,
                                               hipStream_t st);
+__attribute__((weak)) hipError_t launch_compact(const PathArgs &a, hipStream_t st);
 
 }  // namespace rdh

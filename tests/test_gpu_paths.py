@@ -40,7 +40,7 @@ def test_path_kernel_matches_oracle(size, spp, bounces, opts):
 
 @pytest.mark.parametrize("semantics", [0, 1])
 @pytest.mark.parametrize("objects,opts", [
-    (130, dict()), (185, dict()), (240, dict()), (320, dict()), (420, dict()),
+    (130, dict()), (185, dict()), (240, dict()), (320, dict()), (2850, dict()), (3200, dict()),
     (185, dict(lds_bvh=14335)), (185, dict(lds_bvh=14336, lds_objects=0)),
     (60, dict(lds_bvh=14335, pipes=3, queue=4096))])
 def test_trees_around_what_fits_in_lds(objects, opts, semantics):
@@ -52,6 +52,33 @@ def test_trees_around_what_fits_in_lds(objects, opts, semantics):
     ref = (oracle.render(sc, 3, 12, 3) if semantics == 0 else
            oracle.vk_render(sc, ra.camera_vulkan_inverse_view(sc.camera), 3, 12, threads=8))
     np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("scale,shift", [(1.0, 0.0), (2.0 ** -40, 0.0), (2.0 ** 12, 0.0),
+                                         (1.0, 4096.0), (2.0 ** -12, 1.0), (2.0 ** 40, 0.0)])
+@pytest.mark.parametrize("objects", [2, 97, 2400, 3200])
+def test_compact_tree_at_every_scale(objects, scale, shift):
+    # planes are FP16 offsets in a power of two of each node's own from an
+    # origin of its own: tiny and huge scenes, scenes far from zero, and the
+    # tree's form changing in mid-frame
+    sc = scenegen.clustered(6, objects, 70, 41)
+    sc.objects["center"] = sc.objects["center"] * np.float32(scale) + np.float32(shift)
+    sc.objects["size"] *= np.float32(scale)
+    c = sc.camera
+    at = [[float(np.float32(v * scale + shift)) for v in c[k]] for k in ("position", "target")]
+    sc.camera = scene.make_camera(at[0], at[1], (0, 1, 0), 70, 41, fov_deg=60, near=0.1 * scale, far=100 * scale)
+    ref = oracle.render(sc, 4, 12, 3)
+    with ra.HipRenderer(max_sample_count=4, max_bounces=12, seed=3, lds_bvh=0) as r:
+        r.new_frame(sc)
+        for lds in (0, 14336, 0, 14336):
+            r.set_option("lds_bvh", lds)
+            r.render_sample(sc)
+        np.testing.assert_array_equal(r.accumulator().view(np.uint32), ref.view(np.uint32))
+        r.new_frame(sc)
+        for lds in (14336, 0, 0, 0):
+            r.set_option("lds_bvh", lds)
+            r.render_sample(sc)
+        np.testing.assert_array_equal(r.accumulator().view(np.uint32), ref.view(np.uint32))
 
 
 def _arithmetic_scene(view, scale):
