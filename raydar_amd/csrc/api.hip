@@ -236,7 +236,12 @@ rd_status refresh_job(rd_renderer *r) {
 // after a sample depends on that sample's draws, so they follow one another:
 // inside a pass of the path kernel, or in passes of one sample (all pixels)
 // of the wavefront.  The next pass continues every pixel's stream.
-rd_status render_samples(rd_renderer *r, uint32_t k) {
+//
+// `image`, if there is one, is queued with the last pass where that can be
+// (Engine::run_tickets).  One below a megabyte goes straight to pinned memory:
+// a copy with its wait would take 20 us more (a larger one is copied out by
+// several threads in parts, which need the copies' events).
+rd_status render_samples(rd_renderer *r, uint32_t k, rdh::PassImage *image) {
   const rdh::EngineOptions &o = r->eng.opt;
   if (o.vk != r->frame_vk)
     return r->fail(RD_ERR_INVALID_ARGUMENT, "\"semantics\" changed after new_frame: start a new frame");
@@ -251,6 +256,13 @@ rd_status render_samples(rd_renderer *r, uint32_t k) {
   std::string err;
   const uint64_t npix = (uint64_t)r->W * r->H;
   std::vector<rdh::DevJob> host_jobs{r->job_h};
+  image->rgba = r->rgba_d;
+  image->samples = (float)(r->sample_count + k);
+  if (4 * npix < rdh::HostTransfer::kDirect) {
+    unsigned char *p = nullptr;
+    if (!r->eng.check(r->eng.transfer().direct(&p), "hipHostMalloc(image)", &err)) return device_fail(r, err);
+    image->rgba = reinterpret_cast<uchar4 *>(p);
+  }
   uint32_t done = 0;
   while (done < k) {
     uint64_t fit = r->eng.opt.l_capacity / npix;
@@ -269,18 +281,49 @@ rd_status render_samples(rd_renderer *r, uint32_t k) {
     t.spp = spp;
     t.paths = (uint32_t)(spp * npix);
     r->eng.hit_frame = r->frame_serial;
-    if (!r->eng.run_tickets(r->scene.job, {t}, host_jobs, &err)) return device_fail(r, err);
+    if (!r->eng.run_tickets(r->scene.job, {t}, host_jobs, &err, done + spp == k ? image : nullptr))
+      return device_fail(r, err);
     done += spp;
   }
   return RD_OK;
 }
 
 // print_frame_buffer (cpu.rs:221-230) on the device, then copy out.  The `k`
-// samples that render_samples just queued are waited for and counted; the
-// tonemap is queued behind them, and the timers end before it.
-rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba) {
+// samples that render_samples just queued are waited for and counted, and the
+// timers end before the copy (and the tonemap, if it was not part of the pass).
+rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba, const rdh::PassImage &image) {
   std::string err;
   const uint64_t npix = (uint64_t)r->W * r->H;
+  auto counted = [&] {
+    if (!k) return;
+    r->sample_count += k;
+    if (r->sample_count == r->cfg.max_sample_count) {
+      r->render_timer.end();
+      r->frame_timer.end();
+    }
+    r->sample_timer.end_multiple(k);
+  };
+  if (image.queued && image.rgba != r->rgba_d) {
+    if (!r->eng.check(hipStreamSynchronize(r->eng.stream), "render", &err)) return device_fail(r, err);
+    counted();
+    std::memcpy(rgba, image.rgba, 4 * npix);
+    return RD_OK;
+  }
+  if (image.queued) {
+    // An event tells when the pass has ended while the copies run on.  Behind
+    // several pipes they are queued once it has: queued before, they started
+    // 2 ms late (183 objects at 4K, 8 spp 8.9 ms, so 7.0).
+    if (!r->eng.check(hipEventRecord(r->rendered, r->eng.stream), "hipEventRecord", &err) ||
+        (r->eng.pipes_used > 1 && !r->eng.check(hipEventSynchronize(r->rendered), "render", &err)))
+      return device_fail(r, err);
+    const rdh::HostTransfer::Read read{rgba, r->rgba_d, 4 * npix};
+    const hipError_t e = r->eng.transfer().read(&read, 1, r->eng.stream, r->eng.device, [&] {
+      const hipError_t w = hipEventSynchronize(r->rendered);
+      if (w == hipSuccess) counted();
+      return w;
+    });
+    return r->eng.check(e, "read image", &err) ? RD_OK : device_fail(r, err);
+  }
   const int grid = (int)std::min<uint64_t>((npix + 255) / 256, 8192);
   // An event tells when the passes have ended while the tonemap runs on; for
   // images below a megabyte it costs more (20 us) than the gap it fills.
@@ -295,14 +338,7 @@ rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba) {
   if (!r->eng.check(e, "tonemap", &err) ||
       (ahead && !r->eng.check(hipEventSynchronize(r->rendered), "render", &err)))
     return device_fail(r, err);
-  if (k) {
-    r->sample_count += k;
-    if (r->sample_count == r->cfg.max_sample_count) {
-      r->render_timer.end();
-      r->frame_timer.end();
-    }
-    r->sample_timer.end_multiple(k);
-  }
+  counted();
   if (!r->eng.read(rgba, r->rgba_d, 4 * npix, "read image", &err)) return device_fail(r, err);
   return RD_OK;
 }
@@ -422,9 +458,10 @@ rd_status rd_render_sample(rd_renderer *r, const rd_scene *scene, uint8_t *rgba,
   // the Vulkan renderer renders every sample in one dispatch (vulkan.rs:109-184)
   const uint32_t k = r->frame_vk ? r->cfg.max_sample_count - r->sample_count
                                  : std::min(r->samples_per_pass, r->cfg.max_sample_count - r->sample_count);
-  rd_status st = render_samples(r, k);
+  rdh::PassImage image;
+  rd_status st = render_samples(r, k, &image);
   if (st != RD_OK) return st;
-  st = finish_image(r, k, rgba);
+  st = finish_image(r, k, rgba, image);
   if (st != RD_OK) return st;
   *produced = 1;
   return RD_OK;
@@ -437,11 +474,12 @@ rd_status rd_render_frame(rd_renderer *r, const rd_scene *scene, uint8_t *rgba, 
   rd_status st = rd_new_frame(r, scene);
   if (st != RD_OK) return st;
   const uint32_t k = r->cfg.max_sample_count - std::min(r->sample_count, r->cfg.max_sample_count);
+  rdh::PassImage image;
   if (k) {
-    st = render_samples(r, k);
+    st = render_samples(r, k, &image);
     if (st != RD_OK) return st;
   }
-  return finish_image(r, k, rgba);
+  return finish_image(r, k, rgba, image);
 }
 
 rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t *rgba,
@@ -588,6 +626,9 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   // as many samples as the radiance slots hold, in sample order
   const std::vector<rdh::DevJob> host_jobs{job};
   const uint32_t total = r->cfg.max_sample_count;
+  rdh::PassImage image;
+  image.rgba = img;
+  image.samples = (float)total;
   rdh::DevTicket probe{};
   probe.spp = 1;
   if (se.takes_paths(job, probe)) {
@@ -610,15 +651,17 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
       t.spp = (uint32_t)std::min<uint64_t>(total - done, fit);
       t.paths = (uint32_t)(t.spp * npix);
       se.hit_frame = 1;  // (the binding holds no earlier frame's hits)
-      ok = se.run_tickets(d_job, {t}, host_jobs, &err);
+      rdh::PassImage *last = done + t.spp == total ? &image : nullptr;
+      ok = se.run_tickets(d_job, {t}, host_jobs, &err, last);
       done += t.spp;
     }
   }
   const int grid = (int)std::min<uint64_t>((npix + 255) / 256, 8192);
   ok = ok &&
-       se.check(rdh::launch_tonemap(d_job, (uint32_t)npix, (float)(ok ? total : 0), img, eb.counters,
-                                    false, grid, st),
-                "tonemap", &err) &&
+       (image.queued ||
+        se.check(rdh::launch_tonemap(d_job, (uint32_t)npix, (float)(ok ? total : 0), img, eb.counters,
+                                     false, grid, st),
+                 "tonemap", &err)) &&
        se.read(rgba, img, 4 * npix, "read image", &err);
   std::string sync_err;
   const bool synced = se.check(hipStreamSynchronize(st), "render", &sync_err);

@@ -630,7 +630,7 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
 }
 
 bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
-                         const std::vector<DevJob> &host_jobs, std::string *err) {
+                         const std::vector<DevJob> &host_jobs, std::string *err, PassImage *image) {
   const uint64_t frame = hit_frame;  // set by the caller for this pass only
   hit_frame = 0;
   if (tickets.empty()) return true;
@@ -657,6 +657,15 @@ bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
   }
   if (paths) {
     if (!run_paths(d_jobs, host_jobs[0], traced[0], frame, err)) return false;
+    if (image && !opt.kernel_timing) {
+      const uint32_t npix = host_jobs[0].width * host_jobs[0].height;
+      const int grid = 8 * num_cus;
+      image->queued = true;
+      return check(accumulated ? launch_tonemap(d_jobs, npix, image->samples, image->rgba, counters, false, grid,
+                                                stream, true)
+                               : launch_finish(d_jobs, traced[0], npix, L, image->samples, image->rgba, grid, stream),
+                   "finish", err);
+    }
   } else if (!traced.empty()) {
     // Pipes: a one-job pass is divided by samples (pipe k traces samples
     // [s_k, s_k+1) into their own radiance slots), anything else runs whole.

@@ -117,6 +117,14 @@ struct ExternalBuffers {
   uint32_t compact_nodes;
 };
 
+// The image wanted after a pass: bytes for every pixel at `rgba` (memory the
+// device writes) of `samples` samples.
+struct PassImage {
+  uchar4 *rgba = nullptr;
+  float samples = 0.0f;
+  bool queued = false;  // the pass has queued it
+};
+
 class Engine {
  public:
   ~Engine();
@@ -153,8 +161,11 @@ class Engine {
   // writing this engine's radiance arena.  The pipes' kernels run
   // concurrently, so one pipe's closest-hit work (ALU-bound) overlaps
   // another's shading (memory-bound).
+  //
+  // With `image`, a pass of the path kernel queues its image too.
   bool run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
-                   const std::vector<DevJob> &host_jobs, std::string *err);
+                   const std::vector<DevJob> &host_jobs, std::string *err,
+                   PassImage *image = nullptr);
 
   // Whether the path kernel renders this pass.
   bool takes_paths(const DevJob &j, const DevTicket &t) const;

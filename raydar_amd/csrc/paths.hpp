@@ -62,5 +62,10 @@ __attribute__((weak)) int path_blocks_per_cu(const PathArgs &a, bool record);
 __attribute__((weak)) hipError_t launch_paths(const PathArgs &a, bool record, int grid,
                                               hipStream_t st);
 __attribute__((weak)) hipError_t launch_compact(const PathArgs &a, hipStream_t st);
+// Adds the radiance slots of `t` to the accumulator and writes the image bytes
+// of the `samples` samples it then holds, for npix pixels; npix > 0.
+__attribute__((weak)) hipError_t launch_finish(const DevJob *job, const DevTicket &t, uint32_t npix,
+                                               const float4 *L, float samples, uchar4 *rgba,
+                                               int max_grid, hipStream_t st);
 
 }  // namespace rdh

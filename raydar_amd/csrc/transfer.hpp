@@ -8,6 +8,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
+#include <functional>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -98,8 +99,19 @@ class HostTransfer {
     return upload(dst, &p, 1, stream);
   }
 
+  // Pinned memory of kDirect bytes for the device to write by itself: valid
+  // until the next read.
+  static constexpr uint64_t kDirect = 1u << 20;
+  hipError_t direct(unsigned char **p) {
+    const hipError_t e = reserve();
+    *p = ring_;
+    return e;
+  }
+
   // Waits for the stream's work so far and copies the reads' bytes to the host.
-  hipError_t read(const Read *reads, int n, hipStream_t stream, int device) {
+  // `queued`, if there is one, is called once the first copies are queued.
+  hipError_t read(const Read *reads, int n, hipStream_t stream, int device,
+                  const std::function<hipError_t()> &queued = nullptr) {
     std::vector<Read> chunks;
     uint64_t total = 0;
     for (int k = 0; k < n; ++k) {
@@ -117,6 +129,7 @@ class HostTransfer {
     if (count <= slots && total < kThreaded) {
       for (size_t i = 0; i < count && e == hipSuccess; ++i)
         e = hipMemcpyAsync(ring_ + i * kSlot, chunks[i].src, chunks[i].bytes, hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess && queued) e = queued();
       const hipError_t s = hipStreamSynchronize(stream);
       if (e != hipSuccess || s != hipSuccess) return e != hipSuccess ? e : s;
       for (size_t i = 0; i < count; ++i) std::memcpy(chunks[i].dst, ring_ + i * kSlot, chunks[i].bytes);
@@ -168,6 +181,7 @@ class HostTransfer {
       }
     };
     for (size_t i = 0; i < slots; ++i) issue(i);
+    if (queued && (e = queued()) != hipSuccess) failed.store(e);
     std::vector<std::thread> helpers;
     try {
       helpers.reserve(kHelpers);
@@ -192,7 +206,7 @@ class HostTransfer {
   static constexpr uint64_t kMinUpload = 256u << 10, kMaxUpload = 4u << 20;
   static constexpr uint64_t kSlot = 2u << 20;      // a copy of the ring
   static constexpr uint64_t kPart = 256u << 10;    // what a thread takes of it
-  static constexpr uint64_t kThreaded = 1u << 20;  // reads of one thread, and bytes per further one
+  static constexpr uint64_t kThreaded = kDirect;  // reads of one thread, and bytes per further one
   static constexpr size_t kSlots = 4, kHelpers = 3;
 
   hipError_t grow_upload(uint64_t bytes) {

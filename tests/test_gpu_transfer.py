@@ -36,3 +36,27 @@ def test_scenes_of_growing_size_through_one_renderer():
             r.render_frame(sc)
             ref = oracle.render(sc, 1, 4, 3)
             np.testing.assert_array_equal(r.accumulator().view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("semantics", [0, 1])
+@pytest.mark.parametrize("width,height,per_pass", [
+    (1, 1, 2), (511, 512, 2), (512, 512, 1), (513, 512, 2)])  # images written by the device below 1 MiB
+def test_image_of_every_pass_around_the_direct_limit(width, height, per_pass, semantics):
+    sc = scenegen.plain_1080p(1, width, height)
+    spp = 4
+    with ra.HipRenderer(max_sample_count=spp, max_bounces=3, seed=5, semantics=semantics,
+                        l_capacity=max(1 << 16, width * height)) as r:  # a pass holds one sample
+        r.set_samples_per_pass(per_pass)
+        r.new_frame(sc)
+        step = spp if semantics else per_pass
+        for done in range(step, spp + 1, step):
+            img = r.render_sample()
+            if semantics:
+                ref = oracle.vk_render(sc, ra.camera_vulkan_inverse_view(sc.camera), done, 3, threads=8)
+                want = oracle.vk_tonemap(ref, done)
+            else:
+                ref = oracle.render(sc, done, 3, 5, threads=8)
+                want = oracle.tonemap(ref, done)
+            np.testing.assert_array_equal(r.accumulator().view(np.uint32), ref.view(np.uint32))
+            np.testing.assert_array_equal(img.reshape(-1), want)
+            assert r.sample_count == done
