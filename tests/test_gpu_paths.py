@@ -187,3 +187,16 @@ def test_path_kernel_vulkan_semantics_match_oracle(size, spp, bounces, opts):
     ref = oracle.vk_render(sc, ra.camera_vulkan_inverse_view(sc.camera), spp, bounces, threads=8)
     np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
     np.testing.assert_array_equal(img.reshape(-1), oracle.vk_tonemap(ref, spp))
+
+
+@pytest.mark.parametrize("objects", range(1, 10))
+def test_nodes_with_each_number_of_leaves(objects):
+    # a root of one to four leaves with empty slots, then leaves beside inner
+    # children, spheres and cubes in one wave, entered in every combination
+    sc = scenegen.plain_1080p(4, 77, 50)
+    sc.objects = sc.objects[[0, 65, 1, 66, 2, 67, 3, 68, 4][:objects]]
+    with ra.HipRenderer(max_sample_count=4, max_bounces=12, seed=3) as r:
+        r.render_frame(sc)
+        acc = r.accumulator()
+    ref = oracle.render(sc, 4, 12, 3)
+    np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
