@@ -259,11 +259,13 @@ void k_paths(PathArgs a) {
   // The lane's stack column: rows of kRow bytes, the last holding kNoNode for
   // good, so that a pop needs no look at the depth.
   constexpr uint32_t kRow = BLOCK * (uint32_t)sizeof(StackT);
-  const uint32_t stack_first = (a.stack_rows - 2u) * kRow + threadIdx.x * (uint32_t)sizeof(StackT);
-  auto stack_at = [&](uint32_t off) -> StackT & { return *reinterpret_cast<StackT *>(dynamic_lds + off); };
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)dynamic_lds;
+  const uint32_t stack_first = lds_base + (a.stack_rows - 2u) * kRow + threadIdx.x * (uint32_t)sizeof(StackT);
+  typedef __attribute__((address_space(3))) StackT LdsStackT;
+  auto stack_at = [](uint32_t off) -> LdsStackT & { return *(LdsStackT *)off; };
   stack_at(stack_first + kRow) = (StackT)kNoNode;
   // a pooled walk's primitives entered but not yet tested: kPoolRows rows
-  const uint32_t pool_first = stack_bytes + threadIdx.x * (uint32_t)sizeof(StackT);
+  const uint32_t pool_first = lds_base + stack_bytes + threadIdx.x * (uint32_t)sizeof(StackT);
   VecF4 *lds_nodes = reinterpret_cast<VecF4 *>(dynamic_lds + stack_bytes + (kPooled ? pool_bytes<BLOCK>() : 0u));
   const uint32_t node_vecs = LDS ? 8 * n_nodes4 : 0u, prim_vecs = LDS ? 2 * n_prims : 0u;
   VecF4 *lds_prims = lds_nodes + node_vecs;
@@ -375,6 +377,17 @@ void k_paths(PathArgs a) {
       load_prim(prims, j, &pr);
     }
     test_in_walk<VK>(r, ya, nf.ix, nf.iy, nf.iz, pr, &best);
+  };
+  // off, a row further if key's sign bit is set: a shift and a shift-add (as
+  // one expression the compiler makes it three instructions; with stack
+  // addresses kept absolute and one comparison less a step 97 objects at 1080p,
+  // 64 spp 10.30 -> 10.07 ms, 4096 objects 14.05 -> 13.37)
+  auto row_if = [](uint32_t key, uint32_t off) {
+    uint32_t bit = key >> 31;
+    asm("" : "+v"(bit));
+    off += bit * kRow;
+    asm("" : "+v"(off));
+    return off;
   };
   // the primitive of a one-primitive leaf (in LDS and compact trees the code's
   // lower half)
@@ -564,7 +577,7 @@ void k_paths(PathArgs a) {
       } else {
         if ((uint32_t)__popcll(at_nodes) <= keep) break;
       }
-      if (node != kNoNode) {
+      if (__builtin_amdgcn_inverse_ballot_w64(at_nodes)) {
 #ifdef RDH_CHECKED
         node = chk(node, n_nodes4, K_NODE, a.ctl);
 #endif
@@ -658,13 +671,13 @@ void k_paths(PathArgs a) {
           // the entered leaves' primitives go above the lane's others; a key
           // plus one has the sign bit set for a leaf's alone
           stack_at(pool) = leaf_prim(ch.x);
-          pool += ((e0 + 1u) >> 31) * kRow;
+          pool = row_if(e0 + 1u, pool);
           stack_at(pool) = leaf_prim(ch.y);
-          pool += ((e1 + 1u) >> 31) * kRow;
+          pool = row_if(e1 + 1u, pool);
           stack_at(pool) = leaf_prim(ch.z);
-          pool += ((e2 + 1u) >> 31) * kRow;
+          pool = row_if(e2 + 1u, pool);
           stack_at(pool) = leaf_prim(ch.w);
-          pool += ((e3 + 1u) >> 31) * kRow;
+          pool = row_if(e3 + 1u, pool);
         }
         const uint32_t lo = umin(umin(e0, e1), e2), mid = umed3(e0, e1, e2), hi = umax(umax(e0, e1), e2);
         const uint32_t r0 = umin(lo, e3), r1 = umed3(lo, mid, e3);
@@ -674,17 +687,17 @@ void k_paths(PathArgs a) {
         // next one put over it.  The nearest is next, or the top of the stack
         // (kNoNode above the first).
 #ifdef RDH_CHECKED
-        if (chk(sp, stack_bytes - 2u * kRow, K_STACK, a.ctl) == 0u) sp = stack_first - 2u * kRow;
+        if (chk(sp - lds_base, stack_bytes - 2u * kRow, K_STACK, a.ctl) == 0u) sp = stack_first - 2u * kRow;
 #endif
         stack_at(sp + 2u * kRow) = (StackT)r3;
-        sp += (r3 >> 31) * kRow;
+        sp = row_if(r3, sp);
         stack_at(sp + kRow) = (StackT)r2;
-        sp += (r2 >> 31) * kRow;
+        sp = row_if(r2, sp);
         stack_at(sp) = (StackT)r1;
-        sp += (r1 >> 31) * kRow;
+        sp = row_if(r1, sp);
         const uint32_t popped = stack_at(sp);
         node = (int32_t)r0 < 0 ? popped : r0 & 0xffffu;
-        sp += (r0 >> 31) * kRow - 3u * kRow;
+        sp = row_if(r0, sp) - 3u * kRow;
         if constexpr (LDS && LEAF1) {
           // the entered leaves' bits, and a primitive a trip: its half word of
           // the codes is picked by a byte permutation (selecting it by three
