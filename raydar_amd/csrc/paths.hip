@@ -687,7 +687,8 @@ void k_paths(PathArgs a) {
         // next one put over it.  The nearest is next, or the top of the stack
         // (kNoNode above the first).
 #ifdef RDH_CHECKED
-        if (chk(sp - lds_base, stack_bytes - 2u * kRow, K_STACK, a.ctl) == 0u) sp = stack_first - 2u * kRow;
+        // (one up: the first row of lane 0 is at 0, as is what chk puts in place)
+        if (chk(sp - lds_base + 1u, stack_bytes - 2u * kRow + 1u, K_STACK, a.ctl) == 0u) sp = stack_first - 2u * kRow;
 #endif
         stack_at(sp + 2u * kRow) = (StackT)r3;
         sp = row_if(r3, sp);
