@@ -469,7 +469,7 @@ def main():
             "workload": f"{args.workload}: {sc.width}x{sc.height}, {job.spp} spp, {job.bounces} bounces, "
                         f"{len(sc.objects)} objects, seed {job.seed}",
             "paths_per_step": paths_per_step,
-            "renderer": "plain per-scene HIP renderer (wavefront: generate/extend/shade, SAH BVH)",
+            "renderer": "plain per-scene HIP renderer (whole paths in one kernel, SAH BVH)",
             "options": {k: r.get_option(k) for k in ("block", "queue", "leaf", "grid", "traversal",
                                                       "bvh4", "pipes")},
             "pipes_used": pipes_used,
@@ -483,7 +483,8 @@ def main():
             "bound": "fp32_valu",
             "compute": "FP32 vector ALU (this path has no dense contraction and uses no MFMA); "
                        "peak is MI355X FP32 157.3 TFLOP/s",
-            "kernel": "extend (closest hit: BVH traversal + exact sphere/cube tests)",
+            "kernel": "paths (closest hit: BVH traversal + exact sphere/cube tests, whose "
+                      "operations are counted; and shading, whose are not)",
             "achieved": round(achieved, 4),
             "peak": PEAK_FP32_TFLOPS,
             "unit": "TFLOP/s",
