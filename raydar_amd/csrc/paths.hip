@@ -763,8 +763,10 @@ const void *paths_fn_of(PathTree tree, bool record) {
     case kTreeMemory:
       return record ? (const void *)k_paths<kPathBlock, true, kTreeMemory, VK>
                     : (const void *)k_paths<kPathBlock, false, kTreeMemory, VK>;
-    case kTreeCompact:  // camera rays share their nodes: recorded from the tree itself
-      if (!record) return (const void *)k_paths<kPathBlock, false, kTreeCompact, VK>;
+    case kTreeCompact:  // (not with Vulkan semantics: plan_paths)
+      // camera rays share their nodes: recorded from the tree itself
+      if constexpr (!VK)
+        if (!record) return (const void *)k_paths<kPathBlock, false, kTreeCompact, VK>;
       [[fallthrough]];
     case kTreeLeaf1:
       return record ? (const void *)k_paths<kPathBlock, true, kTreeLeaf1, VK>
@@ -797,14 +799,20 @@ uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
 // were slower than the walk in memory: 640 threads 300 objects 1.33 -> 1.45 ms,
 // 500 objects 1.46 -> 1.69 (1280x720, 16 spp, whole call).
 //
-// A larger tree of one-primitive leaves is walked as DevNode4C from 1280 nodes
-// (160 KB of DevNode4) on: four 16-byte loads a node instead of seven, which
-// counts once the node fetches miss the L1, but a third more instructions.
-// 1280x720, 32 spp, full -> compact: 1000 objects (458 nodes) 1.87 -> 1.91 ms,
-// 1500 2.23 -> 2.32, 2500 3.13 -> 3.15, 4096 (1777 nodes) 4.52 -> 4.40, 8000
-// 7.19 -> 6.71.
+// A larger tree of one-primitive leaves is walked as DevNode4C, four 16-byte
+// loads a node instead of seven, where that outweighs a third more instructions:
+// in a large tree, whose node fetches miss the L1, and in a long pass, whose
+// rate counts and not the latency of its last paths.  1280x720, 16 spp, full ->
+// compact: 1000 objects (455 nodes) 1.03 -> 1.04 ms, 1400 (621) 1.24 -> 1.23,
+// 2000 1.56 -> 1.50, 2400 1.78 -> 1.66, 4096 (1777) 2.63 -> 2.26, 8000 4.62 ->
+// 4.01; 1080p, 2 spp: 2400 1.06 -> 1.10, 4096 1.28 -> 1.33, 8000 1.71 -> 1.73,
+// 14000 2.07 -> 1.97: the line is nodes times paths.  With Vulkan semantics
+// (four waves per SIMD, more registers) the full nodes are faster at every
+// size: 2400 2.48 against 2.26, 4096 2.92 and 2.56, 14000 5.55 and 5.28.
 void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh, uint64_t lds_objects) {
-  constexpr uint32_t kCompactNodes = 1280;
+  constexpr uint64_t kCompactNodes = 768, kCompactWork = 14ull << 30;
+  const bool compact = !a->vk && j.n_nodes4 >= kCompactNodes &&
+                       (uint64_t)a->npix * a->samples * j.n_nodes4 >= kCompactWork;
   a->stack_rows = j.stack4 + 4;  // a sentinel below, and three written above the top
   const bool leaf1 = j.max_leaf == 1;
   const uint64_t blocks = 4 * path_waves(false, a->vk) / (kPathBlock / 64);
@@ -813,7 +821,7 @@ void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh, uint64_t lds_obj
   const uint64_t objects = sizeof(DevObject) * (uint64_t)j.n_prims;
   const bool lds = tree <= lds_bvh && stack + tree <= room;
   a->tree = lds ? (leaf1 ? kTreeLdsLeaf1 : kTreeLds)
-                : !leaf1 ? kTreeMemory : j.n_nodes4 >= kCompactNodes ? kTreeCompact : kTreeLeaf1;
+                : !leaf1 ? kTreeMemory : compact ? kTreeCompact : kTreeLeaf1;
   a->lds_bvh_bytes = lds ? (uint32_t)tree : 0u;
   const uint64_t used = stack + (lds ? tree : pool_bytes<kPathBlock>());
   a->lds_obj_bytes = objects <= lds_objects && used + objects <= room ? (uint32_t)objects : 0u;

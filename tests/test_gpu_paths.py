@@ -200,3 +200,22 @@ def test_nodes_with_each_number_of_leaves(objects):
         acc = r.accumulator()
     ref = oracle.render(sc, 4, 12, 3)
     np.testing.assert_array_equal(acc.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("height,scale,shift", [
+    (960, 1.0, 0.0), (640, 1.0, 0.0),  # on both sides of where half-size nodes are used
+    (960, 2.0 ** -40, 0.0), (960, 2.0 ** 12, 0.0), (960, 1.0, 4096.0), (960, 2.0 ** -12, 1.0), (960, 2.0 ** 40, 0.0)])
+def test_large_tree_and_long_pass_at_every_scale(height, scale, shift):
+    sc = scenegen.clustered(6, 14000, 1536, height)
+    sc.objects["center"] = sc.objects["center"] * np.float32(scale) + np.float32(shift)
+    sc.objects["size"] *= np.float32(scale)
+    c = sc.camera
+    at = [[float(np.float32(v * scale + shift)) for v in c[k]] for k in ("position", "target")]
+    sc.camera = scene.make_camera(at[0], at[1], (0, 1, 0), 1536, height, fov_deg=60, near=0.1 * scale,
+                                  far=100 * scale)
+    with ra.HipRenderer(max_sample_count=2, max_bounces=4, seed=3) as r:
+        r.render_frame(sc)
+        acc = r.accumulator()
+    pix = np.arange(0, 1536 * height, 1999, dtype=np.uint32)
+    ref = oracle.render(sc, 2, 4, 3, pixels=pix, threads=8)
+    np.testing.assert_array_equal(acc[pix].view(np.uint32), ref.view(np.uint32))
