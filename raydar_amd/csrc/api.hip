@@ -603,6 +603,7 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   ds.max_leaf = b.max_leaf;
   ds.n_prims = (uint32_t)b.prims.size();
   ds.r0 = b.r0;
+  ds.reach = b.reach;
   ds.depth = b.depth;
   float *acc = reinterpret_cast<float *>(base + o_acc);
   uchar4 *img = reinterpret_cast<uchar4 *>(base + o_img);
@@ -874,6 +875,7 @@ rd_status debug_setup(const rd_scene *scene, int leaf, DebugCtx *c) {
   ds.n_nodes = (uint32_t)b.nodes.size();
   ds.n_prims = (uint32_t)b.prims.size();
   ds.r0 = b.r0;
+  ds.reach = b.reach;
   rdh::DevJob j;
   rdh::fill_job(*scene, ds, nullptr, 0, 0, &j);
   c->job = nullptr;
@@ -973,6 +975,7 @@ rd_status rd_debug_extend(const rd_scene *scene, int leaf, const rd_extend_varia
     ds.stack4 = b.stack4;
     ds.n_prims = (uint32_t)b.prims.size();
     ds.r0 = b.r0;
+    ds.reach = b.reach;
     ds.depth = b.depth;
     if ((!b.nodes.empty() && !ds.nodes) || (!b.prims.empty() && !ds.prims) || (n4 && !ds.nodes4))
       return RD_ERR_OUT_OF_MEMORY;

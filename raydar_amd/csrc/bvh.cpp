@@ -7,7 +7,10 @@
 // and the hit point it reports lies within that distance of the sphere.  Such
 // "phantom" hits are part of the reference's answer, so every primitive box is
 // grown by twice that excess (2e-6 L^2 inside the square root) for every ray
-// origin with |o|_1 <= r0, plus 1e-6 L for the box test's own rounding.  Rays
+// origin with |o|_1 <= r0, plus 1e-6 L (17u L) for the box test's own rounding:
+// u|o| each for o -+ margin and its product with 1/d, u|p - o| each for 1/d and
+// a plane p's final fma, and u|q - o| for the inner fma of a half-size node with
+// origin q (DevNode4C, whose planes are rounded outward by k_compact).  Rays
 // starting beyond r0 (only possible after hitting a primitive larger than the
 // rest of the scene, e.g. a ground sphere's far side) add a per-ray margin of
 // 2e-3 |o|_1 at traversal time (ray_tolerance in pathmath.hpp).  The CPU tests
@@ -408,6 +411,7 @@ bool build_scene(const rd_scene &scene, int leaf_size, BuiltScene *out, std::str
     if (std::fabs((double)o.size) <= 0.25 * r_all) r_small = std::max(r_small, ext);
   }
   out->r0 = (float)r_small;
+  out->reach = (float)r_all;
 
   Builder bld;
   bld.leaf_size = leaf_size;

@@ -26,6 +26,7 @@ struct BuiltScene {
   std::vector<DevObject> objects;  // original order
   uint32_t depth = 0;              // max node depth (root = 1)
   float r0 = 0.f;                  // |o|_1 bound covered by the static padding
+  float reach = 0.f;               // no primitive or camera lies farther from 0 on any axis
   double sah_cost = 0.0;
 };
 

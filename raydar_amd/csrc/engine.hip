@@ -314,6 +314,7 @@ bool Engine::alloc_scene(const BuiltScene &b, DeviceScene *out, std::string *err
   out->max_leaf = b.max_leaf;
   out->n_prims = (uint32_t)b.prims.size();
   out->r0 = b.r0;
+  out->reach = b.reach;
   out->depth = b.depth;
   HostTransfer::Piece p[5];
   const uint64_t total = scene_pieces(b, nullptr, p);
@@ -954,6 +955,7 @@ void fill_job(const rd_scene &s, const DeviceScene &ds, float *acc, uint32_t max
     j->solid[k] = s.world.solid_color[k];
   }
   j->r0_tol = ds.r0;
+  j->reach = ds.reach;
   j->depth = ds.depth;
   j->nodes4 = ds.nodes4;
   j->n_nodes4 = ds.n_nodes4;

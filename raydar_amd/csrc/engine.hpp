@@ -36,7 +36,7 @@ struct DeviceScene {
   DevPrim *prims = nullptr;
   DevObject *objects = nullptr;
   uint32_t n_nodes = 0, n_prims = 0;
-  float r0 = 0.f;
+  float r0 = 0.f, reach = 0.f;
   uint32_t depth = 0;
   size_t bytes = 0;
 };

@@ -128,6 +128,7 @@ struct DevJob {
   uint32_t n_nodes4;        // the same tree as 4-wide nodes
   uint32_t stack4;          // stack entries a 4-wide traversal can hold
   uint32_t max_leaf;        // primitives in the largest leaf (1: one per leaf)
+  float reach;              // BuiltScene::reach
   const DevNode4 *nodes4;
   uint32_t *vk_rng;         // Vulkan semantics: each pixel's PCG state between passes
   HitWord *first_hit;       // several jobs: each pixel's camera-ray hit, all zero until

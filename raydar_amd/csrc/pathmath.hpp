@@ -284,33 +284,42 @@ RD_HD void test_prim(const RayPre &r, const DevPrim &p, float *bt, uint32_t *bid
 // expand the box by `tol` on every side: entry = max over axes of
 // min(lo*inv - A, hi*inv - B), exit = min of the max; clamped at t = 0.
 struct SlabRay {
-  float ix, iy, iz;     // 1 / d with |d_i| clamped away from 0 (finite)
+  float ix, iy, iz;     // 1 / d with |d_i| clamped away from 0
   float ax, ay, az;     // (o + tol) * inv
   float bx, by, bz;     // (o - tol) * inv
 };
 // On the GPU the reciprocal is rcp_rn's fast form, the rounded one for every
-// |d| in [2^-60, 2^60); outside that it may be off by an ulp, which the
+// |d| in [2^-60, 2^60); above that it may be off by an ulp, which the
 // rounding margin every box carries (1e-6 L, the padding note of bvh.cpp)
 // covers.
+//
+// A component below 2^-60, zero too, counts as 2^-60: with |d| >= 2^-38
+// (walkable()) the ray moves by less than that margin along such an axis on
+// its way through the scene, so it is inside the axis's planes from end to end
+// or outside, and a margin's worth of distance times 2^60 lies beyond any
+// hit's.  The clamp is no smaller because the walk's products must stay
+// finite: with walkable()'s |o_i| < 2^64 a plane's fma then takes a finite
+// subtrahend and rounds, or overflows, to the side it lies on.  (With 1e-30
+// the subtrahend was infinite from |o_i| = 3.4e8 on, a half-size node's factor
+// from nodes of 5e8, and hits were lost.)
+constexpr float kMinSlabDir = 0x1p-60f;
 RD_HD float safe_inv(float d) {
-  const float m = fabsf(d) < 1e-30f ? copysignf(1e-30f, d) : d;
+  const float m = fabsf(d) < kMinSlabDir ? copysignf(kMinSlabDir, d) : d;
 #if defined(__HIP_DEVICE_COMPILE__)
   return rcp_rn_normal(m);
 #else
   return 1.0f / m;
 #endif
 }
-// Whether the box walk answers exactly as the scan would: finite origin and
-// direction, and no direction component that safe_inv would clamp unless it
-// is an exact zero next to a nonzero component (an axis-parallel ray, whose
-// slabs safe_inv scales correctly).  An all-zero direction or a tiny nonzero
-// component makes the reference's divisions by d (cpu.rs:74-79) overflow
-// differently from the clamped scale; such rays take the linear scan.
+// Whether the box walk answers exactly as the scan would: an origin and a
+// direction whose squares are finite (|o_i|, |d_i| < 2^64), a direction that
+// safe_inv's clamp is small against, and no tiny nonzero component: there the
+// reference's divisions by d (cpu.rs:74-79) overflow differently from the
+// clamped scale.  Other rays take the linear scan.
 RD_HD bool tiny_nonzero(float d) { return d != 0.0f && fabsf(d) < 1e-30f; }
 RD_HD bool walkable(const RayPre &r) {
-  return isfinite(r.ox) && isfinite(r.oy) && isfinite(r.oz) && isfinite(r.dx) && isfinite(r.dy) &&
-         isfinite(r.dz) && !(r.dx == 0.0f && r.dy == 0.0f && r.dz == 0.0f) &&
-         !tiny_nonzero(r.dx) && !tiny_nonzero(r.dy) && !tiny_nonzero(r.dz);
+  return r.oo < INFINITY && r.a >= 0x1p-76f && r.a < INFINITY && !tiny_nonzero(r.dx) &&
+         !tiny_nonzero(r.dy) && !tiny_nonzero(r.dz);
 }
 RD_HD SlabRay slab_ray(const RayPre &r, float tol) {
   SlabRay s;

@@ -200,7 +200,7 @@ __global__ __launch_bounds__(64) void k_compact(const DevJob *job, DevNode4C *ou
       }
     // any origin will do; this one is near the middle
     origin[x] = bitsf(fbits(0.5f * a + 0.5f * b) & 0xffff0000u);
-    // for the subtractions below and the walk's inner rounding
+    // for the subtractions below
     slack[x] = 0x1p-21f * (fabsf(a) + fabsf(b));
     reach = fmaxf(reach, fmaxf(fabsf(a - origin[x]), fabsf(b - origin[x])) + slack[x]);
   };
@@ -589,9 +589,9 @@ void k_paths(PathArgs a) {
         if constexpr (kCompact) {
           // DevNode4C: a plane's distance is (origin + h * unit) * i - n, as
           // fma(h, unit * i, fma(origin, i, -n)) with an exact first product
-          // (unit is a power of two); the inner one rounds by 2^-24 of the
-          // origin's distance, which the margin of k_compact covers.  A NaN from
-          // overflow drops its axis from the test.
+          // (unit is a power of two, and the product finite: plan_paths); the
+          // inner one rounds by 2^-24 of the node origin's distance from the
+          // ray's, which the 1e-6 L of every primitive's box covers (bvh.cpp).
           const __attribute__((address_space(1))) unsigned char *gb =
               (const __attribute__((address_space(1))) unsigned char *)a.compact;
           const uint32_t nb = node * (uint32_t)sizeof(DevNode4C);
@@ -809,10 +809,12 @@ uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
 // 4.01; 1080p, 2 spp: 2400 1.06 -> 1.10, 4096 1.28 -> 1.33, 8000 1.71 -> 1.73,
 // 14000 2.07 -> 1.97: the line is nodes times paths.  With Vulkan semantics
 // (four waves per SIMD, more registers) the full nodes are faster at every
-// size: 2400 2.48 against 2.26, 4096 2.92 and 2.56, 14000 5.55 and 5.28.
+// size: 2400 2.48 against 2.26, 4096 2.92 and 2.56, 14000 5.55 and 5.28.  Nor for
+// scenes beyond 2^62, where a node's unit times 1/d (at most 2^60) could overflow.
 void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh, uint64_t lds_objects) {
   constexpr uint64_t kCompactNodes = 768, kCompactWork = 14ull << 30;
-  const bool compact = !a->vk && j.n_nodes4 >= kCompactNodes &&
+  constexpr float kCompactReach = 0x1p62f;
+  const bool compact = !a->vk && j.n_nodes4 >= kCompactNodes && j.reach <= kCompactReach &&
                        (uint64_t)a->npix * a->samples * j.n_nodes4 >= kCompactWork;
   a->stack_rows = j.stack4 + 4;  // a sentinel below, and three written above the top
   const bool leaf1 = j.max_leaf == 1;
