@@ -1,0 +1,30 @@
+"""The library's host code on the fake HIP device with the path kernel among the
+fake kernels (tests/fakehip/fake_paths.cpp): the route nearly every scene takes
+on a GPU (run_paths, its camera-hit tables, half-size trees and work lists, the
+streams it is spread over, the batch's passes launched as they are issued, the
+image queued with its pass), under AddressSanitizer + UndefinedBehaviorSanitizer
+and ThreadSanitizer.  test_fake_device.py runs the wavefront throughout."""
+import pytest
+
+from tests.test_fake_device import _build, _run
+
+
+@pytest.fixture(scope="module")
+def asan(tmp_path_factory):
+    return _build(str(tmp_path_factory.mktemp("fakepaths")), "paths_asan")
+
+
+@pytest.fixture(scope="module")
+def tsan(tmp_path_factory):
+    return _build(str(tmp_path_factory.mktemp("fakepaths_tsan")), "paths_tsan")
+
+
+@pytest.mark.parametrize("args,nosync", [(["path_frames"], "1"), (["plain"], "0"), (["noalloc"], "1"),
+                                         (["batch"], "0")])
+def test_path_kernel_host_code_asan(asan, args, nosync):
+    _run(asan, args, 900, FAKEHIP_FREE_NOSYNC=nosync)
+
+
+@pytest.mark.parametrize("args", [["path_frames"], ["plain"]])
+def test_path_kernel_host_code_tsan(tsan, args):
+    _run(tsan, args, 900)
