@@ -73,7 +73,8 @@ struct SJob {
   float *out_acc = nullptr;
   uint8_t *progress = nullptr;
   uint64_t bytes = 0;
-  uint64_t path_frame = 0;         // nonzero: traced by the path kernel (Engine::run_paths' frame)
+  bool paths = false;              // traced by the path kernel, which keeps in `space`
+  PathSpace space;                 // (behind the accumulator) what the job's passes share
   int state = 0;                   // 0 queued, 1 resident, 2 done, 3 failed
   int32_t status = RD_OK;
   Clock::time_point t_submit, t_admit, t_done;
@@ -303,7 +304,6 @@ class Streamer {
   uint32_t uploaded_ = 0, ticket_lo_ = 0;  // tickets issued, first not yet accumulated
   uint32_t on_device_ = 0;                 // tickets in the device table
   bool wave_running_ = false;              // the last launch() queued wavefront iterations
-  uint64_t path_frames_ = 0;               // jobs admitted to the path kernel
   uint64_t ctl_total_ = 0, last_cursor_ = 0;
   uint32_t last_count_ = 0;
   uint32_t stalls_ = 0;
@@ -327,7 +327,7 @@ class Streamer {
   }
 
   void release_job(SJob *j) {
-    if (j->state != 1 && !j->acc && !j->dev.nodes && !j->dev.prims) return;
+    if (j->state != 1 && !j->acc && !j->dev.base) return;
     eng.free_scene(&j->dev);
     eng.dfree(j->acc);
     eng.dfree(j->rgba_d);
@@ -335,12 +335,36 @@ class Streamer {
     j->rgba_d = nullptr;
   }
 
+  // Bytes of the job's accumulator and what follows it (j->space): the path
+  // kernel's camera-hit table and compact tree if it is to trace the job, else
+  // the wavefront's camera-hit table.
+  uint64_t acc_bytes(const SJob &j, uint32_t compact_nodes, bool paths) const {
+    const uint64_t npix = (uint64_t)j.W * j.H;
+    if (!paths) return (16 + sizeof(HitWord)) * npix;
+    return compact_at(npix) + sizeof(DevNode4C) * compact_nodes;
+  }
+  static uint64_t compact_at(uint64_t npix) { return ((16 + kCamBytes) * npix + 255) & ~255ull; }
+
   bool admit() {
     while (!queued_.empty()) {
       SJob *j = queued_.front();
       if (free_slots_.empty()) break;
+      // The path kernel's tables are part of what its job needs; a job that
+      // fits the budget without them alone is the wavefront's.
+      DeviceScene sizes;
+      Engine::describe_scene(j->built, &sizes);
+      DevJob dj{};
+      fill_job(j->scene, sizes, nullptr, j->bounces, j->seed, &dj);
+      DevTicket probe{};
+      probe.spp = j->pass_spp;
+      bool paths = eng.takes_paths(dj, probe);
+      const uint32_t compact = paths ? eng.compact_nodes(dj, probe) : 0u;
+      const uint64_t more = paths ? acc_bytes(*j, compact, true) - acc_bytes(*j, 0, false) : 0;
+      if (paths && !pool->fits_alone(j->bytes + more)) paths = false;
+      const uint64_t need = j->bytes + (paths ? more : 0);
       // wait for room unless nothing is resident (a job that fits alone always runs)
-      if (!pool->reserve(j->bytes)) break;
+      if (!pool->reserve(need)) break;
+      j->bytes = need;
       queued_.pop_front();
       // until the job is resident a failure gives its reservation back
       struct Unreserve {
@@ -355,19 +379,24 @@ class Streamer {
       free_slots_.pop_back();
       const uint64_t npix = (uint64_t)j->W * j->H;
       if (!eng.upload_scene(j->built, &j->dev, &err)) return false;
-      // the accumulator (16 B per pixel) is followed by the job's camera-ray
-      // hit table (8 B per pixel), zero (not recorded) like the accumulator
-      if (!eng.check(eng.dmalloc((void **)&j->acc, 24 * npix), "hipMalloc(accumulator)", &err)) return false;
+      if (!eng.check(eng.dmalloc((void **)&j->acc, acc_bytes(*j, compact, paths)), "hipMalloc(accumulator)", &err))
+        return false;
       if (!eng.check(eng.dmalloc((void **)&j->rgba_d, 4 * npix), "hipMalloc(image)", &err)) return false;
-      if (!eng.check(launch_zero_acc(j->acc, 6 * npix, eng.stream), "zero accumulator", &err)) return false;
-      DevJob &dj = h_jobs_[j->slot];
+      // the wavefront's table starts zero (not recorded) like the accumulator
+      if (!eng.check(launch_zero_acc(j->acc, (paths ? 4 : 6) * npix, eng.stream), "zero accumulator", &err))
+        return false;
       fill_job(j->scene, j->dev, j->acc, j->bounces, j->seed, &dj);
-      dj.first_hit = reinterpret_cast<HitWord *>(j->acc + 4 * npix);
-      DevTicket probe{};
-      probe.spp = j->pass_spp;
-      j->path_frame = eng.takes_paths(dj, probe) ? ++path_frames_ : 0;
+      unsigned char *behind = reinterpret_cast<unsigned char *>(j->acc);
+      if (paths)
+        j->space = PathSpace{behind + 16 * npix, npix, 0,
+                             reinterpret_cast<DevNode4C *>(behind + compact_at(npix)), compact, 0, true};
+      else
+        dj.first_hit = reinterpret_cast<HitWord *>(behind + 16 * npix);
+      j->paths = paths;
+      h_jobs_[j->slot] = dj;
       if (!eng.upload(d_jobs_ + j->slot, &dj, sizeof(DevJob), "upload job", &err)) return false;
-      if (j->built.nodes.size() > kNarrowStackNodes) wide_ = true;  // (never a path-kernel job)
+      // (a path-kernel job's tree is never that large)
+      if (j->built.nodes.size() > kNarrowStackNodes) wide_ = true;
       j->built = BuiltScene();  // host copy no longer needed
       j->state = 1;
       j->t_admit = Clock::now();
@@ -388,7 +417,7 @@ class Streamer {
     bool wave = false;
     for (SJob *j : resident_) {
       while (j->passes_issued < j->passes_total &&
-             (j->path_frame ? path_paths < kPathRound : ctl_total_ - last_cursor_ < ahead)) {
+             (j->paths ? path_paths < kPathRound : ctl_total_ - last_cursor_ < ahead)) {
         if (tickets_.size() >= ticket_cap) break;  // resumes after the next rewind
         const uint64_t npix = (uint64_t)j->W * j->H;
         const uint32_t s0 = j->passes_issued * j->pass_spp;
@@ -408,13 +437,8 @@ class Streamer {
         ticket_fin_.push_back(0);
         j->tickets.push_back(ti);
         j->passes_issued++;
-        if (j->path_frame) {
-          const uint64_t held = eng.cam_bytes();
-          if (!eng.run_paths(d_jobs_ + j->slot, h_jobs_[j->slot], t, j->path_frame, &err)) return false;
-          if (eng.cam_bytes() > held) {  // the engine keeps its table between jobs
-            pool->add_fixed((int64_t)(eng.cam_bytes() - held));
-            fixed_bytes_ += eng.cam_bytes() - held;
-          }
+        if (j->paths) {
+          if (!eng.run_paths(d_jobs_ + j->slot, h_jobs_[j->slot], t, 1, &j->space, &err)) return false;
           path_paths += t.paths;
           if (j->progress) break;
         } else {
@@ -445,7 +469,7 @@ class Streamer {
   bool want_w4() const {
     if (!eng.opt.bvh4 || wide_ || eng.opt.brute_force || eng.opt.refill <= 0) return false;
     for (const SJob *j : resident_)
-      if (!j->path_frame && j->dev.n_nodes > 0 && (j->dev.n_nodes4 == 0 || j->dev.stack4 + 3 > (uint32_t)kStackDepth))
+      if (!j->paths && j->dev.n_nodes > 0 && (j->dev.n_nodes4 == 0 || j->dev.stack4 + 3 > (uint32_t)kStackDepth))
         return false;
     return true;
   }
@@ -571,7 +595,7 @@ class Streamer {
     if (!eng.check(hipStreamSynchronize(eng.stream), "iteration", &err)) return false;
     if (wave_running_ && !check_wave()) return false;
     for (uint32_t t = ticket_lo_; t < n; ++t)
-      if (!ticket_fin_[t] && (ticket_job_[t]->path_frame ||
+      if (!ticket_fin_[t] && (ticket_job_[t]->paths ||
                               (wave_running_ && done_host_[t] == tickets_[t].paths)))
         ticket_fin_[t] = 1;
     // accumulate finished passes in pass order, per job

@@ -68,12 +68,7 @@ void Engine::bind_external(const ExternalBuffers &b, const Engine &owner) {
   l_alloc = b.l_slots;
   ticket_alloc = b.tickets_n;
   path_ctl_ = b.ctl;  // (no wavefront runs between the passes of a call)
-  cam_ = b.cam;
-  cam_px_ = b.cam_px;
-  cam_frame_ = 0;
-  compact_ = b.compact;
-  compact_nodes_ = b.compact_nodes;
-  compact_frame_ = 0;
+  space_ = PathSpace{b.cam, b.cam_px, 0, b.compact, b.compact_nodes, 0, true};
   opt.queue = b.queue;
   opt.l_capacity = b.l_slots;
   opt.pipes = 1;
@@ -93,13 +88,10 @@ void Engine::release_buffers() {
   if (first_hit_) { (void)hipFree(first_hit_); first_hit_ = nullptr; }
   first_hit_px_ = 0;
   first_hit_frame_ = 0;
-  if (cam_) { (void)hipFree(cam_); cam_ = nullptr; }
   if (path_ctl_) { (void)hipFree(path_ctl_); path_ctl_ = nullptr; }
-  if (compact_) { (void)hipFree(compact_); compact_ = nullptr; }
-  compact_nodes_ = 0;
-  compact_frame_ = 0;
-  cam_px_ = 0;
-  cam_frame_ = 0;
+  if (space_.cam) (void)hipFree(space_.cam);
+  if (space_.compact) (void)hipFree(space_.compact);
+  space_ = PathSpace();
   q_alloc = 0;
   l_alloc = 0;
   if (d_tickets) { (void)hipFree(d_tickets); d_tickets = nullptr; }
@@ -181,7 +173,7 @@ uint64_t Engine::device_bytes() const {
   // two queues of 14 words per slot plus the 8-byte hit record
   uint64_t b = (uint64_t)kSegments * seg_cap * (2 * 56 + 8) + l_alloc * sizeof(float4) +
                (uint64_t)ticket_alloc * (sizeof(DevTicket) + 8) + first_hit_px_ * sizeof(HitWord) +
-               cam_px_ * kCamBytes + compact_nodes_ * sizeof(DevNode4C);
+               space_.cam_px * kCamBytes + space_.compact_nodes * sizeof(DevNode4C);
   for (const auto &e : aux_) b += e->device_bytes();
   return b;
 }
@@ -306,8 +298,7 @@ static uint64_t scene_pieces(const BuiltScene &b, const DevJob *job, HostTransfe
   return end;
 }
 
-bool Engine::alloc_scene(const BuiltScene &b, DeviceScene *out, std::string *err) {
-  free_scene(out);
+void Engine::describe_scene(const BuiltScene &b, DeviceScene *out) {
   out->n_nodes = (uint32_t)b.nodes.size();
   out->n_nodes4 = (uint32_t)b.nodes4.size();
   out->stack4 = b.stack4;
@@ -316,6 +307,11 @@ bool Engine::alloc_scene(const BuiltScene &b, DeviceScene *out, std::string *err
   out->r0 = b.r0;
   out->reach = b.reach;
   out->depth = b.depth;
+}
+
+bool Engine::alloc_scene(const BuiltScene &b, DeviceScene *out, std::string *err) {
+  free_scene(out);
+  describe_scene(b, out);
   HostTransfer::Piece p[5];
   const uint64_t total = scene_pieces(b, nullptr, p);
   out->bytes = p[1].bytes + p[2].bytes + p[3].bytes + p[4].bytes;
@@ -478,59 +474,77 @@ int Engine::pipes_for(const DevTicket &t, bool lds) const {
 // tree), event counts, and the launch forms asked for by option (one ray per
 // lane, other workgroup sizes, every camera ray traced).
 bool Engine::takes_paths(const DevJob &j, const DevTicket &t) const {
-  if (!launch_paths || (external_ && (cam_px_ < (uint64_t)j.width * j.height || compact_nodes_ < j.n_nodes4)))
-    return false;
+  if (!launch_paths || (space_.fixed && space_.cam_px < (uint64_t)j.width * j.height)) return false;
   return !opt.count && opt.hit_reuse && !opt.brute_force && opt.refill > 0 && opt.bvh4 &&
          opt.block == 256 && j.max_bounces > 0 && j.max_bounces <= 255 && t.spp < (1u << 24) &&
          j.n_nodes4 > 0 && j.n_nodes <= kNarrowStackNodes && j.stack4 + 3 <= (uint32_t)kStackDepth;
 }
 
-bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame,
-                       std::string *err) {
-  const uint64_t npix = (uint64_t)j.width * j.height;
-  if (npix > cam_px_) {
-    if (cam_) (void)hipFree(cam_);
-    cam_ = nullptr;
-    cam_px_ = 0;
-    cam_frame_ = 0;
-    if (!check(hipMalloc((void **)&cam_, kCamBytes * npix), "hipMalloc(camera hits)", err)) return false;
-    cam_px_ = npix;
-  }
-  if (!path_ctl_ && !check(hipMalloc(&path_ctl_, sizeof(QueueCtl)), "hipMalloc(work list)", err))
-    return false;
-  // an earlier pass of the same frame recorded them
-  const bool carried = frame != 0 && frame == cam_frame_;
-  cam_frame_ = 0;
-
+// The pass and what its launches have in common.
+PathArgs Engine::path_args(const DevJob &j, const DevTicket &t) const {
   PathArgs a{};
-  a.job = d_job;
-  a.ctl = path_ctl_;
-  a.cam_ray = reinterpret_cast<float4 *>(cam_);
-  a.cam_hit = reinterpret_cast<uint2 *>(cam_ + sizeof(float4) * npix);
   a.L = L;
   a.l_cap = l_alloc;
   a.l_offset = t.l_offset;
-  a.npix = (uint32_t)npix;
+  a.npix = (uint32_t)((uint64_t)j.width * j.height);
   a.sample_base = t.sample_base;
   a.samples = t.spp;
   a.vk = opt.vk;
   a.refill = (uint32_t)opt.refill;
+  a.n_nodes4 = j.n_nodes4;
   // (the tree bound's default and more: whatever fits)
   plan_paths(&a, j, opt.lds_bvh >= EngineOptions().lds_bvh ? UINT64_MAX : opt.lds_bvh, opt.lds_objects);
+  return a;
+}
 
-  a.n_nodes4 = j.n_nodes4;
-  if (a.tree == kTreeCompact) {
-    if (j.n_nodes4 > compact_nodes_) {
-      if (compact_) (void)hipFree(compact_);
-      compact_ = nullptr;
-      compact_nodes_ = 0;
-      compact_frame_ = 0;
-      const uint32_t n = std::max(1024u, j.n_nodes4 + j.n_nodes4 / 4);
-      if (!check(hipMalloc((void **)&compact_, sizeof(DevNode4C) * n), "hipMalloc(compact tree)", err)) return false;
-      compact_nodes_ = n;
+uint32_t Engine::compact_nodes(const DevJob &j, const DevTicket &t) const {
+  return path_args(j, t).tree == kTreeCompact ? j.n_nodes4 : 0u;
+}
+
+bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame, PathSpace *space,
+                       std::string *err) {
+  PathSpace &sp = *space;
+  PathArgs a = path_args(j, t);
+  const uint64_t npix = a.npix;
+  // (compact and full nodes of one-primitive leaves differ in nothing else)
+  if (a.tree == kTreeCompact && sp.fixed && j.n_nodes4 > sp.compact_nodes) a.tree = kTreeLeaf1;
+  const bool grow_cam = npix > sp.cam_px;
+  const bool grow_compact = a.tree == kTreeCompact && j.n_nodes4 > sp.compact_nodes;
+  if (grow_cam || grow_compact) {
+    if (sp.fixed) {
+      *err = "path kernel's borrowed buffers too small (internal error)";
+      return false;
     }
-    a.compact = compact_;
+    // a free does not wait for a pass that is still queued
+    if (!check(hipStreamSynchronize(stream), "paths", err)) return false;
   }
+  if (grow_cam) {
+    if (sp.cam) (void)hipFree(sp.cam);
+    sp.cam = nullptr;
+    sp.cam_px = sp.cam_frame = 0;
+    if (!check(hipMalloc((void **)&sp.cam, kCamBytes * npix), "hipMalloc(camera hits)", err)) return false;
+    sp.cam_px = npix;
+  }
+  if (grow_compact) {
+    if (sp.compact) (void)hipFree(sp.compact);
+    sp.compact = nullptr;
+    sp.compact_nodes = 0;
+    sp.compact_frame = 0;
+    const uint32_t n = std::max(1024u, j.n_nodes4 + j.n_nodes4 / 4);
+    if (!check(hipMalloc((void **)&sp.compact, sizeof(DevNode4C) * n), "hipMalloc(compact tree)", err)) return false;
+    sp.compact_nodes = n;
+  }
+  if (!path_ctl_ && !check(hipMalloc(&path_ctl_, sizeof(QueueCtl)), "hipMalloc(work list)", err))
+    return false;
+  // an earlier pass of the same frame recorded them
+  const bool carried = frame != 0 && frame == sp.cam_frame;
+  sp.cam_frame = 0;
+
+  a.job = d_job;
+  a.ctl = path_ctl_;
+  a.cam_ray = reinterpret_cast<float4 *>(sp.cam);
+  a.cam_hit = reinterpret_cast<uint2 *>(sp.cam + sizeof(float4) * npix);
+  if (a.tree == kTreeCompact) a.compact = sp.compact;
 
   // Everything is queued without a wait in between; the caller waits for the
   // accumulation.  A launch's waves take its work list in chunks through a
@@ -599,10 +613,10 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
   }
   if (a.tree == kTreeCompact) {
     // (an option may have sent the frame's first passes to the other form)
-    const bool have = frame != 0 && frame == compact_frame_;
-    compact_frame_ = 0;
+    const bool have = frame != 0 && frame == sp.compact_frame;
+    sp.compact_frame = 0;
     if (!have && !check(launch_compact(a, stream), "compact tree", err)) return false;
-    compact_frame_ = frame;
+    sp.compact_frame = frame;
   }
   if (!carried && !launch(true)) return false;
   if (!launch(false)) return false;
@@ -629,7 +643,7 @@ bool Engine::run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t,
   }
 #endif
   drain.ok = true;
-  cam_frame_ = frame;
+  sp.cam_frame = frame;
   return true;
 }
 
@@ -660,7 +674,7 @@ bool Engine::run_tickets(const DevJob *d_jobs, std::vector<DevTicket> tickets,
     return false;
   }
   if (paths) {
-    if (!run_paths(d_jobs, host_jobs[0], traced[0], frame, err)) return false;
+    if (!run_paths(d_jobs, host_jobs[0], traced[0], frame, &space_, err)) return false;
     if (image && !opt.kernel_timing) {
       const uint32_t npix = host_jobs[0].width * host_jobs[0].height;
       const int grid = 8 * num_cus;

@@ -125,6 +125,18 @@ struct PassImage {
   bool queued = false;  // the pass has queued it
 };
 
+// What passes of the path kernel over one frame share: the camera-ray hits and
+// the compact tree that the first of them made.
+struct PathSpace {
+  unsigned char *cam = nullptr;  // camera-hit table
+  uint64_t cam_px = 0;           // pixels it has room for
+  uint64_t cam_frame = 0;        // frame whose hits it holds (0: none)
+  DevNode4C *compact = nullptr;  // compact tree
+  uint32_t compact_nodes = 0;    // nodes it has room for
+  uint64_t compact_frame = 0;    // frame whose tree it is (0: none)
+  bool fixed = false;            // the memory is another owner's: not grown, not freed
+};
+
 class Engine {
  public:
   ~Engine();
@@ -143,6 +155,7 @@ class Engine {
   // Allocates a scene's device copy; copies it (in stream order), with a job
   // record if there is one; both.
   bool alloc_scene(const BuiltScene &b, DeviceScene *out, std::string *err);
+  static void describe_scene(const BuiltScene &b, DeviceScene *out);  // its sizes alone
   bool copy_scene(const BuiltScene &b, const DeviceScene &s, const DevJob *job, std::string *err);
   bool upload_scene(const BuiltScene &b, DeviceScene *out, std::string *err) {
     return alloc_scene(b, out, err) && copy_scene(b, *out, nullptr, err);
@@ -172,10 +185,12 @@ class Engine {
   // A pass of the path kernel into the radiance slots t.l_offset.., queued on
   // this engine's stream and not waited for (nor, but for Vulkan semantics,
   // accumulated).  Passes with the same nonzero `frame` share the camera-ray
-  // hits the first of them records.
-  bool run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame,
+  // hits the first of them records in `space`, and its tree.
+  bool run_paths(const DevJob *d_job, const DevJob &j, const DevTicket &t, uint64_t frame, PathSpace *space,
                  std::string *err);
-  uint64_t cam_bytes() const { return cam_px_ * kCamBytes; }
+  // Nodes of a compact tree that the path kernel wants for this pass (0: it
+  // walks another form).
+  uint32_t compact_nodes(const DevJob &j, const DevTicket &t) const;
 
   // Host copies on `stream` (see HostTransfer).
   HostTransfer &transfer() { return *transfer_; }
@@ -252,12 +267,8 @@ class Engine {
   uint64_t first_hit_frame_ = 0;              // hit_frame whose hits first_hit_ holds (0: none)
   QueueCtl *path_ctl_ = nullptr;              // the path kernel's work-list counters (`ctl`
                                               // may hold a wavefront's queues meanwhile)
-  unsigned char *cam_ = nullptr;              // the path kernel's camera-hit table
-  uint64_t cam_px_ = 0;                       // pixels it holds
-  uint64_t cam_frame_ = 0;                    // hit_frame whose hits it holds (0: none)
-  DevNode4C *compact_ = nullptr;              // the path kernel's compact tree
-  uint64_t compact_frame_ = 0;                // hit_frame whose tree it is (0: none)
-  uint32_t compact_nodes_ = 0;                // nodes it has room for
+  PathSpace space_;                           // run_tickets' passes of the path kernel
+  PathArgs path_args(const DevJob &j, const DevTicket &t) const;
 };
 
 // Message returned by rd_last_error(NULL) (calls with no renderer handle).

@@ -3,6 +3,8 @@
 //   path_frames  frames, progressive passes, restarts and new scenes on one
 //                renderer, both semantics, the tree in every form, options
 //                that send single passes of a frame to the wavefront
+//   path_budget  a server whose budget a job fits without the path kernel's
+//                tables, with them and with room to spare
 // Test infrastructure only.
 #define main stress_main
 #include "stress.cpp"
@@ -58,13 +60,60 @@ void path_frames() {
   }
 }
 
+void path_budget() {
+  rd_server *s = nullptr;
+  rd_server_config any{0, 8, 0, 65536, 0};
+  if (rd_server_create(&any, &s) != RD_OK) return fail("server create");
+  rd_server_stats st{};
+  rd_server_stats_get(s, &st);
+  const uint64_t engine = st.engine_bytes;
+  rd_server_destroy(s);
+  std::vector<JobSpec> jobs;
+  for (int i = 0; i < 6; ++i) jobs.push_back(JobSpec{clustered(40 + i, 400, 1920, 1080 + 8 * i), 20, 6, 40ull + i});
+  // bytes a pixel that the budget leaves each job, and at least what the job
+  // reports to hold: accumulator, image and the tables of its kernel
+  const struct {
+    uint64_t per_pixel, held;
+  } cases[] = {{29, 28}, {60, 44}, {100, 44}, {1000, 44}};
+  for (const auto &c : cases) {
+    const uint64_t npix = 1920ull * (1080 + 8 * 5);
+    rd_server_config cfg{engine + c.per_pixel * npix + (1 << 20), 8, 0, 65536, 0};
+    const std::string what = "budget of " + std::to_string(c.per_pixel) + " bytes a pixel";
+    if (rd_server_create(&cfg, &s) != RD_OK) return fail(what + ": create");
+    for (int round = 0; round < 2; ++round) {  // what ran before changes nothing
+      std::vector<Out> outs(jobs.size());
+      std::vector<uint64_t> ids(jobs.size(), 0);
+      for (size_t i = 0; i < jobs.size(); ++i) {
+        rd_job_desc d = desc(jobs[i], &outs[i], true, i % 2 == 0);
+        if (rd_server_submit(s, &d, &ids[i]) != RD_OK) fail(what + ": " + rd_server_last_error(s));
+      }
+      for (size_t i = 0; i < jobs.size(); ++i) {
+        rd_job_result r{};
+        if (!ids[i]) continue;
+        if (rd_server_wait(s, ids[i], -1, &r) != RD_OK || !r.done || r.status != RD_OK) {
+          fail(what + ": job " + std::to_string(i) + ": " + rd_server_last_error(s));
+          continue;
+        }
+        check_out(jobs[i], outs[i], what);
+        const uint64_t px = (uint64_t)jobs[i].scene->s.camera.resolution_x * jobs[i].scene->s.camera.resolution_y;
+        if (r.device_bytes < c.held * px || r.device_bytes > (c.held + 1) * px)
+          fail(what + ": job holds " + std::to_string(r.device_bytes) + " bytes");
+      }
+    }
+    rd_server_stats_get(s, &st);
+    if (st.engine_bytes + st.hbm_peak > cfg.hbm_budget_bytes) fail(what + ": passed");
+    rd_server_destroy(s);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::string scenario = argc > 1 ? argv[1] : "";
-  if (scenario != "path_frames") return stress_main(argc, argv);
+  if (scenario != "path_frames" && scenario != "path_budget") return stress_main(argc, argv);
   fakehip::set_max_delay_us(20);
-  path_frames();
+  if (scenario == "path_frames") path_frames();
+  if (scenario == "path_budget") path_budget();
   device_clean(scenario.c_str());
   const auto st = fakehip::stats();
   std::printf("%llu kernels, %llu copies, %llu mallocs\n", (unsigned long long)st.kernels,
