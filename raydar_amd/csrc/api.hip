@@ -620,7 +620,7 @@ rd_status rd_render_frame_noalloc(rd_renderer *r, const rd_scene *scene, uint8_t
   // every call starts from its own state: the accumulator is cleared by a
   // kernel and the control block by run_tickets; the rest is written before
   // it is read
-  bool ok = se.check(se.transfer().upload(base + o_nodes, scene_pieces, 4, st), "upload scene", &err) &&
+  bool ok = se.check(se.transfer().upload_reserved(base + o_nodes, scene_pieces, 4, st), "upload scene", &err) &&
             se.upload(d_job, &job, sizeof(job), "upload job", &err);
   ok = ok && se.check(rdh::launch_zero_acc(acc, 4 * npix, st), "zero accumulator", &err);
   // render_next_sample timers (cpu.rs:194-196, 212-218) around passes of

@@ -98,6 +98,28 @@ class HostTransfer {
     const Piece p{src, 0, bytes};
     return upload(dst, &p, 1, stream);
   }
+  // The same within the memory that reserve() allocated, whatever the size:
+  // through the ring, which the reads behind it in the stream may use, with a
+  // wait only where the upload fills it.
+  hipError_t upload_reserved(void *dst, const Piece *pieces, int n, hipStream_t stream) {
+    uint64_t total = 0;
+    for (int k = 0; k < n; ++k)
+      if (pieces[k].bytes) total = std::max(total, pieces[k].offset + pieces[k].bytes);
+    for (uint64_t at = 0; at < total; at += kSlots * kSlot) {
+      const uint64_t end = std::min<uint64_t>(total, at + kSlots * kSlot);
+      hipError_t e = hipStreamSynchronize(stream);  // the ring's earlier contents have left it
+      if (e != hipSuccess) return e;
+      for (int k = 0; k < n; ++k) {
+        const uint64_t lo = std::max(at, pieces[k].offset), hi = std::min(end, pieces[k].offset + pieces[k].bytes);
+        if (lo < hi)
+          std::memcpy(ring_ + (lo - at), static_cast<const unsigned char *>(pieces[k].src) + (lo - pieces[k].offset),
+                      hi - lo);
+      }
+      e = hipMemcpyAsync(static_cast<unsigned char *>(dst) + at, ring_, end - at, hipMemcpyHostToDevice, stream);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
 
   // Pinned memory of kDirect bytes for the device to write by itself: valid
   // until the next read.

@@ -40,6 +40,7 @@ void set_max_delay_us(int max_us);
 struct Stats {
   uint64_t ops = 0, kernels = 0, copies = 0, graph_launches = 0, frees = 0, mallocs = 0;
   uint64_t live_allocs = 0, streams = 0;
+  uint64_t host_mallocs = 0, host_frees = 0;  // pinned memory
 };
 Stats stats();
 void count_kernel();

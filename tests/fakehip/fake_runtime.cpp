@@ -381,6 +381,7 @@ hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
   if (!*p) return ret(hipErrorOutOfMemory);
   std::lock_guard<std::mutex> g(g_mu);
   g_pinned[(uintptr_t)*p] = bytes;
+  g_stats.host_mallocs++;
   return hipSuccess;
 }
 
@@ -393,6 +394,7 @@ hipError_t hipHostFree(void *p) {
       g_errors.push_back("hipHostFree of a pointer that is not pinned host memory");
       return ret(hipErrorInvalidValue);
     }
+    g_stats.host_frees++;
   }
   std::free(p);
   return hipSuccess;

@@ -3,6 +3,9 @@
 //   path_frames  frames, progressive passes, restarts and new scenes on one
 //                renderer, both semantics, the tree in every form, options
 //                that send single passes of a frame to the wavefront
+//   noalloc_large  rd_render_frame_noalloc of scenes beyond the reserved upload
+//                memory, by the path kernel and the wavefront: nothing is
+//                allocated or freed during a call, pinned memory neither
 //   path_budget  a server whose budget a job fits without the path kernel's
 //                tables, with them and with room to spare
 // Test infrastructure only.
@@ -60,6 +63,33 @@ void path_frames() {
   }
 }
 
+void noalloc_large() {
+  rd_config cfg{1, 12};
+  rd_renderer *r = nullptr;
+  if (rd_create(&cfg, &r) != RD_OK) return fail("rd_create");
+  for (int n : {50, 1100, 1300, 5000, 30000, 60000, 50})
+    for (int block : {256, 128}) {
+      JobSpec j{clustered(n, n, 200, 150), 5, 12, (uint64_t)n};
+      const std::string what = "noalloc " + std::to_string(n) + " objects, block " + std::to_string(block);
+      rd_set_option(r, "block", block);
+      rd_set_max_sample_count(r, j.spp);
+      rd_set_seed(r, j.seed);
+      Out o;
+      o.rgba.assign(4ull * 200 * 150, 0);
+      const auto before = fakehip::stats();
+      if (rd_render_frame_noalloc(r, &j.scene->s, o.rgba.data(), o.rgba.size()) != RD_OK) {
+        fail(what + ": " + rd_last_error(r));
+        continue;
+      }
+      const auto after = fakehip::stats();
+      if (after.mallocs != before.mallocs || after.frees != before.frees) fail(what + ": device memory allocated");
+      if (after.host_mallocs != before.host_mallocs || after.host_frees != before.host_frees)
+        fail(what + ": pinned memory allocated or freed");
+      check_out(j, o, what);
+    }
+  rd_destroy(r);
+}
+
 void path_budget() {
   rd_server *s = nullptr;
   rd_server_config any{0, 8, 0, 65536, 0};
@@ -110,10 +140,12 @@ void path_budget() {
 
 int main(int argc, char **argv) {
   const std::string scenario = argc > 1 ? argv[1] : "";
-  if (scenario != "path_frames" && scenario != "path_budget") return stress_main(argc, argv);
+  if (scenario != "path_frames" && scenario != "path_budget" && scenario != "noalloc_large")
+    return stress_main(argc, argv);
   fakehip::set_max_delay_us(20);
   if (scenario == "path_frames") path_frames();
   if (scenario == "path_budget") path_budget();
+  if (scenario == "noalloc_large") noalloc_large();
   device_clean(scenario.c_str());
   const auto st = fakehip::stats();
   std::printf("%llu kernels, %llu copies, %llu mallocs\n", (unsigned long long)st.kernels,
