@@ -227,7 +227,8 @@ rd_status rd_read_accumulator(rd_renderer *r, float *out, size_t float_capacity)
  *                 chunks of c paths are dealt round-robin to the waves
  *                 (default 64)
  *   "lds_bvh"     scenes whose BVH nodes + primitives take at most this many
- *                 bytes are traversed from LDS (default 14336; 0 = never)
+ *                 bytes are traversed from LDS (0 = never; default 14336, for
+ *                 the path kernel whatever its LDS holds beside its stacks)
  *   "lds_objects" scenes whose objects (64 B each) take at most this many
  *                 bytes are shaded from a copy in LDS (default 16384; 0 = never)
  *   "bvh4"        1 = traverse the tree collapsed to 4-wide nodes (default),
@@ -256,7 +257,13 @@ rd_status rd_read_accumulator(rd_renderer *r, float *out, size_t float_capacity)
  *                 once (vulkan.rs:109-184).  Takes effect at the next
  *                 new_frame; needs block 256, refill > 0 and no counting;
  *                 not available in rd_render_frame_noalloc or the batch and
- *                 server handles. */
+ *                 server handles.
+ * A pass is traced by the path kernel (whole paths in one launch) unless an
+ * option asks for what only the wavefront kernels have, at about half the
+ * speed: "block" other than 256, "traversal" 1, "refill" 0, "bvh4" 0,
+ * "hit_reuse" 0 or "count" 1.  "lane_chunk", "shade_blocks" and "sync_every"
+ * are the wavefront's alone, and "queue" is, but for its part in "pipes".
+ * Images do not depend on which of the two traces a pass. */
 rd_status rd_set_option(rd_renderer *r, const char *key, int64_t value);
 rd_status rd_get_option(const rd_renderer *r, const char *key, int64_t *value);
 
@@ -293,7 +300,8 @@ rd_status rd_reset_counters(rd_renderer *r);
 
 /* Per-kernel device time (hipEvent pairs on the library's stream) of the
  * passes rendered while option "count" was 0 and option "kernel_timing" was
- * 1.  Index: 0 generate, 1 extend, 2 shade, 3 accumulate, 4 tonemap. */
+ * 1.  Index: 0 generate, 1 extend, 2 shade, 3 accumulate, 4 tonemap.  The path
+ * kernel's launches, which trace and shade, count as extend. */
 typedef struct rd_kernel_times {
   double total_ms[5];
   uint64_t launches[5];

@@ -72,6 +72,9 @@ void rd_batch_destroy(rd_batch *b);
  * kernels, small trees in LDS, samples split over pipes) driven by a host
  * thread of its own, one job after another, while the pipes take the other
  * jobs; read-only "solo_jobs" (jobs the lane has rendered, cumulative).
+ * A job's passes go to the path kernel unless an option asks for the wavefront
+ * kernels (rd_set_option), which "queue", "lane_chunk", "graph" and
+ * "iters_per_pump" are for.
  * Images do not depend on these options. */
 rd_status rd_batch_set_option(rd_batch *b, const char *key, int64_t value);
 rd_status rd_batch_get_option(const rd_batch *b, const char *key, int64_t *value);

@@ -492,8 +492,8 @@ PathArgs Engine::path_args(const DevJob &j, const DevTicket &t) const {
   a.vk = opt.vk;
   a.refill = (uint32_t)opt.refill;
   a.n_nodes4 = j.n_nodes4;
-  // (the tree bound's default and more: whatever fits)
-  plan_paths(&a, j, opt.lds_bvh >= EngineOptions().lds_bvh ? UINT64_MAX : opt.lds_bvh, opt.lds_objects);
+  // (the option's default, the wavefront's bound: whatever fits)
+  plan_paths(&a, j, opt.lds_bvh == EngineOptions().lds_bvh ? UINT64_MAX : opt.lds_bvh, opt.lds_objects);
   return a;
 }
 

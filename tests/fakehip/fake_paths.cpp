@@ -16,6 +16,7 @@
 #include "fake_kernels.cpp"
 #undef launch_tonemap
 
+#include <atomic>
 #include <cstring>
 
 #include "../../raydar_amd/csrc/paths.hpp"
@@ -188,6 +189,9 @@ void fake_paths(const PathArgs a, bool record, int grid) {
 
 }  // namespace
 
+std::atomic<uint64_t> g_tree_bytes{0};  // of the last planned pass, for the scenarios
+std::atomic<bool> g_tree_in_lds{false};
+
 // The real plan's choices, with lines low enough for the scenarios to cross.
 void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh, uint64_t lds_objects) {
   a->stack_rows = j.stack4 + 4;
@@ -197,6 +201,8 @@ void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh, uint64_t lds_obj
   a->tree = lds ? (leaf1 ? kTreeLdsLeaf1 : kTreeLds)
                 : !leaf1 ? kTreeMemory
                          : !a->vk && (uint64_t)a->npix * a->samples >= 1u << 18 ? kTreeCompact : kTreeLeaf1;
+  g_tree_bytes = tree;
+  g_tree_in_lds = lds;
   a->lds_bvh_bytes = lds ? (uint32_t)tree : 0u;
   a->lds_obj_bytes = objects <= lds_objects ? (uint32_t)objects : 0u;
 }

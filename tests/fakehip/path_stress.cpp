@@ -3,12 +3,21 @@
 //   path_frames  frames, progressive passes, restarts and new scenes on one
 //                renderer, both semantics, the tree in every form, options
 //                that send single passes of a frame to the wavefront
+//   lds_limit    the option that bounds a tree in LDS bounds the path kernel's
 //   noalloc_large  rd_render_frame_noalloc of scenes beyond the reserved upload
 //                memory, by the path kernel and the wavefront: nothing is
 //                allocated or freed during a call, pinned memory neither
 //   path_budget  a server whose budget a job fits without the path kernel's
 //                tables, with them and with room to spare
 // Test infrastructure only.
+#include <atomic>
+#include <cstdint>
+
+namespace rdh {
+extern std::atomic<uint64_t> g_tree_bytes;  // fake_paths.cpp
+extern std::atomic<bool> g_tree_in_lds;
+}  // namespace rdh
+
 #define main stress_main
 #include "stress.cpp"
 #undef main
@@ -61,6 +70,27 @@ void path_frames() {
       frame(r, jobs[(i * 7 + pipes) % jobs.size()], i % 3 == 2, "path frame " + std::to_string(i));
     rd_destroy(r);
   }
+}
+
+void lds_limit() {
+  auto sc = clustered(3, 200, 64, 48);
+  rd_config cfg{1, 4};
+  rd_renderer *r = nullptr;
+  if (rd_create(&cfg, &r) != RD_OK) return fail("rd_create");
+  std::vector<uint8_t> img(4 * 64 * 48);
+  auto in_lds = [&](int64_t limit) {
+    if (limit >= 0 && rd_set_option(r, "lds_bvh", limit) != RD_OK) fail("lds_bvh");
+    if (rd_render_frame(r, &sc->s, img.data(), img.size()) != RD_OK) fail(rd_last_error(r));
+    return rdh::g_tree_in_lds.load();
+  };
+  if (!in_lds(-1)) fail("by default a tree that fits is walked from LDS");
+  const int64_t tree = (int64_t)rdh::g_tree_bytes.load();
+  if (tree <= 14336 + 8) return fail("the tree says nothing: " + std::to_string(tree));
+  for (int64_t limit : {tree, tree + 1, (int64_t)131072})
+    if (!in_lds(limit)) fail("tree in memory below a limit of " + std::to_string(limit));
+  for (int64_t limit : {(int64_t)0, (int64_t)14335, (int64_t)14337, tree - 1})
+    if (in_lds(limit)) fail("tree in LDS above a limit of " + std::to_string(limit));
+  rd_destroy(r);
 }
 
 void noalloc_large() {
@@ -140,12 +170,14 @@ void path_budget() {
 
 int main(int argc, char **argv) {
   const std::string scenario = argc > 1 ? argv[1] : "";
-  if (scenario != "path_frames" && scenario != "path_budget" && scenario != "noalloc_large")
+  if (scenario != "path_frames" && scenario != "path_budget" && scenario != "noalloc_large" &&
+      scenario != "lds_limit")
     return stress_main(argc, argv);
   fakehip::set_max_delay_us(20);
   if (scenario == "path_frames") path_frames();
   if (scenario == "path_budget") path_budget();
   if (scenario == "noalloc_large") noalloc_large();
+  if (scenario == "lds_limit") lds_limit();
   device_clean(scenario.c_str());
   const auto st = fakehip::stats();
   std::printf("%llu kernels, %llu copies, %llu mallocs\n", (unsigned long long)st.kernels,
