@@ -9,7 +9,6 @@
 #include <cstdint>
 #include <cstring>
 #include <functional>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -211,7 +210,7 @@ class HostTransfer {
         helpers.emplace_back([&] {
           if (hipSetDevice(device) == hipSuccess) work();
         });
-    } catch (const std::system_error &) {  // fewer threads then
+    } catch (...) {  // no thread or no memory for one: fewer threads then
     }
     work();
     for (std::thread &t : helpers) t.join();

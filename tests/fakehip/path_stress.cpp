@@ -4,6 +4,7 @@
 //                renderer, both semantics, the tree in every form, options
 //                that send single passes of a frame to the wavefront
 //   lds_limit    the option that bounds a tree in LDS bounds the path kernel's
+//   no_memory    image readback while the host has no memory for its threads
 //   noalloc_large  rd_render_frame_noalloc of scenes beyond the reserved upload
 //                memory, by the path kernel and the wavefront: nothing is
 //                allocated or freed during a call, pinned memory neither
@@ -12,6 +13,20 @@
 // Test infrastructure only.
 #include <atomic>
 #include <cstdint>
+#include <cstdlib>
+#include <new>
+
+#include "../../raydar_amd/csrc/transfer.hpp"
+
+// The allocation of this thread that fails, counted down (0: none does).
+static thread_local int t_fail_new = 0;
+void *operator new(size_t n) {
+  if (t_fail_new > 0 && --t_fail_new == 0) throw std::bad_alloc();
+  if (void *p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 namespace rdh {
 extern std::atomic<uint64_t> g_tree_bytes;  // fake_paths.cpp
@@ -93,6 +108,32 @@ void lds_limit() {
   rd_destroy(r);
 }
 
+void no_memory() {
+  // the callback runs just before the reading threads are made
+  constexpr uint64_t bytes = 9u << 20;
+  hipStream_t stream;
+  unsigned char *device = nullptr;
+  if (hipStreamCreate(&stream) != hipSuccess || hipMalloc((void **)&device, bytes) != hipSuccess) return fail("setup");
+  std::vector<unsigned char> src(bytes), dst(bytes);
+  for (uint64_t i = 0; i < bytes; ++i) src[i] = (unsigned char)(i * 2654435761u >> 13);
+  if (hipMemcpy(device, src.data(), bytes, hipMemcpyHostToDevice) != hipSuccess) return fail("setup");
+  {
+    rdh::HostTransfer transfer;
+    for (int nth : {0, 1, 2, 3, 4}) {
+      std::fill(dst.begin(), dst.end(), 0);
+      const rdh::HostTransfer::Read read{dst.data(), device, bytes};
+      const hipError_t e = transfer.read(&read, 1, stream, 0, [&] {
+        t_fail_new = nth;
+        return hipSuccess;
+      });
+      t_fail_new = 0;
+      if (e != hipSuccess || dst != src) fail("read with allocation " + std::to_string(nth) + " failing");
+    }
+  }
+  (void)hipFree(device);
+  (void)hipStreamDestroy(stream);
+}
+
 void noalloc_large() {
   rd_config cfg{1, 12};
   rd_renderer *r = nullptr;
@@ -171,13 +212,14 @@ void path_budget() {
 int main(int argc, char **argv) {
   const std::string scenario = argc > 1 ? argv[1] : "";
   if (scenario != "path_frames" && scenario != "path_budget" && scenario != "noalloc_large" &&
-      scenario != "lds_limit")
+      scenario != "lds_limit" && scenario != "no_memory")
     return stress_main(argc, argv);
   fakehip::set_max_delay_us(20);
   if (scenario == "path_frames") path_frames();
   if (scenario == "path_budget") path_budget();
   if (scenario == "noalloc_large") noalloc_large();
   if (scenario == "lds_limit") lds_limit();
+  if (scenario == "no_memory") no_memory();
   device_clean(scenario.c_str());
   const auto st = fakehip::stats();
   std::printf("%llu kernels, %llu copies, %llu mallocs\n", (unsigned long long)st.kernels,
