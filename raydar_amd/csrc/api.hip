@@ -291,11 +291,14 @@ rd_status render_samples(rd_renderer *r, uint32_t k, rdh::PassImage *image) {
 // print_frame_buffer (cpu.rs:221-230) on the device, then copy out.  The `k`
 // samples that render_samples just queued are waited for and counted, and the
 // timers end before the copy (and the tonemap, if it was not part of the pass).
+// They count also if only the image fails: the accumulator holds them.
 rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba, const rdh::PassImage &image) {
   std::string err;
   const uint64_t npix = (uint64_t)r->W * r->H;
+  bool open = k > 0;  // not counted yet
   auto counted = [&] {
-    if (!k) return;
+    if (!open) return;
+    open = false;
     r->sample_count += k;
     if (r->sample_count == r->cfg.max_sample_count) {
       r->render_timer.end();
@@ -303,8 +306,12 @@ rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba, const rdh::Pas
     }
     r->sample_timer.end_multiple(k);
   };
+  auto failed = [&] {
+    if (open && hipStreamSynchronize(r->eng.stream) == hipSuccess) counted();
+    return device_fail(r, err);
+  };
   if (image.queued && image.rgba != r->rgba_d) {
-    if (!r->eng.check(hipStreamSynchronize(r->eng.stream), "render", &err)) return device_fail(r, err);
+    if (!r->eng.check(hipStreamSynchronize(r->eng.stream), "render", &err)) return failed();
     counted();
     std::memcpy(rgba, image.rgba, 4 * npix);
     return RD_OK;
@@ -315,31 +322,31 @@ rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba, const rdh::Pas
     // 2 ms late (183 objects at 4K, 8 spp 8.9 ms, so 7.0).
     if (!r->eng.check(hipEventRecord(r->rendered, r->eng.stream), "hipEventRecord", &err) ||
         (r->eng.pipes_used > 1 && !r->eng.check(hipEventSynchronize(r->rendered), "render", &err)))
-      return device_fail(r, err);
+      return failed();
     const rdh::HostTransfer::Read read{rgba, r->rgba_d, 4 * npix};
     const hipError_t e = r->eng.transfer().read(&read, 1, r->eng.stream, r->eng.device, [&] {
       const hipError_t w = hipEventSynchronize(r->rendered);
       if (w == hipSuccess) counted();
       return w;
     });
-    return r->eng.check(e, "read image", &err) ? RD_OK : device_fail(r, err);
+    return r->eng.check(e, "read image", &err) ? RD_OK : failed();
   }
   const int grid = (int)std::min<uint64_t>((npix + 255) / 256, 8192);
   // An event tells when the passes have ended while the tonemap runs on; for
   // images below a megabyte it costs more (20 us) than the gap it fills.
   const bool ahead = k && 4 * npix >= 1u << 20;
   if (ahead && !r->eng.check(hipEventRecord(r->rendered, r->eng.stream), "hipEventRecord", &err))
-    return device_fail(r, err);
+    return failed();
   if (k && !ahead && !r->eng.check(hipStreamSynchronize(r->eng.stream), "render", &err))
-    return device_fail(r, err);
+    return failed();
   const hipError_t e = rdh::launch_tonemap(r->scene.job, (uint32_t)npix, (float)(r->sample_count + k), r->rgba_d,
                                            r->eng.counters, r->eng.opt.count != 0, grid, r->eng.stream,
                                            r->frame_vk != 0);
   if (!r->eng.check(e, "tonemap", &err) ||
       (ahead && !r->eng.check(hipEventSynchronize(r->rendered), "render", &err)))
-    return device_fail(r, err);
+    return failed();
   counted();
-  if (!r->eng.read(rgba, r->rgba_d, 4 * npix, "read image", &err)) return device_fail(r, err);
+  if (!r->eng.read(rgba, r->rgba_d, 4 * npix, "read image", &err)) return failed();
   return RD_OK;
 }
 

@@ -191,6 +191,7 @@ void fake_paths(const PathArgs a, bool record, int grid) {
 
 std::atomic<uint64_t> g_tree_bytes{0};  // of the last planned pass, for the scenarios
 std::atomic<bool> g_tree_in_lds{false};
+std::atomic<int> g_fail_tonemaps{0};  // launches of it that fail
 
 // The real plan's choices, with lines low enough for the scenarios to cross.
 void plan_paths(PathArgs *a, const DevJob &j, uint64_t lds_bvh, uint64_t lds_objects) {
@@ -249,6 +250,10 @@ hipError_t launch_tonemap(const DevJob *job, uint32_t n, float spp, uchar4 *out,
                           hipStream_t st, bool) {
   hook_paths();
   if (grid <= 0) return hipErrorInvalidValue;
+  if (g_fail_tonemaps > 0) {
+    --g_fail_tonemaps;
+    return hipErrorInvalidValue;
+  }
   fakehip::enqueue(st, [job, n, spp, out] {
     fakehip::count_kernel();
     std::lock_guard<std::mutex> g(g_k);

@@ -4,6 +4,8 @@
 //                renderer, both semantics, the tree in every form, options
 //                that send single passes of a frame to the wavefront
 //   lds_limit    the option that bounds a tree in LDS bounds the path kernel's
+//   no_image     passes whose image fails: the samples are in the accumulator
+//                and count
 //   no_memory    image readback while the host has no memory for its threads
 //   noalloc_large  rd_render_frame_noalloc of scenes beyond the reserved upload
 //                memory, by the path kernel and the wavefront: nothing is
@@ -25,12 +27,14 @@ void *operator new(size_t n) {
   if (void *p = std::malloc(n ? n : 1)) return p;
   throw std::bad_alloc();
 }
+void *operator new(size_t n, const std::nothrow_t &) noexcept { return std::malloc(n ? n : 1); }
 void operator delete(void *p) noexcept { std::free(p); }
 void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 namespace rdh {
 extern std::atomic<uint64_t> g_tree_bytes;  // fake_paths.cpp
 extern std::atomic<bool> g_tree_in_lds;
+extern std::atomic<int> g_fail_tonemaps;
 }  // namespace rdh
 
 #define main stress_main
@@ -106,6 +110,31 @@ void lds_limit() {
   for (int64_t limit : {(int64_t)0, (int64_t)14335, (int64_t)14337, tree - 1})
     if (in_lds(limit)) fail("tree in LDS above a limit of " + std::to_string(limit));
   rd_destroy(r);
+}
+
+void no_image() {
+  for (uint32_t side : {60u, 700u}) {  // images below and above a megabyte
+    JobSpec j{clustered(side, 80, side, side), 12, 6, 77};
+    rd_config cfg{12, 6};
+    rd_renderer *r = nullptr;
+    if (rd_create(&cfg, &r) != RD_OK) return fail("rd_create");
+    rd_set_seed(r, j.seed);
+    rd_set_samples_per_pass(r, 4);
+    rd_set_option(r, "kernel_timing", 1);  // (the tonemap is then a launch of its own)
+    Out o;
+    o.rgba.assign(4ull * side * side, 0);
+    if (rd_new_frame(r, &j.scene->s) != RD_OK) return fail(rd_last_error(r));
+    for (int pass = 1, produced = 0; pass <= 3; ++pass) {
+      rdh::g_fail_tonemaps = pass == 2;
+      const rd_status st = rd_render_sample(r, nullptr, o.rgba.data(), o.rgba.size(), &produced);
+      if (st != (pass == 2 ? RD_ERR_DEVICE : RD_OK)) fail("status of pass " + std::to_string(pass));
+      if (rd_sample_count(r) != 4u * pass) fail(std::to_string(rd_sample_count(r)) + " samples counted");
+    }
+    o.acc.assign(o.rgba.size(), 0.0f);
+    if (rd_read_accumulator(r, o.acc.data(), o.acc.size()) != RD_OK) fail("accumulator");
+    check_out(j, o, "frame with a pass of no image");
+    rd_destroy(r);
+  }
 }
 
 void no_memory() {
@@ -212,7 +241,7 @@ void path_budget() {
 int main(int argc, char **argv) {
   const std::string scenario = argc > 1 ? argv[1] : "";
   if (scenario != "path_frames" && scenario != "path_budget" && scenario != "noalloc_large" &&
-      scenario != "lds_limit" && scenario != "no_memory")
+      scenario != "lds_limit" && scenario != "no_memory" && scenario != "no_image")
     return stress_main(argc, argv);
   fakehip::set_max_delay_us(20);
   if (scenario == "path_frames") path_frames();
@@ -220,6 +249,7 @@ int main(int argc, char **argv) {
   if (scenario == "noalloc_large") noalloc_large();
   if (scenario == "lds_limit") lds_limit();
   if (scenario == "no_memory") no_memory();
+  if (scenario == "no_image") no_image();
   device_clean(scenario.c_str());
   const auto st = fakehip::stats();
   std::printf("%llu kernels, %llu copies, %llu mallocs\n", (unsigned long long)st.kernels,
