@@ -73,6 +73,13 @@ rd_status rd_debug_world(const rd_scene *scene, const float *dirs, uint32_t n, f
 /* Philox-4x32-10 on the GPU: in n x 6 words (counter[4], key[2]), out n x 4. */
 rd_status rd_debug_philox(const uint32_t *in, uint32_t n, uint32_t *out);
 
+/* The kernels' short exact forms on the GPU (pathmath.hpp), out[i] for which =
+ * 0: the root of a[i]; 1: 1 / a[i]; 2: a[i] / b[i], for |a| in [2^-60, 2^60] and
+ * |b| in [2^-20, 2^20]; 3: the x component of (a[i], b[i], 0) normalised;
+ * 4 and 5: the forms of 0 and 1 without their guards, for a[i] in
+ * [2^-96, 2^100) and |a[i]| in [2^-60, 2^60). */
+rd_status rd_debug_arith(int which, const float *a, const float *b, uint32_t n, float *out);
+
 /* A plain device copy of `bytes` (multiple of 16, <= 32 GiB) between two
  * fresh buffers, `reps` launches of k_copy_calibration, each timed with
  * hipEvents into ms[reps] (may be NULL).  It reads and writes exactly

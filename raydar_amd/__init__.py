@@ -73,6 +73,7 @@ def lib():
         "rd_debug_camera_rays": (C.c_int, [sp, C.c_void_p, C.c_uint32, C.c_void_p]),
         "rd_debug_world": (C.c_int, [sp, C.c_void_p, C.c_uint32, C.c_void_p]),
         "rd_debug_philox": (C.c_int, [C.c_void_p, C.c_uint32, C.c_void_p]),
+        "rd_debug_arith": (C.c_int, [C.c_int, C.c_void_p, C.c_void_p, C.c_uint32, C.c_void_p]),
         "rd_debug_copy_calibration": (C.c_int, [C.c_uint64, C.c_uint32, C.c_void_p]),
         "rd_debug_host_bvh_info": (C.c_int, [sp, C.c_int, P(C.c_uint32), P(C.c_uint32),
                                              C.c_char_p, C.c_size_t]),
@@ -352,6 +353,18 @@ def debug_philox(ctr_key):
     ctr_key = np.ascontiguousarray(ctr_key, np.uint32).reshape(-1, 6)
     out = np.zeros((len(ctr_key), 4), np.uint32)
     check(lib().rd_debug_philox(_ptr(ctr_key), len(ctr_key), _ptr(out)))
+    return out
+
+
+def debug_arith(which, a, b=None):
+    """The kernels' exact short forms: "sqrt", "rcp", "div" (a / b), "unit" (x of
+    the normalised (a, b, 0)), and the first two without their guards."""
+    a = np.ascontiguousarray(a, np.float32)
+    b = a if b is None else np.ascontiguousarray(b, np.float32)
+    assert a.shape == b.shape and a.ndim == 1
+    out = np.zeros_like(a)
+    k = ("sqrt", "rcp", "div", "unit", "sqrt_normal", "rcp_normal").index(which)
+    check(lib().rd_debug_arith(k, _ptr(a), _ptr(b), len(a), _ptr(out)))
     return out
 
 

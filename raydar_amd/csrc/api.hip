@@ -1148,6 +1148,24 @@ rd_status rd_debug_philox(const uint32_t *in, uint32_t n, uint32_t *out) {
   return finish(hipSuccess);
 }
 
+rd_status rd_debug_arith(int which, const float *a, const float *b, uint32_t n, float *out) {
+  if (which < 0 || which > 5 || !a || !b || !out) return RD_ERR_INVALID_ARGUMENT;
+  int nd = 0;
+  if (!rdh::launch_debug_arith || hipGetDeviceCount(&nd) != hipSuccess || nd == 0) {
+    (void)hipGetLastError();
+    rdh::set_global_error("no HIP device available");
+    return RD_ERR_DEVICE;
+  }
+  DebugCtx c;
+  const float *d_a = c.dev(a, n), *d_b = c.dev(b, n);
+  float *d_out = c.dev<float>(nullptr, n);
+  if (!d_a || !d_b || !d_out) return RD_ERR_OUT_OF_MEMORY;
+  rd_status st = finish(rdh::launch_debug_arith(which, d_a, d_b, n, d_out, nullptr));
+  if (st != RD_OK) return st;
+  if (n) (void)hipMemcpy(out, d_out, 4ull * n, hipMemcpyDeviceToHost);
+  return finish(hipSuccess);
+}
+
 rd_status rd_debug_copy_calibration(uint64_t bytes, uint32_t reps, float *ms) {
   if (bytes == 0 || bytes % 16 || bytes > (1ull << 35) || reps == 0 || reps > 1000)
     return RD_ERR_INVALID_ARGUMENT;

@@ -758,6 +758,19 @@ __global__ __launch_bounds__(256) void k_finish(const DevJob *job, DevTicket T, 
   }
 }
 
+__global__ __launch_bounds__(256) void k_debug_arith(int which, const float *a, const float *b, uint32_t n,
+                                                     float *out) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n) return;
+  const float x = a[i], y = b[i];
+  out[i] = which == 0   ? sqrt_rn(x)
+           : which == 1 ? rcp_rn(x)
+           : which == 2 ? div_rn(x, y, rcp_rn_normal(y))
+           : which == 3 ? normalize(f3(x, y, 0.0f)).x
+           : which == 4 ? sqrt_rn_normal(x)
+                        : rcp_rn_normal(x);
+}
+
 template <bool VK>
 const void *paths_fn_of(PathTree tree, bool record) {
   switch (tree) {
@@ -856,6 +869,12 @@ hipError_t launch_finish(const DevJob *job, const DevTicket &t, uint32_t npix, c
                          uchar4 *rgba, int max_grid, hipStream_t st) {
   const uint32_t grid = std::min<uint32_t>((npix + 255u) / 256u, (uint32_t)max_grid);
   k_finish<<<grid, 256, 0, st>>>(job, t, npix, L, samples, rgba);
+  return hipGetLastError();
+}
+
+hipError_t launch_debug_arith(int which, const float *a, const float *b, uint32_t n, float *out, hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  k_debug_arith<<<(uint32_t)((n + 255ull) / 256), 256, 0, st>>>(which, a, b, n, out);
   return hipGetLastError();
 }
 

@@ -67,5 +67,8 @@ __attribute__((weak)) hipError_t launch_compact(const PathArgs &a, hipStream_t s
 __attribute__((weak)) hipError_t launch_finish(const DevJob *job, const DevTicket &t, uint32_t npix,
                                                const float4 *L, float samples, uchar4 *rgba,
                                                int max_grid, hipStream_t st);
+// Parity-test entry (rd_debug_arith): `n` values by the short exact forms.
+__attribute__((weak)) hipError_t launch_debug_arith(int which, const float *a, const float *b, uint32_t n,
+                                                    float *out, hipStream_t st);
 
 }  // namespace rdh
