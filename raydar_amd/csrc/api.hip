@@ -131,6 +131,7 @@ struct rd_renderer {
   uint32_t *vk_rng = nullptr;  // Vulkan semantics: per-pixel PCG state
   uint32_t W = 0, H = 0;
   bool has_frame = false;
+  bool queued = false;  // work on the resident frame's buffers may still be queued
   // bumped by new_frame and restart_frame: the passes of one frame share
   // their camera-ray hits (recorded by the frame's first pass)
   uint64_t frame_serial = 0;
@@ -181,6 +182,10 @@ rd_status snapshot(rd_renderer *r, const rd_scene *s, bool zero_acc) {
   if (!rdh::build_scene(*s, r->eng.opt.leaf, &built, &err)) return r->fail(RD_ERR_INVALID_ARGUMENT, err);
   if (!rdh::check_bvh(built, &err)) return r->fail(RD_ERR_INVALID_ARGUMENT, "BVH build: " + err);
   r->has_frame = false;  // until the new one is whole
+  // The old one's buffers go back to the cache, which may free them, and a free
+  // does not wait for an upload or a clearing that no pass has followed yet.
+  if (r->queued && !r->eng.check(hipStreamSynchronize(r->eng.stream), "new frame", &err)) return device_fail(r, err);
+  r->queued = true;
   if (!r->eng.alloc_scene(built, &r->scene, &err)) return device_fail(r, err);
   const uint32_t W = s->camera.resolution_x, H = s->camera.resolution_y;
   if (W != r->W || H != r->H || !r->acc) {
@@ -251,6 +256,7 @@ rd_status render_samples(rd_renderer *r, uint32_t k, rdh::PassImage *image) {
   r->prepare_timer.end_if_not_ended();
   r->render_timer.start_if_not_started();
   r->sample_timer.start();
+  r->queued = true;
   rd_status st = refresh_job(r);
   if (st != RD_OK) return st;
   std::string err;
@@ -314,6 +320,7 @@ rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba, const rdh::Pas
     if (!r->eng.check(hipStreamSynchronize(r->eng.stream), "render", &err)) return failed();
     counted();
     std::memcpy(rgba, image.rgba, 4 * npix);
+    r->queued = false;
     return RD_OK;
   }
   if (image.queued) {
@@ -329,7 +336,9 @@ rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba, const rdh::Pas
       if (w == hipSuccess) counted();
       return w;
     });
-    return r->eng.check(e, "read image", &err) ? RD_OK : failed();
+    if (!r->eng.check(e, "read image", &err)) return failed();
+    r->queued = false;
+    return RD_OK;
   }
   const int grid = (int)std::min<uint64_t>((npix + 255) / 256, 8192);
   // An event tells when the passes have ended while the tonemap runs on; for
@@ -347,6 +356,7 @@ rd_status finish_image(rd_renderer *r, uint32_t k, uint8_t *rgba, const rdh::Pas
     return failed();
   counted();
   if (!r->eng.read(rgba, r->rgba_d, 4 * npix, "read image", &err)) return failed();
+  r->queued = false;
   return RD_OK;
 }
 
@@ -440,6 +450,7 @@ rd_status rd_restart_frame(rd_renderer *r) {
   r->frame_timer.start();
   r->prepare_timer.start();
   r->sample_count = 0;
+  r->queued = true;
   std::string err;
   if (!r->eng.check(rdh::launch_zero_acc(r->acc, 4ull * r->W * r->H, r->eng.stream),
                     "zero accumulator", &err))

@@ -6,6 +6,7 @@
 //   lds_limit    the option that bounds a tree in LDS bounds the path kernel's
 //   no_image     passes whose image fails: the samples are in the accumulator
 //                and count
+//   new_scenes   one new scene after another, with nothing rendered between
 //   no_memory    image readback while the host has no memory for its threads
 //   noalloc_large  rd_render_frame_noalloc of scenes beyond the reserved upload
 //                memory, by the path kernel and the wavefront: nothing is
@@ -137,6 +138,25 @@ void no_image() {
   }
 }
 
+void new_scenes() {
+  // The first image's accumulator and bytes are more than a renderer keeps for reuse, so
+  // the second scene has the former freed, with its clearing perhaps still queued.
+  fakehip::set_max_delay_us(3000);
+  for (int k = 0; k < 12; ++k) {
+    auto big = clustered(k, 20, 16384, 16384), small = clustered(k, 20, 40, 30);
+    rd_config cfg{2, 6};
+    rd_renderer *r = nullptr;
+    if (rd_create(&cfg, &r) != RD_OK) return fail("rd_create");
+    if (rd_new_frame(r, &big->s) != RD_OK) fail(rd_last_error(r));
+    if (k % 2 && rd_restart_frame(r) != RD_OK) fail(rd_last_error(r));
+    if (rd_new_frame(r, &small->s) != RD_OK) fail(rd_last_error(r));
+    std::vector<uint8_t> img(4 * 40 * 30);
+    if (k % 3 == 0 && rd_render_frame(r, &small->s, img.data(), img.size()) != RD_OK) fail(rd_last_error(r));
+    rd_destroy(r);
+  }
+  fakehip::set_max_delay_us(20);
+}
+
 void no_memory() {
   // the callback runs just before the reading threads are made
   constexpr uint64_t bytes = 9u << 20;
@@ -241,7 +261,7 @@ void path_budget() {
 int main(int argc, char **argv) {
   const std::string scenario = argc > 1 ? argv[1] : "";
   if (scenario != "path_frames" && scenario != "path_budget" && scenario != "noalloc_large" &&
-      scenario != "lds_limit" && scenario != "no_memory" && scenario != "no_image")
+      scenario != "lds_limit" && scenario != "no_memory" && scenario != "no_image" && scenario != "new_scenes")
     return stress_main(argc, argv);
   fakehip::set_max_delay_us(20);
   if (scenario == "path_frames") path_frames();
@@ -250,6 +270,7 @@ int main(int argc, char **argv) {
   if (scenario == "lds_limit") lds_limit();
   if (scenario == "no_memory") no_memory();
   if (scenario == "no_image") no_image();
+  if (scenario == "new_scenes") new_scenes();
   device_clean(scenario.c_str());
   const auto st = fakehip::stats();
   std::printf("%llu kernels, %llu copies, %llu mallocs\n", (unsigned long long)st.kernels,

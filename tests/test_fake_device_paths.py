@@ -22,7 +22,7 @@ def tsan(tmp_path_factory):
 @pytest.mark.parametrize("args,nosync", [(["path_frames"], "1"), (["plain"], "0"), (["noalloc"], "1"),
                                          (["batch"], "1"), (["path_budget"], "1"),
                                          (["noalloc_large"], "0"), (["lds_limit"], "0"), (["no_memory"], "0"),
-                                         (["no_image"], "0"),
+                                         (["no_image"], "0"), (["new_scenes"], "1"),
                                          (["server", "--seconds", "20", "--speed", "20"], "1")])
 def test_path_kernel_host_code_asan(asan, args, nosync):
     _run(asan, args, 900, FAKEHIP_FREE_NOSYNC=nosync)
