@@ -239,14 +239,14 @@ def calibrate_copy(nbytes):
           flush=True)
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "extend_plain_1080p_hbm_traffic.md")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "path_plain_1080p_hbm_traffic.md")
 
 
 KERNEL_SOURCES = ("kernels.hip", "paths.hip", "kernel_util.hpp", "pathmath.hpp", "layout.hpp", "engine.hip")
 
 
 def kernel_sources_sha16():
-    """Hash of the sources that decide the extend kernel's memory traffic."""
+    """Hash of the sources that decide the path kernel's memory traffic."""
     import hashlib
     h = hashlib.sha256()
     for name in KERNEL_SOURCES:
@@ -255,8 +255,8 @@ def kernel_sources_sha16():
     return h.hexdigest()[:16]
 
 
-def extend_traffic(workload):
-    """HBM bytes per extend launch from the committed rocprofv3 --pmc summary
+def path_traffic(workload):
+    """HBM bytes of the path kernel's launches of one pass from the committed rocprofv3 --pmc summary
     (FETCH_SIZE + WRITE_SIZE, each scaled by the copy-kernel calibration).
     The counters cannot be read from inside this process, so the figure is
     the one measured for this workload by the command the summary names, and
@@ -428,9 +428,9 @@ def main():
     ext_flop_per_launch = extend_flops(cnt) / max(ext_n, 1)
     ext_avg_s = ext_ms / 1e3 / max(ext_n, 1)
     achieved = ext_flop_per_launch / ext_avg_s / 1e12 if ext_avg_s > 0 else 0.0
-    # the same kernel on every camera ray (hit_reuse 0: each sample traces
-    # its pixel's camera ray, as the reference does): one counting and one
-    # kernel-timing frame, for comparison with the production figure above
+    # every camera ray traced (hit_reuse 0: each sample traces its pixel's
+    # camera ray, as the reference does; by the wavefront's kernels): one counting
+    # and one kernel-timing frame, for comparison with the production figure above
     r.set_option("hit_reuse", 0)
     r.reset_counters()
     r.set_option("count", 1)
@@ -448,7 +448,7 @@ def main():
     nr_s = nr_ms / 1e3 / max(nr_n, 1)
     nr_achieved = nr_flop / nr_s / 1e12 if nr_s > 0 else 0.0
     rays_per_step = cnt["segments"]
-    traffic, traffic_note = extend_traffic(args.workload)
+    traffic, traffic_note = path_traffic(args.workload)
     total_flop = path_flops(cnt)
     step_s = ms_per_step / 1e3
 
@@ -497,9 +497,10 @@ def main():
             "launches": ext_n,
             "timing": "each launch timed alone (kernel-timing pass, launches serialized)",
             "every_camera_ray_traced": {
-                "note": "same kernel with option hit_reuse 0 (each sample traces its pixel's "
-                        "camera ray, as the reference does; same image): the camera rays it "
-                        "then traces are its cheapest, most coherent work",
+                "note": "the wavefront's closest-hit kernel, alone, with option hit_reuse 0 (each "
+                        "sample traces its pixel's camera ray, as the reference does; same image; "
+                        "the path kernel has no such form): the camera rays it then traces are "
+                        "its cheapest, most coherent work",
                 "achieved": round(nr_achieved, 4),
                 "frac": round(nr_achieved / PEAK_FP32_TFLOPS, 6),
                 "frac_of_issue_ceiling": round(nr_achieved / ISSUE_TOPS, 6),

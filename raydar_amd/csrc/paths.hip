@@ -820,7 +820,9 @@ uint32_t dynamic_lds_bytes(const PathArgs &a, bool record) {
 // compact: 1000 objects (455 nodes) 1.03 -> 1.04 ms, 1400 (621) 1.24 -> 1.23,
 // 2000 1.56 -> 1.50, 2400 1.78 -> 1.66, 4096 (1777) 2.63 -> 2.26, 8000 4.62 ->
 // 4.01; 1080p, 2 spp: 2400 1.06 -> 1.10, 4096 1.28 -> 1.33, 8000 1.71 -> 1.73,
-// 14000 2.07 -> 1.97: the line is nodes times paths.  With Vulkan semantics
+// 14000 2.07 -> 1.97: the line is nodes times paths, where no pass measured loses
+// (8000 objects in the short pass come to 1.45e10) and 2000 in the long one, at
+// 1.3e10, leave 4 % behind.  With Vulkan semantics
 // (four waves per SIMD, more registers) the full nodes are faster at every
 // size: 2400 2.48 against 2.26, 4096 2.92 and 2.56, 14000 5.55 and 5.28.  Nor for
 // scenes beyond 2^62, where a node's unit times 1/d (at most 2^60) could overflow.
