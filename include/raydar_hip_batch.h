@@ -89,9 +89,9 @@ const char *rd_batch_last_error(const rd_batch *b);
  * library's defaults (block 256, leaf 1, queue 2^24).
  *
  * Results are kept per device: the key is the GPU (name, architecture, CU
- * count, memory size, PCI location), the batch's pipe count and solo
- * threshold, and the shape of the sample mix (per job: object count,
- * resolution, samples, bounce limit).  Tuning the same mix again on the same
+ * count, memory size, PCI location), the library's kernels, the batch's pipe
+ * count and solo threshold, and the shape of the sample mix (per job: object
+ * count, resolution, samples, bounce limit).  Tuning the same mix again on the same
  * GPU returns the kept result at once (cached = 1) and applies it.  The
  * cache lives in the process; with RAYDAR_HIP_TUNE_CACHE=<file> set it is
  * also read from and appended to that file (one line per result), so later

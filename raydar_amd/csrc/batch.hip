@@ -1037,8 +1037,10 @@ const char *tune_file() {
   return f && *f ? f : nullptr;
 }
 
-// Device identity + batch shape + per-job work shape, as one line of text
-// (no tabs or newlines: it is the first field of a cache-file line).
+// Device identity + kernels + batch shape + per-job work shape, as one line of
+// text (no tabs or newlines: it is the first field of a cache-file line).
+// Results that name no kernels were timed on the wavefront's, when every
+// workgroup size ran the same ones; they are not taken.
 bool tune_key(const rd_batch *b, const rd_job_desc *jobs, uint32_t n, std::string *key) {
   int dev = 0;
   hipDeviceProp_t p;
@@ -1050,7 +1052,7 @@ bool tune_key(const rd_batch *b, const rd_job_desc *jobs, uint32_t n, std::strin
   for (const char *c = p.name; *c && k.size() < 64; ++c) k += (*c == '\t' || *c == '\n') ? ' ' : *c;
   k += "|" + std::string(p.gcnArchName) + "|cu" + std::to_string(p.multiProcessorCount) + "|mem" +
        std::to_string((unsigned long long)p.totalGlobalMem) + "|pci" + std::to_string(p.pciDomainID) +
-       ":" + std::to_string(p.pciBusID) + ":" + std::to_string(p.pciDeviceID) + "|pipes" +
+       ":" + std::to_string(p.pciBusID) + ":" + std::to_string(p.pciDeviceID) + "|kernels=paths|pipes" +
        std::to_string(b->st.m.size()) + "|solo" + std::to_string((unsigned long long)b->solo.min_paths) +
        "|graph" + std::to_string(b->st.first().use_graph) + "|jobs" + std::to_string(n);
   // FNV-1a over each job's work shape

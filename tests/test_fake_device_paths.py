@@ -31,3 +31,17 @@ def test_path_kernel_host_code_asan(asan, args, nosync):
 @pytest.mark.parametrize("args", [["path_frames"], ["plain"]])
 def test_path_kernel_host_code_tsan(tsan, args):
     _run(tsan, args, 900)
+
+
+def test_autotune_results_of_the_wavefront_alone_are_not_taken(asan, tmp_path):
+    # a file of results from before the path kernel (lines whose key does not
+    # name the kernels): a workgroup size that was best then would keep a batch
+    # off the path kernel
+    f = tmp_path / "tune.txt"
+    _run(asan, ["autotune"], 900, RAYDAR_HIP_TUNE_CACHE=str(f))
+    lines = f.read_text().splitlines()
+    old = [l.replace("|kernels=paths", "") for l in lines]
+    f.write_text("\n".join(old) + "\n")
+    again = _run(asan, ["autotune"], 900, RAYDAR_HIP_TUNE_CACHE=str(f))
+    assert "autotune cached=0" in again and "other mix cached=0" in again
+    assert f.read_text().splitlines()[:2] == old
